@@ -272,19 +272,50 @@ __global__ __launch_bounds__(kNormThreads) void k2d_norm(const int32_t *__restri
 
 
 // ---------------------------------------------------------------------------
-// Tile gather.  Block = 4 waves = one 64x64 tile.  Wave w owns the 16-column
-// strip [16w, 16w+16) of the tile; lane l works on column 16w + (l & 15) and
-// rows 4k + (l >> 4), k = 0..15, so each lane accumulates 16 pixels in FP64
-// registers.  Per batch of particles the row terms (x offset^2, x overlap) of
-// all 64 tile rows are tabulated once in LDS; per particle each lane computes
-// its column terms, and waves skip particles that miss their strip or row
-// groups (wave-uniform scalar tests).  Per pixel: one sqrt, the kernel
-// polynomial with the row overlap folded into its (1 - u) factor (shape_row),
-// and NP FP64 FMAs (the plane multiplier already carries the particle's scale
-// and the lane's column overlap).
+// Tile gather.  A block takes a work item of one 64x64 tile, cut into 8x8
+// sub-blocks of 8x8 pixels; a wave owns the sub-blocks of one or two 8-column
+// strips, a lane one pixel of each, accumulated in FP64 registers.  Per batch
+// of particles the block tabulates in LDS the row and column terms of the 64
+// tile rows and columns and, by ballot, which sub-blocks each particle
+// reaches; a wave walks the particles that reach its strips and evaluates
+// only those sub-blocks (wave-uniform scalar tests).  Per pixel: one sqrt,
+// the kernel polynomial with the row overlap folded into its (1 - u) factor
+// (shape_row), and NP FP64 FMAs (the plane multiplier carries the particle's
+// scale and the lane's column overlap).
+//
+// What bounds it: VALU issue.  A disc of radius r is covered by sub-blocks of
+// pi r^2 + 32 r + 64 pixels on average (1.44 of its area at r = 25), against
+// pi r^2 + 64 r + 256 (1.95) for the 16-column strips tested 16 rows at a
+// time that this replaces; the rest is the tables (about 0.46 of 2.2 ms on
+// the lattice blast) and, at three or four planes, the waves' unequal shares
+// between two barriers (about 20 %; dealing the sub-blocks to the waves along
+// diagonals evens the shares but reads the column terms per sub-block: 2.7
+// ms).  The FP64 matrix instructions share the vector unit's time on this
+// part (a 4x4x4 costs 17 cycles beside 4 per vector FMA), so the plane sums
+// stay on it.
 // ---------------------------------------------------------------------------
-constexpr int kGBatch = 32;
-constexpr int kGStep = 4;  // row groups per skip test (measured best of 1, 2, 4, 8, 16)
+constexpr int kGSub = 8;             // sub-block side
+constexpr int kGSubs = kGT / kGSub;  // sub-blocks per tile side
+// Waves per block.  Up to two planes, four waves own two strips of
+// sub-blocks each (bx = w and w + 4) and evaluate one sub-block per test, the
+// two strips' same rows following each other; three or four planes, eight
+// waves own one strip each, so that the accumulators leave room for four
+// waves per SIMD, and evaluate two sub-blocks of the strip side by side where
+// both are reached.  Measured (2^24 cluster set on 4096^2, two planes; 2^20
+// lattice blast on 1024^2, three planes; a 16-map batch, four planes): four
+// waves 242 / 2.53 / 12.1 ms, eight waves 250 / 2.24 / 11.3 ms; before
+// (16-column strips tested 16 rows at a time, four waves) 246 / 2.48 / 12.4
+// ms.
+constexpr int gather_waves(int np) { return np > 2 ? 8 : 4; }
+constexpr int gather_threads(int np) { return gather_waves(np) * kWave; }
+// particles per batch of tables: three or four FP64 planes run two blocks per
+// CU whatever the LDS below 80 KB, and longer batches even out the waves'
+// shares between two barriers
+constexpr int gather_batch(int np, bool f64) { return np > 2 && f64 ? 64 : 32; }
+// particles whose records a block loads into LDS at a time: the loads'
+// latency (list entry, then record and quantities) is paid once per two
+// batches (cluster set: 236 ms, 243 ms with a load per batch)
+constexpr int gather_stage(int np, bool f64) { return 2 * gather_batch(np, f64); }
 
 // A: the accumulator type, double, or float with S2G_FLAG_FP32_ACCUM (an
 // item's pixel sums in FP32, written to its FP64 partials)
@@ -302,14 +333,20 @@ __device__ __forceinline__ void gather_tile(const int4 *__restrict__ items,
 {
     if (d_nitems && ((int64_t)blockIdx.x >= *d_nitems || *d_flag))
         return;  // the whole block
+    constexpr int kGBatch = gather_batch(NP, sizeof(A) == 8);
+    constexpr int kGStage = gather_stage(NP, sizeof(A) == 8);
+    constexpr int kGThreads = gather_threads(NP), kW = gather_waves(NP);
+    constexpr int D = kGSubs / kW;  // strips per wave
     __shared__ float2 s_row[kGBatch][kGT];
     __shared__ float2 s_col[kGBatch][kGT];
-    __shared__ double s_x[kGBatch], s_y[kGBatch], s_h[kGBatch];
-    __shared__ float s_hinv[kGBatch];
-    __shared__ double s_hinvd[kGBatch];
-    __shared__ int s_i0[kGBatch], s_i1[kGBatch], s_j0[kGBatch], s_j1[kGBatch];
-    __shared__ double s_mult[NP][kGBatch];
-    __shared__ int s_k[kGBatch][4];  // row-group range per (particle, strip), -1: none
+    __shared__ double s_x[kGStage], s_y[kGStage], s_h[kGStage];
+    __shared__ double s_hinvd[kGStage];
+    __shared__ int4 s_box[kGStage];
+    __shared__ double s_mult[NP][kGStage];
+    // per particle: bit bx * 8 + by = sub-block (by, bx) is reached; bit j =
+    // the overlap of column j is below 1
+    __shared__ uint64_t s_mask[kGBatch];
+    __shared__ uint64_t s_edge[kGBatch];
 
     const int4 it = items[blockIdx.x];
     const int ntj = maps[it.w].ntj;
@@ -317,125 +354,156 @@ __device__ __forceinline__ void gather_tile(const int4 *__restrict__ items,
     const T *binq = (const T *)maps[it.w].binq;
     const int64_t pbase = maps[it.w].pbase;
     const int ti0 = (tile / ntj) * kGT, tj0 = (tile % ntj) * kGT;
-    const int wv = threadIdx.x / kWave, ln = threadIdx.x % kWave;
-    const int rg = ln >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), ln = threadIdx.x % kWave;
+    const int lr = ln / kGSub, lc = ln % kGSub;
 
-    A acc[kGRows][NP];
+    A acc[D][kGSubs][NP];
 #pragma unroll
-    for (int k = 0; k < kGRows; ++k)
+    for (int s = 0; s < D; ++s)
 #pragma unroll
-        for (int q = 0; q < NP; ++q)
-            acc[k][q] = A(0);
+        for (int k = 0; k < kGSubs; ++k)
+#pragma unroll
+            for (int q = 0; q < NP; ++q)
+                acc[s][k][q] = A(0);
 
     for (int base = 0; base < it.z; base += kGBatch) {
         const int cnt = it.z - base < kGBatch ? it.z - base : kGBatch;
-        if (threadIdx.x < cnt) {
-            const int p = pairs[it.y + base + threadIdx.x];
-            const Rec2 r = rec[p];
-            s_x[threadIdx.x] = r.x;
-            s_y[threadIdx.x] = r.y;
-            s_h[threadIdx.x] = r.h;
-            const double hi = r.fb ? 0.0 : 1.0 / r.h;
-            s_hinv[threadIdx.x] = (float)hi;
-            s_hinvd[threadIdx.x] = hi;
-            s_i0[threadIdx.x] = r.i0;
-            s_i1[threadIdx.x] = r.i1;
-            s_j0[threadIdx.x] = r.j0;
-            s_j1[threadIdx.x] = r.j1;
+        const int sb = base % kGStage;  // the batch's first staged record
+        if (sb == 0) {
+            if (threadIdx.x < kGStage && base + (int)threadIdx.x < it.z) {
+                const int p = pairs[it.y + base + threadIdx.x];
+                const Rec2 r = rec[p];
+                s_x[threadIdx.x] = r.x;
+                s_y[threadIdx.x] = r.y;
+                s_h[threadIdx.x] = r.h;
+                s_hinvd[threadIdx.x] = r.fb ? 0.0 : 1.0 / r.h;
+                s_box[threadIdx.x] = make_int4(r.i0 - ti0, r.i1 - ti0, r.j0 - tj0, r.j1 - tj0);
 #pragma unroll
-            for (int q = 0; q < NP; ++q) {
-                const int P = plane0 + q;
-                const double mult =
-                    P == nq ? 1.0 : ld(binq, (int64_t)(p - pbase) * nq + (P < nq ? P : 0));
-                s_mult[q][threadIdx.x] = mult * r.s;
+                for (int q = 0; q < NP; ++q) {
+                    const int P = plane0 + q;
+                    const double mult =
+                        P == nq ? 1.0 : ld(binq, (int64_t)(p - pbase) * nq + (P < nq ? P : 0));
+                    s_mult[q][threadIdx.x] = mult * r.s;
+                }
             }
+            __syncthreads();
         }
-        __syncthreads();
         // row and column tables of the batch for the 64 tile rows and
         // columns: ((x offset / h)^2, x overlap^(1/n)) and
         // ((y offset / h)^2, y overlap); offset / h is formed in FP64 and
         // rounded once, so no rounding of 1/h scales a whole footprint
-        for (int e = threadIdx.x; e < cnt * kGT; e += 256) {
+        for (int e = threadIdx.x; e < cnt * kGT; e += kGThreads) {
             const int b = e / kGT, rr = e % kGT;
             const double fi = (double)(ti0 + rr), fj = (double)(tj0 + rr);
-            const float xs = (float)(coff1(s_x[b], fi) * s_hinvd[b]);
-            const float a = overlap_root<K>((float)overlap1(s_x[b], s_h[b], fi));
+            const double x = s_x[sb + b], y = s_y[sb + b], h = s_h[sb + b], hi = s_hinvd[sb + b];
+            const float xs = (float)(coff1(x, fi) * hi);
+            const float a = overlap_root<K>((float)overlap1(x, h, fi));
             s_row[b][rr] = make_float2(xs * xs, a);
-            const float ys = (float)(coff1(s_y[b], fj) * s_hinvd[b]);
-            const float ay = fmaxf((float)overlap1(s_y[b], s_h[b], fj), 0.0f);
+            const float ys = (float)(coff1(y, fj) * hi);
+            const float ay = fmaxf((float)overlap1(y, h, fj), 0.0f);
             s_col[b][rr] = make_float2(ys * ys, ay);
-        }
-        // row groups each wave's strip needs for each particle: the footprint
-        // box, narrowed to the rows that can reach the kernel disc from the
-        // strip's 16 columns, |x - i - 1/2| < sqrt(h^2 - dy^2) + 1/4 with dy
-        // the smallest distance of a column centre from y.  The quarter-pixel
-        // margin keeps every skipped pixel at u >= 1 up to FP32 rounding
-        // (W = 0, or below 1e-20 relative).
-        if (threadIdx.x < cnt * 4) {
-            const int b = threadIdx.x >> 2, w = threadIdx.x & 3;
-            const int c0 = tj0 + 16 * w;
-            int packed = -1;
-            if (!(c0 + 15 < s_j0[b] || c0 > s_j1[b])) {
-                const int i0 = s_i0[b] - ti0, i1 = s_i1[b] - ti0;
-                int klo = i0 > 0 ? (i0 >> 2) : 0;
-                int khi = (i1 >> 2) < kGRows - 1 ? (i1 >> 2) : kGRows - 1;
-                if (s_hinv[b] != 0.0f) {
-                    const float xc = (float)s_x[b], yc = (float)s_y[b], hf = (float)s_h[b];
-                    const float dy = fmaxf(0.0f, fmaxf((float)c0 + 0.5f - yc,
-                                                       yc - ((float)c0 + 15.5f)));
-                    if (dy < hf + 0.25f) {
-                        const float hx = sqrtf(fmaxf(hf * hf - dy * dy, 0.0f)) + 0.25f;
-                        const int ra = (int)floorf(xc - 0.5f - hx) - ti0;
-                        const int rb = (int)ceilf(xc - 0.5f + hx) - ti0;
-                        klo = (ra >> 2) > klo ? (ra >> 2) : klo;
-                        khi = (rb >> 2) < khi ? (rb >> 2) : khi;
-                    } else {
-                        khi = -1;
-                    }
-                }
-                if (klo <= khi)
-                    packed = klo | (khi << 8);
+            // this wave holds the particle's 64 columns and sub-blocks (one
+            // lane each).  A sub-block is reached if it meets the footprint
+            // box and, unless the particle takes the fallback, its nearest
+            // pixel centre lies within h + 1/4 of the particle.  The
+            // quarter-pixel margin keeps every skipped pixel at u >= 1 up to
+            // FP32 rounding (W = 0, or below 1e-20 relative); radii whose
+            // square would leave FP32 take every sub-block of the box.
+            const int4 bo = s_box[sb + b];
+            const int i8 = (rr % kGSubs) * kGSub, j8 = (rr / kGSubs) * kGSub;
+            const float xc = (float)(x - (double)ti0), yc = (float)(y - (double)tj0);
+            const float hm = (float)h + 0.25f;
+            const float c0 = (float)i8 + 0.5f, d0 = (float)j8 + 0.5f;
+            const float dx = fmaxf(0.0f, fmaxf(c0 - xc, xc - (c0 + (float)(kGSub - 1))));
+            const float dy = fmaxf(0.0f, fmaxf(d0 - yc, yc - (d0 + (float)(kGSub - 1))));
+            const bool in = i8 <= bo.y && i8 + kGSub - 1 >= bo.x && j8 <= bo.w &&
+                            j8 + kGSub - 1 >= bo.z &&
+                            (hi == 0.0 || !(hm < 1e15f) || dx * dx + dy * dy < hm * hm);
+            const uint64_t m = __ballot(in), ed = __ballot(ay < 1.0f);
+            if (rr == 0) {
+                s_mask[b] = m;
+                s_edge[b] = ed;
             }
-            s_k[b][w] = packed;
         }
         __syncthreads();
-        for (int b = 0; b < cnt; ++b) {
-            const int kk = __builtin_amdgcn_readfirstlane(s_k[b][wv]);
-            if (kk < 0)
-                continue;
-            const int klo = kk & 0xff, khi = kk >> 8;
-            const float2 cv = s_col[b][16 * wv + (ln & 15)];
-            const float yd2 = cv.x;
-            // the lane's column overlap is common to its 16 pixels: fold it
-            // into the FP64 plane multipliers
-            const double ayd = (double)cv.y;
-            A mult[NP];
+        // this wave's sub-blocks of particle lane b, strip s in bits 8 s on;
+        // the particles with any sub-block to evaluate are taken in order
+        int mk = 0;
+        bool ed = false;
+        if (ln < cnt) {
 #pragma unroll
-            for (int q = 0; q < NP; ++q)
-                mult[q] = (A)(s_mult[q][b] * ayd);
-            // kGStep row groups per wave-uniform test, so their LDS reads and
-            // dependency chains overlap.  A group outside [klo, khi] adds
-            // exact zeros (a = 0 outside the footprint, u >= 1 outside the
-            // row range), so the image is the same as with one group per test
-            // (evaluating only the groups in the range, with the chunks at
-            // the range's ends taken one group at a time, was slower: 272 ->
-            // 314 ms on the cluster set).
+            for (int s = 0; s < D; ++s) {
+                const int sh = kGSub * (wv + kW * s);
+                mk |= (int)((s_mask[ln] >> sh) & 0xff) << (kGSubs * s);
+                ed = ed || ((s_edge[ln] >> sh) & 0xff) != 0;
+            }
+        }
+        uint64_t live = __ballot(mk != 0);
+        const uint64_t edge = __ballot(ed);
+        while (live) {
+            const int b = __builtin_ctzll(live);
+            live &= live - 1;
+            const int m = __builtin_amdgcn_readlane(mk, b);
+            // the lane's column overlap is common to its pixels of a strip:
+            // fold it into the FP64 plane multipliers
+            float yd2[D];
+            A mult[D][NP];
 #pragma unroll
-            for (int k0 = 0; k0 < kGRows; k0 += kGStep) {
-                if (k0 + kGStep - 1 < klo || k0 > khi)
-                    continue;
-                float wk[kGStep];
-#pragma unroll
-                for (int d = 0; d < kGStep; ++d) {
-                    const float2 rvk = s_row[b][4 * (k0 + d) + rg];
-                    wk[d] = shape_row<K>(__builtin_amdgcn_sqrtf(rvk.x + yd2), rvk.y);
-                }
-#pragma unroll
-                for (int d = 0; d < kGStep; ++d) {
-                    const A f = (A)wk[d];
+            for (int s = 0; s < D; ++s) {
+                const float2 cv = s_col[b][kGSub * (wv + kW * s) + lc];
+                yd2[s] = cv.x;
+                if (D > 1 || (edge >> b & 1)) {
 #pragma unroll
                     for (int q = 0; q < NP; ++q)
-                        acc[k0 + d][q] = fma(f, mult[q], acc[k0 + d][q]);
+                        mult[s][q] = (A)(s_mult[q][sb + b] * (double)cv.y);
+                } else {
+#pragma unroll
+                    for (int q = 0; q < NP; ++q)
+                        mult[s][q] = (A)s_mult[q][sb + b];
+                }
+            }
+            auto weight = [&](float2 rv, int s) {
+                return (A)shape_row<K>(__builtin_amdgcn_sqrtf(rv.x + yd2[s]), rv.y);
+            };
+            if constexpr (D > 1) {
+#pragma unroll
+                for (int k = 0; k < kGSubs; ++k) {
+                    const float2 rv = s_row[b][kGSub * k + lr];
+#pragma unroll
+                    for (int s = 0; s < D; ++s)
+                        if (m & (1 << (kGSubs * s + k))) {
+                            const A f = weight(rv, s);
+#pragma unroll
+                            for (int q = 0; q < NP; ++q)
+                                acc[s][k][q] = fma(f, mult[s][q], acc[s][k][q]);
+                        }
+                }
+            } else {
+                // pairs of sub-blocks (rows k, k + 1) that are both reached
+                // (bit of the first) run side by side, so that their
+                // dependency chains overlap; then the ones reached alone
+                int both = m & (m >> 1) & 0x55;
+                int one = m & ~(both * 3);
+                asm("" : "+s"(both), "+s"(one));  // keep the tests below apart
+#pragma unroll
+                for (int k = 0; k < kGSubs; k += 2) {
+                    if (both & (1 << k)) {
+                        const A f0 = weight(s_row[b][kGSub * k + lr], 0);
+                        const A f1 = weight(s_row[b][kGSub * (k + 1) + lr], 0);
+#pragma unroll
+                        for (int q = 0; q < NP; ++q) {
+                            acc[0][k][q] = fma(f0, mult[0][q], acc[0][k][q]);
+                            acc[0][k + 1][q] = fma(f1, mult[0][q], acc[0][k + 1][q]);
+                        }
+                    }
+#pragma unroll
+                    for (int d = 0; d < 2; ++d)
+                        if (one & (1 << (k + d))) {
+                            const A f = weight(s_row[b][kGSub * (k + d) + lr], 0);
+#pragma unroll
+                            for (int q = 0; q < NP; ++q)
+                                acc[0][k + d][q] = fma(f, mult[0][q], acc[0][k + d][q]);
+                        }
                 }
             }
         }
@@ -445,19 +513,16 @@ __device__ __forceinline__ void gather_tile(const int4 *__restrict__ items,
 #pragma unroll
     for (int q = 0; q < NP; ++q)
 #pragma unroll
-        for (int k = 0; k < kGRows; ++k)
-            dst[(q * kGT + 4 * k + rg) * kGT + 16 * wv + (ln & 15)] = (double)acc[k][q];
+        for (int s = 0; s < D; ++s)
+#pragma unroll
+            for (int k = 0; k < kGSubs; ++k)
+                dst[(q * kGT + kGSub * k + lr) * kGT + kGSub * (wv + kW * s) + lc] =
+                    (double)acc[s][k][q];
 }
 
-// up to two planes: 128 VGPRs, four waves per SIMD (the accumulators need
-// 64); three or four planes: 168 VGPRs, three waves per SIMD (four planes
-// spill a few registers, which costs less than the lost wave: the batched
-// 64-map set's gather 85 -> 73 ms).  Tried and dropped: eight waves per
-// block with half the tile's rows per wave, so that four planes fit 128
-// VGPRs at four waves per SIMD: the batched set's gather 70.6 -> 81.5 ms
-// (each wave repeats the per-particle set-up for half the pixels).
+// all variants hold at most 128 VGPRs (no spills): four waves per SIMD
 template <typename T, int K, int NP>
-__global__ __launch_bounds__(256, 4) void k2d_gather(const int4 *__restrict__ items,
+__global__ __launch_bounds__(gather_threads(NP), 4) void k2d_gather(const int4 *__restrict__ items,
                                                      const int32_t *__restrict__ pairs,
                                                      const Rec2 *__restrict__ rec,
                                                      const Map2D *__restrict__ maps, int nq,
@@ -469,7 +534,7 @@ __global__ __launch_bounds__(256, 4) void k2d_gather(const int4 *__restrict__ it
                                   d_flag);
 }
 template <typename T, int K, int NP>
-__global__ __launch_bounds__(256, 3) void k2d_gather_wide(const int4 *__restrict__ items,
+__global__ __launch_bounds__(gather_threads(NP), 4) void k2d_gather_wide(const int4 *__restrict__ items,
                                                        const int32_t *__restrict__ pairs,
                                                        const Rec2 *__restrict__ rec,
                                                        const Map2D *__restrict__ maps, int nq,
@@ -480,9 +545,9 @@ __global__ __launch_bounds__(256, 3) void k2d_gather_wide(const int4 *__restrict
     gather_tile<T, K, NP, double>(items, pairs, rec, maps, nq, plane0, partial, d_nitems,
                                   d_flag);
 }
-// FP32 accumulators: at most 64 VGPRs for four planes, four waves per SIMD
+// FP32 accumulators: 80 VGPRs for three or four planes, six waves per SIMD
 template <typename T, int K, int NP>
-__global__ __launch_bounds__(256, 4) void k2d_gather_f32acc(const int4 *__restrict__ items,
+__global__ __launch_bounds__(gather_threads(NP), NP > 2 ? 6 : 4) void k2d_gather_f32acc(const int4 *__restrict__ items,
                                                          const int32_t *__restrict__ pairs,
                                                          const Rec2 *__restrict__ rec,
                                                          const Map2D *__restrict__ maps, int nq,
@@ -882,15 +947,15 @@ template <typename T, int K, int NP>
 static void gather_knp(const GatherArgs &g, hipStream_t s)
 {
     if (g.fp32acc)
-        hipLaunchKernelGGL((k2d_gather_f32acc<T, K, NP>), dim3((unsigned)g.nitems), dim3(256), 0,
+        hipLaunchKernelGGL((k2d_gather_f32acc<T, K, NP>), dim3((unsigned)g.nitems), dim3(gather_threads(NP)), 0,
                            s, g.items, g.pairs, g.rec, g.maps, g.nq, g.plane0, g.partial,
                            g.d_nitems, g.d_flag);
     else if constexpr (NP <= 2)
-        hipLaunchKernelGGL((k2d_gather<T, K, NP>), dim3((unsigned)g.nitems), dim3(256), 0, s,
+        hipLaunchKernelGGL((k2d_gather<T, K, NP>), dim3((unsigned)g.nitems), dim3(gather_threads(NP)), 0, s,
                            g.items, g.pairs, g.rec, g.maps, g.nq, g.plane0, g.partial,
                            g.d_nitems, g.d_flag);
     else
-        hipLaunchKernelGGL((k2d_gather_wide<T, K, NP>), dim3((unsigned)g.nitems), dim3(256), 0,
+        hipLaunchKernelGGL((k2d_gather_wide<T, K, NP>), dim3((unsigned)g.nitems), dim3(gather_threads(NP)), 0,
                            s, g.items, g.pairs, g.rec, g.maps, g.nq, g.plane0,
                            g.partial, g.d_nitems, g.d_flag);
 }

@@ -29,9 +29,8 @@ constexpr int kSmallSide2D = 34;
 // side of the small-footprint tiles (a particle's bucket is the tile holding
 // its footprint's first pixel)
 constexpr int kST = 32;
-// 2D gather tile: 64 x 64 pixels, 4 waves x 16 rows x 64 columns.
+// 2D gather tile: 64 x 64 pixels.
 constexpr int kGT = 64;
-constexpr int kGRows = 16;
 
 // 3D: footprint box side <= 8 voxels goes to the scatter path; bricks of 16^3.
 constexpr int kSmallSide3D = 8;

@@ -239,6 +239,31 @@ def test_large_only_is_deterministic(s2g):
     np.testing.assert_array_equal(a, b)
 
 
+@pytest.mark.parametrize("nq", [1, 2, 3])  # two planes per gather launch, three, four
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 129])  # table batches and staged records
+def test_gather_sub_blocks(s2g, orc, nq, n):
+    """Footprints (h = 18 to 45 px, gather path) whose centres and edges sit
+    on and around the corners of the 8x8 sub-blocks and 64x64 tiles, on an
+    image that cuts the last tile: which sub-blocks the gather skips must not
+    show.  Also one particle far wider than the image."""
+    npix = 150
+    r = np.random.default_rng(10 * n + nq)
+    cells = r.integers(0, npix // 8, (n, 2)) * 8.0
+    cells[:: 3] = r.integers(0, 3, cells[:: 3].shape) * 64.0
+    px = cells + r.choice([-0.5, -1e-9, 0.0, 1e-9, 0.5], (n, 2))
+    h = r.choice([18.0, 20.5, 24.0, 32.0, 45.0], n) + r.choice([-1e-9, 0.0, 1e-9], n)
+    h[-1] = 30.0 * npix if n > 1 else h[-1]
+    x = np.zeros((n, 3))
+    x[:, :2] = (px - 0.5 * npix) / npix
+    h = h / npix
+    m, rho, w = (r.uniform(0.5, 2.0, n) for _ in range(3))
+    q = r.uniform(0.5, 2.0, (n, nq)) if nq > 1 else r.uniform(0.5, 2.0, n)
+    gpu = s2g.deposit(x, h, m, rho, q, w, npix=npix, len2pix=float(npix),
+                      kernel=s2g.WendlandC6(2))
+    ref = orc.cic_mapping_2D(x, h, m, rho, q, w, npix, float(npix), "wendlandc6", 2, True)
+    _check_flat(gpu, ref, f"n={n} nq={nq}")
+
+
 def test_cluster_scaled(s2g, orc):
     """Cluster-like particle set (halo + background, h log-uniform over three
     decades) at 2^17 particles on 512^2."""
