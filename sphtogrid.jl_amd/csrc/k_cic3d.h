@@ -37,6 +37,13 @@ void launch_3d_norm(int kernel, const int32_t *list, int64_t ne, int64_t npix, u
 void launch_3d_gather(const Gather3Args &g, hipStream_t s);
 void launch_3d_finalize(const Gather3Args &g, hipStream_t s);
 void launch_3d_small(const Small3Args &a, hipStream_t s);
+// windowed small scatter: particles sorted by the kST3^3 tile (nt per side)
+// of their box's first voxel, one block per work item (at most max_items)
+constexpr int kST3 = 9;
+void launch_3d_small_keys(const int32_t *list, int64_t ns, const Rec3 *rec, int nt,
+                          uint32_t *keys, int32_t *vals, hipStream_t s);
+void launch_3d_small_window(const Small3Args &a, const int4 *items, const int64_t *nitems,
+                            int64_t max_items, const int32_t *plist, int nt, hipStream_t s);
 void launch_3d_reduce(const double *image, int64_t npix, int reduce, double *out, hipStream_t s);
 
 }  // namespace s2g

@@ -119,6 +119,29 @@ def test_clipped_footprints_border_sum(s2g, orc, kernel):
     _check(a, ref, f"border3d/{kernel}")
 
 
+@pytest.mark.parametrize("npix,n", [(9, 40), (10, 700), (37, 6000)])
+@pytest.mark.parametrize("kernel", ["cubic", "wendlandc6"])
+def test_small_window_scatter(s2g, orc, kernel, npix, n):
+    """Boxes of 1 to 8 voxels a side, centres in the whole grid and just past
+    its edges, some piled into one tile (work items of one tile split), enough
+    of them per 9^3 tile for the windowed scatter.  All weights and sums are
+    FP64, so the image follows the oracle to a few hundred roundings:
+    rel-L1 1e-12."""
+    r = np.random.default_rng(npix + n)
+    x = r.uniform(-0.52, 0.52, (n, 3))
+    x[: n // 4] = (8.7 - 0.5 * npix + 0.3 * x[: n // 4]) / npix
+    h = np.exp(r.uniform(np.log(0.05 / npix), np.log(3.5 / npix), n))
+    h[::5] = 3.5 / npix
+    m, rho, w, q = (r.uniform(0.5, 2.0, n) for _ in range(4))
+    st = {}
+    gpu = s2g.deposit(x, h, m, rho, q, w, npix=npix, len2pix=float(npix), dimensions=3,
+                      kernel=_kernel(s2g, kernel), calc_mean=False, stats=st)
+    assert st["n_small"] >= 32 * (-(-npix // 9)) ** 3 and st["n_large"] == 0
+    ref = orc.cic_mapping_3D(x, h, m, rho, q, w, npix, float(npix), kernel, 3, False)
+    for k in range(2):
+        assert rel_l1(gpu[:, k], ref[:, k]) <= 1e-12, k
+
+
 def test_large_only_is_deterministic(s2g):
     npix, n = 48, 150
     x, h, m, rho, q, w = _particles(n, npix, 8, hmin=4.0, hmax=12.0)
