@@ -13,16 +13,21 @@
 // atomics and no memset, and the result is bit-reproducible):
 //   k_tsc_keys     brick of each particle's nearest cell (bricks of
 //                  kTX x kTY x kTZ cells, row-major; dropped particles last)
-//   (radix sort)   stable, so particles keep their input order in a brick
+//                  and, in the key's low six bits, whether that cell is the
+//                  first or last of its brick along each axis
+//   (radix sort)   on the brick bits, stable, so particles keep their input
+//                  order in a brick
 //   k_tsc_offsets  first sorted particle of every brick
 //   k_tsc_prep     grid coordinates (FP64) and quantity in sorted order, and
 //                  each particle's nearest cell packed into one word
-//   k_tsc_gather   one wave per brick: scans the particles of the (up to) 27
-//                  neighbouring bricks, queues those whose 3^3 stencil
-//                  reaches the brick and deposits them into LDS seven at a
-//                  time (9 lanes per particle, one stencil row each), in scan
-//                  order; then writes the brick's cells.
+//   k_tsc_gather   one wave per brick: scans the sorted keys of the (up to)
+//                  27 neighbouring bricks, queues the particles whose 3^3
+//                  stencil reaches the brick and deposits them into LDS seven
+//                  at a time (9 lanes per particle, one stencil row each), in
+//                  queue order; then writes the brick's cells.
 #include "k_tsc.h"
+
+#include <climits>
 
 namespace s2g {
 
@@ -76,7 +81,10 @@ int64_t tsc_nbricks(int64_t npix)
 }
 
 // Sort key: the brick of the particle's nearest cell (clamped into the grid,
-// or wrapped when periodic); dropped particles get nbricks, after all bricks.
+// or wrapped when periodic) above kTscFlagBits bits, two per axis: the cell is
+// the brick's first (bit 2 d), its last (bit 2 d + 1).  Dropped particles get
+// brick nbricks, after all bricks.
+constexpr int kTscFlagBits = 6;
 template <typename T>
 __global__ __launch_bounds__(256) void k_tsc_keys(const T *__restrict__ pos, int64_t n,
                                                   int64_t npix, double len2pix, int periodic,
@@ -90,22 +98,25 @@ __global__ __launch_bounds__(256) void k_tsc_keys(const T *__restrict__ pos, int
     tsc_bricks(npix, nb);
     double g[3];
     int64_t c[3];
-    uint32_t key = (uint32_t)(nb[0] * nb[1] * nb[2]);
+    uint32_t key = (uint32_t)(nb[0] * nb[1] * nb[2]), flags = 0;
     if (tsc_cell(pos, p, npix, len2pix, periodic, g, c)) {
-        const int64_t side[3] = {kTX, kTY, kTZ};
-        int64_t b[3];
+        const int side[3] = {kTX, kTY, kTZ};
+        int b[3];
         for (int d = 0; d < 3; ++d) {
-            int64_t x = periodic ? tsc_wrap(c[d], npix) : c[d];
-            x = x < 0 ? 0 : x > npix - 1 ? npix - 1 : x;
+            int64_t xl = periodic ? tsc_wrap(c[d], npix) : c[d];
+            const int x = (int)(xl < 0 ? 0 : xl > npix - 1 ? npix - 1 : xl);
             b[d] = x / side[d];
+            const int lx = x - b[d] * side[d];
+            flags |= lx == 0 ? 1u << (2 * d) : 0u;
+            flags |= lx == side[d] - 1 || x == npix - 1 ? 2u << (2 * d) : 0u;
         }
         key = (uint32_t)((b[0] * nb[1] + b[1]) * nb[2] + b[2]);
     }
-    keys[p] = key;
+    keys[p] = key << kTscFlagBits | flags;
     vals[p] = (int32_t)p;
 }
 
-// off[b] = first sorted entry with key >= b, b in [0, nbricks]
+// off[b] = first sorted entry of brick >= b, b in [0, nbricks]
 __global__ __launch_bounds__(256) void k_tsc_offsets(const uint32_t *__restrict__ keys,
                                                      int64_t n, int64_t nbricks,
                                                      int64_t *__restrict__ off)
@@ -116,7 +127,7 @@ __global__ __launch_bounds__(256) void k_tsc_offsets(const uint32_t *__restrict_
     int64_t lo = 0, hi = n;
     while (lo < hi) {
         const int64_t mid = (lo + hi) >> 1;
-        if ((int64_t)keys[mid] < b)
+        if ((int64_t)(keys[mid] >> kTscFlagBits) < b)
             lo = mid + 1;
         else
             hi = mid;
@@ -124,17 +135,18 @@ __global__ __launch_bounds__(256) void k_tsc_offsets(const uint32_t *__restrict_
     off[b] = lo;
 }
 
-// packed nearest cell: 21 bits per axis, each stored as c + kCellBias (c is
-// in [-2, npix + 2] when not periodic, wrapped into [0, npix) when periodic)
-constexpr int64_t kCellBias = 4;
+// packed nearest cell: 16 bits per axis, each stored as c + kCellBias (c is
+// in [-2, npix + 2] when not periodic, wrapped into [0, npix) when periodic;
+// npix <= 2048)
+constexpr int kCellBias = 4;
 __device__ __forceinline__ uint64_t tsc_pack(const int64_t c[3])
 {
-    return (uint64_t)(c[0] + kCellBias) << 42 | (uint64_t)(c[1] + kCellBias) << 21 |
+    return (uint64_t)(c[0] + kCellBias) << 32 | (uint64_t)(c[1] + kCellBias) << 16 |
            (uint64_t)(c[2] + kCellBias);
 }
-__device__ __forceinline__ int64_t tsc_unpack(uint64_t v, int d)
+__device__ __forceinline__ int tsc_unpack(uint64_t v, int d)
 {
-    return (int64_t)((v >> (42 - 21 * d)) & 0x1FFFFF) - kCellBias;
+    return (int)((v >> (32 - 16 * d)) & 0xFFFF) - kCellBias;
 }
 
 // sorted grid coordinates and quantity (gq) and packed cells (cell) of the
@@ -162,118 +174,118 @@ __global__ __launch_bounds__(256) void k_tsc_prep(const T *__restrict__ pos,
     cell[k] = tsc_pack(c);
 }
 
-// bitmask of the stencil offsets o in {-1, 0, 1} (bit o + 1) whose cell
-// c + o (wrapped when periodic) lies in [b0, b0 + side) and in the grid
-__device__ __forceinline__ int tsc_reach(int64_t c, int64_t b0, int64_t side, int64_t npix,
-                                         int periodic)
-{
-    int m = 0;
-#pragma unroll
-    for (int o = -1; o <= 1; ++o) {
-        int64_t x = c + o;
-        if (periodic)
-            x = x < 0 ? x + npix : x >= npix ? x - npix : x;
-        const bool in = x >= b0 && x < b0 + side && x >= 0 && x < npix;
-        m |= in ? 1 << (o + 1) : 0;
-    }
-    return m;
-}
-
 // particles per deposit step: 9 lanes each, one stencil row (o0, o1) per
 // lane and its three cells along z
 constexpr int kTscPerStep = kWave / 9;
+// candidates per lane and scan chunk
+constexpr int kTscPer = 4;
 // Deposit queue of the gather: the candidates whose stencil reaches the
-// brick, in scan order (a ring of LDS slots holding sorted particle
-// indices; the deposit step loads their records).  It holds at most
-// kTscPerStep - 1 leftovers plus one chunk of kWave candidates.  The LDS of
-// a block, not the VGPRs, bounds the waves per CU: with 32-byte records in
-// 128 slots 19 waves, in 72 slots 23, with 4-byte indices 33.
-constexpr int kTscQueue = 72;
-static_assert(kTscQueue >= kTscPerStep - 1 + kWave, "queue holds one chunk and the leftovers");
+// brick, as sorted particle indices in a ring of LDS slots.  It holds at most
+// kTscPerStep - 1 leftovers plus one chunk of candidates.
+constexpr int kTscQueue = 264;
+static_assert(kTscQueue >= kTscPerStep - 1 + kTscPer * kWave,
+              "queue holds one chunk and the leftovers");
 
-// One deposit step: particles slots [h, h + cnt) of the queue.  The
-// weights are formed as the oracle forms them: per axis W(g - (c + o) - 1/2)
-// with c = floor(g), and the product (wx * wy) * wz.
-__device__ __forceinline__ void tsc_step(const double4 *__restrict__ gq, const int32_t *queue,
-                                         int h, int cnt, int ln,
-                                         const int64_t b0[3], int64_t npix, int periodic,
+// a particle's record as the deposit step takes it
+struct TscRec {
+    double4 e;    // grid coordinates, quantity
+    uint64_t cv;  // packed nearest cell
+};
+
+// One deposit step: a particle per nine lanes (cnt of them), r the particle of
+// lane group `slot`.  The weights are formed as the oracle forms them: per
+// axis W(g - (c + o) - 1/2) with c = floor(g), and the product (wx * wy) * wz.
+__device__ __forceinline__ void tsc_step(const TscRec &r, int cnt, int slot, int o0, int o1,
+                                         const int b0[3], int npix, int periodic,
                                          double (*acc)[kTX * kTY * kTZ])
 {
-    const int slot = ln / 9, row = ln - 9 * slot;
     if (slot >= cnt)
         return;
-    const double4 e = gq[queue[(h + slot) % kTscQueue]];
-    const double g[3] = {e.x, e.y, e.z};
-    int64_t c[3];
-    for (int d = 0; d < 3; ++d)
-        c[d] = (int64_t)floor(g[d]);
-    const int o0 = row / 3 - 1, o1 = row % 3 - 1;
-    const double wx = tsc_w(sub_rn(g[0], (double)(c[0] + o0) + 0.5));
-    const double wy = tsc_w(sub_rn(g[1], (double)(c[1] + o1) + 0.5));
-    int64_t x = c[0] + o0, y = c[1] + o1;
-    if (periodic) {
-        x = tsc_wrap(x, npix);
-        y = tsc_wrap(y, npix);
-    }
-    const int64_t lx = x - b0[0], ly = y - b0[1];
-    if (x < 0 || x >= npix || lx < 0 || lx >= kTX || y < 0 || y >= npix || ly < 0 ||
-        ly >= kTY)
+    const double4 e = r.e;
+    const uint64_t cv = r.cv;
+    auto wrap = [&](int x) {
+        return periodic ? (x < 0 ? x + npix : x >= npix ? x - npix : x) : x;
+    };
+    const int x = wrap(tsc_unpack(cv, 0) + o0), y = wrap(tsc_unpack(cv, 1) + o1);
+    const int lx = x - b0[0], ly = y - b0[1];
+    if (x >= npix || (unsigned)lx >= (unsigned)kTX || y >= npix || (unsigned)ly >= (unsigned)kTY)
         return;
-    const double wxy = wx * wy;
+    const double wx = tsc_w(sub_rn(e.x, floor(e.x) + (double)o0 + 0.5));
+    const double wy = tsc_w(sub_rn(e.y, floor(e.y) + (double)o1 + 0.5));
+    const double wxy = wx * wy, fz = floor(e.z);
+    const int cz = tsc_unpack(cv, 2), row = (lx * kTY + ly) * kTZ;
 #pragma unroll
     for (int o2 = -1; o2 <= 1; ++o2) {
-        int64_t z = c[2] + o2;
-        if (periodic)
-            z = tsc_wrap(z, npix);
-        const int64_t lz = z - b0[2];
-        const double ww = wxy * tsc_w(sub_rn(g[2], (double)(c[2] + o2) + 0.5));
-        if (z >= 0 && z < npix && lz >= 0 && lz < kTZ && ww != 0.0) {
-            const int cell = (int)((lx * kTY + ly) * kTZ + lz);
-            unsafeAtomicAdd(&acc[0][cell], e.w * ww);
-            unsafeAtomicAdd(&acc[1][cell], ww);
+        const int z = wrap(cz + o2), lz = z - b0[2];
+        const double ww = wxy * tsc_w(sub_rn(e.z, fz + (double)o2 + 0.5));
+        if (z < npix && (unsigned)lz < (unsigned)kTZ && ww != 0.0) {
+            unsafeAtomicAdd(&acc[0][row + lz], e.w * ww);
+            unsafeAtomicAdd(&acc[1][row + lz], ww);
         }
     }
 }
 
+// Brick of a block: block x runs on XCD x % 8, and the XCDs take runs of
+// kTscRun consecutive bricks in turn, so that the two halves of a cache line
+// and the reads of neighbouring bricks meet in one L2 (2^22 particles at
+// 512^3: 1.17 -> 1.06 ms; runs of 16 / 512 bricks 1.28 / 1.37 ms, 32 and 128
+// as 64).
+constexpr int kTscRun = 64;
+__device__ __forceinline__ int tsc_brick()
+{
+    const int x = blockIdx.x, l = x / 8;
+    const int whole = (int)gridDim.x / (8 * kTscRun) * (8 * kTscRun);
+    return x < whole ? (l / kTscRun * 8 + x % 8) * kTscRun + l % kTscRun : x;
+}
+
 // One wave per brick.  Lane j < 27 takes neighbouring brick j (offsets
-// (j/9 - 1, (j/3)%3 - 1, j%3 - 1), each brick once) and reads its particle
-// range; the ranges are laid end to end (wave prefix sum) and scanned 64
-// candidates at a time (packed cells only; the next chunk's cells are loaded
-// before the current chunk is handled).  The candidates whose stencil
-// reaches the brick load their coordinates into the LDS queue in scan order,
-// and the queue is deposited kTscPerStep particles per step.  The order of
-// the additions to a cell follows the scan order, so the sums are
-// reproducible.
+// (j/9 - 1, (j/3)%3 - 1, j%3 - 1), each brick once), reads its particle range
+// and forms the key flags a particle of it needs to reach this brick (the last
+// cell along an axis whose offset is -1, the first one for +1).  The ranges,
+// cut into groups of kTscPer entries, are laid end to end (wave prefix sum)
+// and scanned 64 groups at a time, a group of sorted keys per lane; the
+// entries with the needed flags go to the LDS queue, and the queue is
+// deposited kTscPerStep particles per step.  The order of the additions to a
+// cell follows the scan, so the sums are reproducible.
+//
+// What bounds it: the round trips to memory of a brick (ranges, keys,
+// records; 0.52 ms without the keys and the records, 0.81 without the records)
+// beside the stores of the planes (2.1 GB, 0.34 ms at the fill rate); the
+// arithmetic and the LDS atomics are hidden (skipping the deposit steps saves
+// 0.08 of 1.17 ms).  2^22 particles at 512^3: 1.30 ms with a packed 64-bit
+// cell tested per candidate, one range search per 64 candidates and 4x8x8
+// bricks, 1.17 with key flags tested four per lane, 0.97 with runs per XCD
+// and bricks as long in z as a cache line.  Tried and dropped: two to sixteen
+// waves per block (1.26 - 1.81 ms), waves that take bricks in turn and load
+// the next brick's ranges and keys ahead (128 VGPRs, 1.51 ms).
 __global__ __launch_bounds__(kWave) void k_tsc_gather(const double4 *__restrict__ gq,
                                                       const uint64_t *__restrict__ cell,
-                                                      const int64_t *__restrict__ off,
-                                                      int64_t npix, int periodic,
-                                                      double *__restrict__ grid)
+                                                      const uint32_t *__restrict__ keys,
+                                                      const int64_t *__restrict__ off, int npix,
+                                                      int periodic, double *__restrict__ grid)
 {
     __shared__ double acc[2][kTX * kTY * kTZ];
     __shared__ int32_t queue[kTscQueue];
-    __shared__ int64_t s_start[32];
-    __shared__ int s_base[32];
-    int64_t nb[3];
-    tsc_bricks(npix, nb);
-    const int64_t side[3] = {kTX, kTY, kTZ};
-    const int64_t b = blockIdx.x;
-    const int64_t bi[3] = {b / (nb[1] * nb[2]), (b / nb[2]) % nb[1], b % nb[2]};
-    int64_t b0[3];
+    __shared__ int4 s_rng[32];  // first group, first entry, end, needed flags
+    const int nb[3] = {(npix + kTX - 1) / kTX, (npix + kTY - 1) / kTY, (npix + kTZ - 1) / kTZ};
+    const int side[3] = {kTX, kTY, kTZ};
+    const int b = tsc_brick();
+    const int bi[3] = {b / (nb[1] * nb[2]), (b / nb[2]) % nb[1], b % nb[2]};
+    int b0[3];
     for (int d = 0; d < 3; ++d)
         b0[d] = bi[d] * side[d];
     const int ln = threadIdx.x;
     // neighbour brick of lane ln, if it exists and is not a repeat of an
-    // earlier offset on some axis (periodic grids of one or two bricks)
-    int len = 0;
-    int64_t start = 0;
+    // earlier offset on some axis (periodic grids of one or two bricks, whose
+    // bricks are reached from either side: no flags needed there)
+    int start = 0, end = 0, need = 0;
     if (ln < 27) {
         const int o[3] = {ln / 9 - 1, (ln / 3) % 3 - 1, ln % 3 - 1};
         bool valid = true;
-        int64_t x[3];
+        int x[3];
         for (int d = 0; d < 3; ++d) {
             auto nbr = [&](int oo) {
-                int64_t v = bi[d] + oo;
+                int v = bi[d] + oo;
                 if (periodic)
                     v = v < 0 ? v + nb[d] : v >= nb[d] ? v - nb[d] : v;
                 return v;
@@ -283,104 +295,125 @@ __global__ __launch_bounds__(kWave) void k_tsc_gather(const double4 *__restrict_
                 valid = false;
             for (int oo = -1; oo < o[d]; ++oo)
                 valid = valid && nbr(oo) != x[d];
+            if (!(periodic && nb[d] <= 2))
+                need |= o[d] < 0 ? 2 << (2 * d) : o[d] > 0 ? 1 << (2 * d) : 0;
         }
         if (valid) {
-            const int64_t nbrick = (x[0] * nb[1] + x[1]) * nb[2] + x[2];
-            start = off[nbrick];
-            len = (int)(off[nbrick + 1] - start);
+            const int nbrick = (x[0] * nb[1] + x[1]) * nb[2] + x[2];
+            start = (int)off[nbrick];
+            end = (int)off[nbrick + 1];
         }
     }
-    // exclusive prefix of the range lengths over the lanes
+    // exclusive prefix of the ranges' group counts over the lanes
+    const int len = (end - start + kTscPer - 1) / kTscPer;
     int incl = len;
 #pragma unroll
-    for (int sh = 1; sh < kWave; sh <<= 1) {
+    for (int sh = 1; sh < 32; sh <<= 1) {
         const int t = __shfl_up(incl, sh);
         incl += ln >= sh ? t : 0;
     }
-    const int total = __shfl(incl, 26);
-    const int64_t nd = npix * npix * npix;
+    const int total = __builtin_amdgcn_readlane(incl, 26);
+    const int64_t nd = (int64_t)npix * npix * npix;
     // lane ln writes cells (t, ln / kTZ, ln % kTZ) of the brick, t < kTX
     static_assert(kTY * kTZ == kWave, "one x plane of a brick per wave");
-    const int64_t j = b0[1] + ln / kTZ, k = b0[2] + ln % kTZ;
+    const int j = b0[1] + ln / kTZ, k = b0[2] + ln % kTZ;
+    const bool in = j < npix && k < npix;
+    const int64_t plane = (int64_t)npix * npix;
+    double *out = grid + ((int64_t)b0[0] * npix + j) * npix + k;
     if (total == 0) {  // wave-uniform: no particle reaches the brick
-        for (int64_t i = b0[0]; i < b0[0] + kTX; ++i)
-            if (i < npix && j < npix && k < npix) {
-                const int64_t idx = (i * npix + j) * npix + k;
-                grid[idx] = 0.0;
-                grid[nd + idx] = 0.0;
+        for (int t = 0; t < kTX && b0[0] + t < npix; ++t)
+            if (in) {
+                out[t * plane] = 0.0;
+                out[nd + t * plane] = 0.0;
             }
         return;
     }
     for (int e = ln; e < 2 * kTX * kTY * kTZ; e += kWave)
         (&acc[0][0])[e] = 0.0;
-    if (ln < 27) {
-        s_start[ln] = start;
-        s_base[ln] = incl - len;
-    }
+    if (ln < 32)  // the lanes past the 27 ranges: bases past every group
+        s_rng[ln] = ln < 27 ? make_int4(incl - len, start, end, need)
+                            : make_int4(INT_MAX, 0, 0, 0);
     __syncthreads();
 
-    // candidate v of the concatenated ranges -> sorted particle index: the
-    // last range whose base is <= v (bases are exclusive prefix sums, so an
-    // empty range after the one holding v has a base > v)
-    auto locate = [&](int v) {
-        int lo = 0;
-#pragma unroll
-        for (int step = 16; step >= 1; step >>= 1)
-            if (lo + step < 27 && s_base[lo + step] <= v)
-                lo += step;
-        return s_start[lo] + (int64_t)(v - s_base[lo]);
-    };
     const uint64_t below = ln == 0 ? 0ull : (~0ull >> (kWave - ln));
-    int head = 0, tail = 0;  // queue slots consumed / filled (wave-uniform)
-    int64_t kc = -1;
-    uint64_t cv = 0;
-    if (ln < total) {
-        kc = locate(ln);
-        cv = cell[kc];
-    }
+    const int slot = ln / 9, srow = ln - 9 * slot;
+    const int o0 = srow / 3 - 1, o1 = srow % 3 - 1;
+    int head = 0, fill = 0;  // first queued slot of the ring, entries queued (wave-uniform)
+    // the record of queue entry head + ahead + slot, if it is queued; the
+    // loop below loads a step's records while the previous step is deposited
+    auto fetch = [&](int ahead) {
+        TscRec r = {};
+        if (slot < kTscPerStep && ahead + slot < fill) {
+            int at = head + ahead + slot;
+            at -= at >= kTscQueue ? kTscQueue : 0;
+            const int q = queue[at];
+            r.e = gq[q];
+            r.cv = cell[q];
+        }
+        return r;
+    };
     for (int v0 = 0; v0 < total; v0 += kWave) {
-        bool use = kc >= 0;
-        if (use)
-            for (int d = 0; d < 3; ++d)
-                use = use && tsc_reach(tsc_unpack(cv, d), b0[d], side[d], npix, periodic) != 0;
-        const int64_t kuse = kc;
-        // the next chunk's cells
-        kc = -1;
-        if (v0 + kWave + ln < total) {
-            kc = locate(v0 + kWave + ln);
-            cv = cell[kc];
+        const int v = v0 + ln;
+        int k0 = 0, k1 = 0;
+        uint32_t nf = 0;
+        if (v < total) {
+            // the last range whose first group is <= v (an empty range after
+            // the one holding v starts after v)
+            int lo = 0;
+#pragma unroll
+            for (int step = 16; step >= 1; step >>= 1)
+                if (s_rng[lo + step].x <= v)
+                    lo += step;
+            const int4 r = s_rng[lo];
+            k0 = r.y + (v - r.x) * kTscPer;
+            k1 = r.z;
+            nf = (uint32_t)r.w;
         }
-        const uint64_t mask = __ballot(use);
-        if (use)
-            queue[(tail + (int)__popcll(mask & below)) % kTscQueue] = (int32_t)kuse;
-        tail += (int)__popcll(mask);
+        uint32_t kv[kTscPer];
+#pragma unroll
+        for (int i = 0; i < kTscPer; ++i)
+            kv[i] = k0 + i < k1 ? keys[k0 + i] : 0u;
+#pragma unroll
+        for (int i = 0; i < kTscPer; ++i) {
+            const bool use = k0 + i < k1 && (kv[i] & nf) == nf;
+            const uint64_t mask = __ballot(use);
+            if (use) {
+                int at = head + fill + (int)__popcll(mask & below);
+                at -= at >= kTscQueue ? kTscQueue : 0;
+                queue[at] = k0 + i;
+            }
+            fill += (int)__popcll(mask);
+        }
         __builtin_amdgcn_wave_barrier();
-        while (tail - head >= kTscPerStep) {
-            tsc_step(gq, queue, head, kTscPerStep, ln, b0, npix, periodic, acc);
-            head += kTscPerStep;
+        // after the last chunk the leftovers follow as a short step
+        const int keep = v0 + kWave < total ? kTscPerStep - 1 : 0;
+        TscRec cur = fetch(0);
+        while (fill > keep) {
+            const TscRec next = fetch(kTscPerStep);
+            const int cnt = fill < kTscPerStep ? fill : kTscPerStep;
+            tsc_step(cur, cnt, slot, o0, o1, b0, npix, periodic, acc);
+            fill -= cnt;
+            head += cnt;
+            head -= head >= kTscQueue ? kTscQueue : 0;
+            cur = next;
         }
         __builtin_amdgcn_wave_barrier();
     }
-    if (tail > head)
-        tsc_step(gq, queue, head, tail - head, ln, b0, npix, periodic, acc);
     __syncthreads();
-    for (int t = 0; t < kTX; ++t) {
-        const int64_t i = b0[0] + t;
-        if (i < npix && j < npix && k < npix) {
-            const int64_t idx = (i * npix + j) * npix + k;
-            grid[idx] = acc[0][t * kWave + ln];
-            grid[nd + idx] = acc[1][t * kWave + ln];
+    for (int t = 0; t < kTX && b0[0] + t < npix; ++t)
+        if (in) {
+            out[t * plane] = acc[0][t * kWave + ln];
+            out[nd + t * plane] = acc[1][t * kWave + ln];
         }
-    }
 }
 
 int tsc_key_bits(int64_t npix)
 {
     const int64_t nbr = tsc_nbricks(npix);
     int bits = 1;
-    while (bits < 32 && ((int64_t)1 << bits) <= nbr)
+    while (bits < 32 - kTscFlagBits && ((int64_t)1 << bits) <= nbr)
         ++bits;
-    return bits;
+    return kTscFlagBits + bits;
 }
 
 void launch_tsc_keys(int dtype, const void *pos, int64_t n, int64_t npix, double len2pix,
@@ -423,12 +456,15 @@ void launch_tsc_prep(int dtype, const void *pos, const void *binq, const int32_t
                            cell);
 }
 
-void launch_tsc_gather(const double4 *gq, const uint64_t *cell, const int64_t *off,
-                       int64_t npix, int periodic, double *grid, hipStream_t s)
+int tsc_key_begin_bit() { return kTscFlagBits; }
+
+void launch_tsc_gather(const double4 *gq, const uint64_t *cell, const uint32_t *sorted_keys,
+                       const int64_t *off, int64_t npix, int periodic, double *grid,
+                       hipStream_t s)
 {
     const int64_t nbr = tsc_nbricks(npix);
-    hipLaunchKernelGGL(k_tsc_gather, dim3((unsigned)nbr), dim3(kWave), 0, s, gq, cell, off,
-                       npix, periodic, grid);
+    hipLaunchKernelGGL(k_tsc_gather, dim3((unsigned)nbr), dim3(kWave), 0, s, gq, cell,
+                       sorted_keys, off, (int)npix, periodic, grid);
 }
 
 }  // namespace s2g

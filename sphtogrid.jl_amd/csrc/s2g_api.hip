@@ -2085,13 +2085,13 @@ static void tsc_run(int dtype, const void *d_pos, const void *d_q, int64_t n, in
     if (n > 0) {
         launch_tsc_keys(dtype, d_pos, n, npix, len2pix, periodic, w.keys, w.vals, s);
         sort_pairs(w.sort_tmp, w.sort_bytes, w.keys, w.keys + n, w.vals, w.vals + n, n,
-                   tsc_key_bits(npix), s);
+                   tsc_key_bits(npix), s, tsc_key_begin_bit());
     }
     // n == 0: every offset is 0 (no key is read)
     launch_tsc_offsets(w.keys + n, n, npix, w.off, s);
     launch_tsc_prep(dtype, d_pos, d_q, w.vals + n, w.off, n, npix, len2pix, periodic, w.gq,
                     w.cell, s);
-    launch_tsc_gather(w.gq, w.cell, w.off, npix, periodic, d_grid, s);
+    launch_tsc_gather(w.gq, w.cell, w.keys + n, w.off, npix, periodic, d_grid, s);
 }
 
 // the same on the context's buffers (grown as needed)
@@ -2106,7 +2106,7 @@ static void tsc_ctx(s2g_ctx *c, int dtype, const void *d_pos, const void *d_q, i
     w.off = (int64_t *)c->tsc_off.get(sizeof(int64_t) * (size_t)(tsc_nbricks(npix) + 1));
     w.gq = (double4 *)c->tsc_gq.get(sizeof(double4) * m);
     w.cell = (uint64_t *)c->tsc_cell.get(8 * m);
-    w.sort_bytes = n > 0 ? sort_pairs_tmp_bytes(n, tsc_key_bits(npix)) : 0;
+    w.sort_bytes = n > 0 ? sort_pairs_tmp_bytes(n, tsc_key_bits(npix), tsc_key_begin_bit()) : 0;
     w.sort_tmp = c->sort_tmp.get(w.sort_bytes ? w.sort_bytes : 1);
     tsc_run(dtype, d_pos, d_q, n, npix, params->len2pix, (flags & S2G_FLAG_PERIODIC) ? 1 : 0, w,
             d_grid, s);
@@ -2191,7 +2191,7 @@ int s2g_tsc3d_device_noalloc(s2g_ctx *c, int dtype, const void *d_pos, const voi
         if (!c->scratch)
             throw Error(S2G_EHIP, "fixed work space unavailable: " + c->scratch_err);
         const int64_t npix = params->npixels;
-        const size_t sb = n > 0 ? sort_pairs_tmp_bytes(n, tsc_key_bits(npix)) : 0;
+        const size_t sb = n > 0 ? sort_pairs_tmp_bytes(n, tsc_key_bits(npix), tsc_key_begin_bit()) : 0;
         const size_t need = tsc_work_bytes(n, npix, sb);
         if (need > kScratchBytes)
             throw Error(S2G_EUNSUPPORTED, "work space of " + std::to_string(need) +

@@ -87,3 +87,24 @@ def test_tsc_mapping_average(s2g, orc):
     img2 = s2g.tsc_mapping(pos, q, param=par, dimensions=2, average=False)
     assert img2.shape == (24, 24)
     np.testing.assert_allclose(img2.sum(), ref[:, 0].sum(), rtol=1e-12)
+
+
+@pytest.mark.parametrize("periodic", [False, True])
+@pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 8, 15, 16, 17, 32, 33])
+def test_tsc_brick_edges(s2g, orc, N, periodic):
+    """Grids of one brick, of whole bricks and of a partial last brick along
+    each axis (4 x 4 x 16 cells), with particles on cell and brick faces, just
+    past the grid's edges and, for the small grids, more particles per brick
+    than its queue holds: a particle is taken by every brick its stencil
+    reaches, once."""
+    r = np.random.default_rng(100 + N)
+    n = 3000
+    cells = r.integers(-2, N + 3, (n, 3)).astype(np.float64)
+    cells[::2] = r.integers(0, (N + 3) // 4 + 1, cells[::2].shape) * 4.0
+    g = cells + r.choice([-1e-9, 0.0, 1e-9, 0.5, 0.9], (n, 3))
+    pos = (g - 0.5 * N) / N
+    q = r.uniform(-1, 3, n)
+    got = _tsc_gpu(s2g, pos, q, N, periodic, np.float64)
+    ref = orc.tsc_3d(pos, q, N, float(N), periodic)
+    # n weights of order one per cell at most: 3000 roundings of 1.1e-16
+    np.testing.assert_allclose(got, ref, rtol=1e-12, atol=1e-12)
