@@ -149,11 +149,13 @@ typedef struct s2g_tuning {
                                     (>= 5 keeps every particle of hsml < 2 px, whose
                                     weights need FP64, in the scatter) */
     int32_t small_item_min;      /* least particles per small-footprint work item;
-                                    16..4096, default 256 */
+                                    16..4096, default 256 (half of it in a pass of at
+                                    most 2^18 particles) */
     int32_t small_items_per_cu;  /* small-footprint work items per CU aimed at;
                                     1..64, default 16 */
     int32_t gather_item_min;     /* least (tile, particle) pairs per gather work item;
-                                    8..4096, default 64 */
+                                    8..4096, default 64 (twice that where a launch
+                                    accumulates three or four FP64 planes) */
     int32_t gather_items_per_cu; /* gather work items per CU aimed at; 1..256, default 16 */
     int32_t gather_planes;       /* image planes per gather launch; 1..4, default 4 */
     int32_t small_planes;        /* image planes per small-footprint launch; 1..4, default 4 */

@@ -56,9 +56,10 @@ struct GatherArgs {
     int add = 0;  // finalize adds its sums to the image instead of storing them
 };
 
-// setup over all particles of the pass: records and the class array
+// setup over all particles of the pass: records, the class array and the
+// partition's per-block class counts
 void launch_2d_setup(int dtype, const Map2D *maps, int nmaps, int64_t ntot, int nq, int kernel,
-                     Rec2 *rec, int32_t *cls, hipStream_t s);
+                     Rec2 *rec, int32_t *cls, int64_t *counts, hipStream_t s);
 // ne: the count, or with d_bounds its upper bound (the count then being
 // d_bounds[3] - d_bounds[2] on the device)
 void launch_2d_norm(int kernel, const int32_t *list, int64_t ne, const Map2D *maps, Rec2 *rec,

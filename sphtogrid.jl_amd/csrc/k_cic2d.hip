@@ -30,14 +30,9 @@ namespace s2g {
 // calculate_weights (cic_2D.jl:49-69), all in FP64 without FMA contraction.
 // ---------------------------------------------------------------------------
 template <typename T>
-__global__ __launch_bounds__(256) void k2d_setup(const Map2D *__restrict__ maps, int nmaps,
-                                                 int64_t ntot, int nq, int kernel,
-                                                 Rec2 *__restrict__ rec,
-                                                 int32_t *__restrict__ cls)
+__device__ __forceinline__ Rec2 setup2d(const Map2D *__restrict__ maps, int nmaps, int64_t p,
+                                        int nq, int kernel)
 {
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= ntot)
-        return;
     const int mi = find_entry(maps, nmaps, p, [](const Map2D &e) { return e.pbase; });
     const Map2D &md = maps[mi];
     const int64_t pl = p - md.pbase;
@@ -60,9 +55,7 @@ __global__ __launch_bounds__(256) void k2d_setup(const Map2D *__restrict__ maps,
         if (ld(binq, pl * nq + q) != 0.0)
             allzero = false;
     if (allzero && !(flags & S2G_FLAG_CALC_MEAN)) {
-        rec[p] = r;
-        cls[p] = r.cls;
-        return;
+        return r;
     }
 
     const double h = mul_rn(ld(hsml, pl), len2pix);
@@ -79,9 +72,7 @@ __global__ __launch_bounds__(256) void k2d_setup(const Map2D *__restrict__ maps,
     double xa = floor(sub_rn(x, h)), xb = floor(add_rn(x, h));
     double ya = floor(sub_rn(y, h)), yb = floor(add_rn(y, h));
     if (!(xa == xa) || !(xb == xb) || !(ya == ya) || !(yb == yb) || !(h > 0.0)) {
-        rec[p] = r;  // NaN input or h <= 0: nothing is deposited
-        cls[p] = r.cls;
-        return;
+        return r;  // NaN input or h <= 0: nothing is deposited
     }
     xa = fmin(fmax(xa, -1.0), lim);
     xb = fmin(fmax(xb, -1.0), lim);
@@ -91,9 +82,7 @@ __global__ __launch_bounds__(256) void k2d_setup(const Map2D *__restrict__ maps,
     const int64_t i0 = a0 > 0 ? a0 : 0, i1 = a1 < npix - 1 ? a1 : npix - 1;
     const int64_t j0 = b0 > 0 ? b0 : 0, j1 = b1 < npix - 1 ? b1 : npix - 1;
     if (i0 > i1 || j0 > j1) {
-        rec[p] = r;
-        cls[p] = r.cls;
-        return;
+        return r;
     }
 
     // Fallback iff no footprint pixel centre has u < 1 (u from the
@@ -137,9 +126,28 @@ __global__ __launch_bounds__(256) void k2d_setup(const Map2D *__restrict__ maps,
             r.s = num;
         }
     }
-    rec[p] = r;
-    cls[p] = r.cls;
+    return r;
 }
+
+// counts: the partition's per-block class counts
+template <typename T>
+__global__ __launch_bounds__(kPartBlock) void k2d_setup(const Map2D *__restrict__ maps, int nmaps,
+                                                        int64_t ntot, int nq, int kernel,
+                                                        Rec2 *__restrict__ rec,
+                                                        int32_t *__restrict__ cls,
+                                                        int64_t *__restrict__ counts)
+{
+    const int64_t p = (int64_t)blockIdx.x * kPartBlock + threadIdx.x;
+    int c = kClsSkip;
+    if (p < ntot) {
+        const Rec2 r = setup2d<T>(maps, nmaps, p, nq, kernel);
+        rec[p] = r;
+        c = r.cls;
+        cls[p] = c;
+    }
+    block_class_counts(c, counts);
+}
+
 
 // ---------------------------------------------------------------------------
 // Pixel weights shared by the normalisation sum and the tile gather: both
@@ -320,8 +328,8 @@ constexpr int gather_stage(int np, bool f64) { return 2 * gather_batch(np, f64);
 // A: the accumulator type, double, or float with S2G_FLAG_FP32_ACCUM (an
 // item's pixel sums in FP32, written to its FP64 partials)
 // d_nitems (null in a call sized on the host): the item count on the device,
-// the grid being its upper bound; d_flag != 0 (a replay whose pair lists
-// outgrew their capacity): no item runs
+// the grid being its upper bound; *d_flag != 0 (d_flag may be null; a replay
+// whose pair lists outgrew their capacity): no item runs
 template <typename T, int K, int NP, typename A>
 __device__ __forceinline__ void gather_tile(const int4 *__restrict__ items,
                                             const int32_t *__restrict__ pairs,
@@ -331,7 +339,7 @@ __device__ __forceinline__ void gather_tile(const int4 *__restrict__ items,
                                             const int64_t *__restrict__ d_nitems,
                                             const int *__restrict__ d_flag)
 {
-    if (d_nitems && ((int64_t)blockIdx.x >= *d_nitems || *d_flag))
+    if (d_nitems && ((int64_t)blockIdx.x >= *d_nitems || (d_flag && *d_flag)))
         return;  // the whole block
     constexpr int kGBatch = gather_batch(NP, sizeof(A) == 8);
     constexpr int kGStage = gather_stage(NP, sizeof(A) == 8);
@@ -921,16 +929,17 @@ __global__ __launch_bounds__(256) void k2d_reduce_maps(const Map2D *__restrict__
     }
 
 void launch_2d_setup(int dtype, const Map2D *maps, int nmaps, int64_t ntot, int nq, int kernel,
-                     Rec2 *rec, int32_t *cls, hipStream_t s)
+                     Rec2 *rec, int32_t *cls, int64_t *counts, hipStream_t s)
 {
     if (ntot == 0)
         return;
-    const dim3 g((unsigned)((ntot + 255) / 256)), b(256);
+    const dim3 g((unsigned)partition_blocks(ntot)), b(kPartBlock);
     if (dtype == S2G_F32)
-        hipLaunchKernelGGL(k2d_setup<float>, g, b, 0, s, maps, nmaps, ntot, nq, kernel, rec, cls);
+        hipLaunchKernelGGL(k2d_setup<float>, g, b, 0, s, maps, nmaps, ntot, nq, kernel, rec, cls,
+                           counts);
     else
-        hipLaunchKernelGGL(k2d_setup<double>, g, b, 0, s, maps, nmaps, ntot, nq, kernel, rec,
-                           cls);
+        hipLaunchKernelGGL(k2d_setup<double>, g, b, 0, s, maps, nmaps, ntot, nq, kernel, rec, cls,
+                           counts);
 }
 
 void launch_2d_norm(int kernel, const int32_t *list, int64_t ne, const Map2D *maps, Rec2 *rec,

@@ -9,7 +9,8 @@ using Map3DArgs = Map2DArgs;  // same fields; binq is scalar (nq == 1)
 
 struct Gather3Args {
     int dtype, kernel, np, plane0, nq, nb;
-    int64_t ntiles, nitems, npix;
+    int64_t ntiles, nitems, npix;  // nitems: the count, or its upper bound with d_nitems
+    const int64_t *d_nitems = nullptr;
     const int4 *items;
     const int32_t *pairs;  // particle index per (tile, particle) pair
     const Rec3 *rec;
@@ -29,7 +30,8 @@ struct Small3Args {
     double *image;
 };
 
-void launch_3d_setup(const Map3DArgs &a, Rec3 *rec, int32_t *cls, hipStream_t s);
+// counts: the partition's per-block class counts
+void launch_3d_setup(const Map3DArgs &a, Rec3 *rec, int32_t *cls, int64_t *counts, hipStream_t s);
 // explicit normalisation sums (flags: S2G_FLAG_EXACT_NORM turns off the
 // border-cut closed form)
 void launch_3d_norm(int kernel, const int32_t *list, int64_t ne, int64_t npix, uint32_t flags,
@@ -39,7 +41,6 @@ void launch_3d_finalize(const Gather3Args &g, hipStream_t s);
 void launch_3d_small(const Small3Args &a, hipStream_t s);
 // windowed small scatter: particles sorted by the kST3^3 tile (nt per side)
 // of their box's first voxel, one block per work item (at most max_items)
-constexpr int kST3 = 9;
 void launch_3d_small_keys(const int32_t *list, int64_t ns, const Rec3 *rec, int nt,
                           uint32_t *keys, int32_t *vals, hipStream_t s);
 void launch_3d_small_window(const Small3Args &a, const int4 *items, const int64_t *nitems,

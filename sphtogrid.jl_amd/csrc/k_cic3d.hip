@@ -15,19 +15,12 @@ namespace s2g {
 // calculate_weights (cic_3D.jl:55-75), FP64 without contraction.
 // ---------------------------------------------------------------------------
 template <typename T>
-__global__ __launch_bounds__(256) void k3d_setup(const T *__restrict__ pos,
-                                                 const T *__restrict__ hsml,
-                                                 const T *__restrict__ m,
-                                                 const T *__restrict__ rho,
-                                                 const T *__restrict__ binq,
-                                                 const T *__restrict__ w, int64_t n,
-                                                 int64_t npix, double len2pix, int kernel,
-                                                 uint32_t flags, Rec3 *__restrict__ rec,
-                                                 int32_t *__restrict__ cls)
+__device__ __forceinline__ Rec3 setup3d(const T *__restrict__ pos, const T *__restrict__ hsml,
+                                        const T *__restrict__ m, const T *__restrict__ rho,
+                                        const T *__restrict__ binq, const T *__restrict__ w,
+                                        int64_t npix, double len2pix, int kernel, uint32_t flags,
+                                        int64_t p)
 {
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n)
-        return;
     Rec3 r;
     r.x = r.y = r.z = r.h = r.s = 0.0;
     r.i0 = r.j0 = r.k0 = 0;
@@ -36,9 +29,7 @@ __global__ __launch_bounds__(256) void k3d_setup(const T *__restrict__ pos,
     r.fb = 0;
     // cic_3D.jl:140-144
     if (ld(binq, p) == 0.0 && !(flags & S2G_FLAG_CALC_MEAN)) {
-        rec[p] = r;
-        cls[p] = r.cls;
-        return;
+        return r;
     }
     const double h = mul_rn(ld(hsml, p), len2pix);
     const double l3 = mul_rn(mul_rn(len2pix, len2pix), len2pix);
@@ -67,9 +58,7 @@ __global__ __launch_bounds__(256) void k3d_setup(const T *__restrict__ pos,
             bad = true;
     }
     if (bad) {
-        rec[p] = r;
-        cls[p] = r.cls;
-        return;
+        return r;
     }
     // fallback iff no voxel centre of the footprint has u < 1 (FP64, nearest
     // centre per axis; three candidates cover ties and clamping)
@@ -115,9 +104,28 @@ __global__ __launch_bounds__(256) void k3d_setup(const T *__restrict__ pos,
         r.cls = kClsLargeEx;
         r.s = num;
     }
-    rec[p] = r;
-    cls[p] = r.cls;
+    return r;
 }
+
+// counts: the partition's per-block class counts
+template <typename T>
+__global__ __launch_bounds__(kPartBlock) void k3d_setup(
+    const T *__restrict__ pos, const T *__restrict__ hsml, const T *__restrict__ m,
+    const T *__restrict__ rho, const T *__restrict__ binq, const T *__restrict__ w, int64_t n,
+    int64_t npix, double len2pix, int kernel, uint32_t flags, Rec3 *__restrict__ rec,
+    int32_t *__restrict__ cls, int64_t *__restrict__ counts)
+{
+    const int64_t p = (int64_t)blockIdx.x * kPartBlock + threadIdx.x;
+    int c = kClsSkip;
+    if (p < n) {
+        const Rec3 r = setup3d(pos, hsml, m, rho, binq, w, npix, len2pix, kernel, flags, p);
+        rec[p] = r;
+        c = r.cls;
+        cls[p] = c;
+    }
+    block_class_counts(c, counts);
+}
+
 
 // ---------------------------------------------------------------------------
 // Explicit normalisation: one wave per particle.  The voxel weights are
@@ -372,8 +380,12 @@ __global__ __launch_bounds__(256, 4) void k3d_gather(const int4 *__restrict__ it
                                                      const Rec3 *__restrict__ rec,
                                                      const T *__restrict__ binq, int nq,
                                                      int plane0, int nb,
-                                                     double *__restrict__ partial)
+                                                     double *__restrict__ partial,
+                                                     const int64_t *__restrict__ d_nitems)
 {
+    // d_nitems: the item count on the device, the grid being its upper bound
+    if (d_nitems && (int64_t)blockIdx.x >= *d_nitems)
+        return;  // the whole block
     __shared__ float2 s_tab[3][kGBatch3][kBT];
     __shared__ uint32_t s_hit[kGBatch3][2];
     __shared__ double s_c[kGBatch3][3], s_h[kGBatch3];
@@ -893,21 +905,21 @@ __global__ void k3d_reduce(const double *__restrict__ image, int64_t nd, int red
     default: { constexpr int KK = S2G_KERNEL_WENDLAND_C8; CALL; } break;       \
     }
 
-void launch_3d_setup(const Map3DArgs &a, Rec3 *rec, int32_t *cls, hipStream_t s)
+void launch_3d_setup(const Map3DArgs &a, Rec3 *rec, int32_t *cls, int64_t *counts, hipStream_t s)
 {
     if (a.n == 0)
         return;
-    const dim3 g((unsigned)((a.n + 255) / 256)), blk(256);
+    const dim3 g((unsigned)partition_blocks(a.n)), blk(kPartBlock);
     if (a.dtype == S2G_F32)
         hipLaunchKernelGGL(k3d_setup<float>, g, blk, 0, s, (const float *)a.pos,
                            (const float *)a.hsml, (const float *)a.m, (const float *)a.rho,
                            (const float *)a.binq, (const float *)a.w, a.n, a.npix, a.len2pix,
-                           a.kernel, a.flags, rec, cls);
+                           a.kernel, a.flags, rec, cls, counts);
     else
         hipLaunchKernelGGL(k3d_setup<double>, g, blk, 0, s, (const double *)a.pos,
                            (const double *)a.hsml, (const double *)a.m, (const double *)a.rho,
                            (const double *)a.binq, (const double *)a.w, a.n, a.npix,
-                           a.len2pix, a.kernel, a.flags, rec, cls);
+                           a.len2pix, a.kernel, a.flags, rec, cls, counts);
 }
 
 void launch_3d_norm(int kernel, const int32_t *list, int64_t ne, int64_t npix, uint32_t flags,
@@ -926,10 +938,10 @@ static void gather3_tk(const Gather3Args &g, hipStream_t s)
     const dim3 grid((unsigned)g.nitems), blk(256);
     if (g.np == 1)
         hipLaunchKernelGGL((k3d_gather<T, K, 1>), grid, blk, 0, s, g.items, g.pairs,
-                           g.rec, (const T *)g.binq, g.nq, g.plane0, g.nb, g.partial);
+                           g.rec, (const T *)g.binq, g.nq, g.plane0, g.nb, g.partial, g.d_nitems);
     else
         hipLaunchKernelGGL((k3d_gather<T, K, 2>), grid, blk, 0, s, g.items, g.pairs,
-                           g.rec, (const T *)g.binq, g.nq, g.plane0, g.nb, g.partial);
+                           g.rec, (const T *)g.binq, g.nq, g.plane0, g.nb, g.partial, g.d_nitems);
 }
 
 void launch_3d_gather(const Gather3Args &g, hipStream_t s)

@@ -15,10 +15,55 @@ constexpr int kPairChunk = 4096;
 constexpr int kMaxTiles = 16384;
 
 int64_t partition_blocks(int64_t n);
-// counts: 3*partition_blocks(n)+1 int64; afterwards counts[c*nb] is the first
-// index of class c in the concatenation and counts[3*nb] the grand total
+// counts: 3*partition_blocks(n)+1 int64, the per-block class counts as the
+// setup kernels write them (block_class_counts); afterwards counts[c*nb] is
+// the first index of class c in the concatenation and counts[3*nb] the grand
+// total
 void launch_partition(const int32_t *cls, int64_t n, int64_t *counts, int64_t *scan_tmp,
                       int32_t *l0, int32_t *l1, int32_t *l2, hipStream_t s);
+// The partition and the class bounds of a small pass (at most kPartLight
+// blocks) in one launch instead of four: every block adds up the counts of
+// the blocks before it.  out as launch_class_bounds writes it; counts is left
+// as it is.
+constexpr int64_t kPartLight = 1024;
+void launch_partition_light(const int32_t *cls, int64_t n, const int64_t *counts,
+                            const int64_t *pbase, int nmaps, int32_t *l0, int32_t *l1,
+                            int32_t *l2, int64_t *out, hipStream_t s);
+
+// class membership of the three lists: small, large (closed form or explicit
+// normalisation), large with explicit normalisation
+__device__ __forceinline__ void part_flags(int cls, int &f0, int &f1, int &f2)
+{
+    f0 = cls == kClsSmall;
+    f1 = cls == kClsLargeAn || cls == kClsLargeEx;
+    f2 = cls == kClsLargeEx;
+}
+
+// Per-block class counts of the partition, from the setup kernel's blocks of
+// kPartBlock threads (cls: this thread's particle's class, kClsSkip past the
+// end; every thread of the block calls it)
+__device__ __forceinline__ void block_class_counts(int cls, int64_t *__restrict__ counts)
+{
+    __shared__ int s[3][kPartBlock / kWave];
+    int f0, f1, f2;
+    part_flags(cls, f0, f1, f2);
+    const int wv = threadIdx.x / kWave, ln = threadIdx.x % kWave;
+    const uint64_t b0 = __ballot(f0), b1 = __ballot(f1), b2 = __ballot(f2);
+    if (ln == 0) {
+        s[0][wv] = __popcll(b0);
+        s[1][wv] = __popcll(b1);
+        s[2][wv] = __popcll(b2);
+    }
+    __syncthreads();
+    if (threadIdx.x < 3) {
+        int t = 0;
+        for (int k = 0; k < kPartBlock / kWave; ++k)
+            t += s[threadIdx.x][k];
+        counts[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = t;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 3)
+        counts[3 * (int64_t)gridDim.x] = 0;  // becomes the grand total after the scan
+}
 // After launch_partition over the particles of several maps: out[0..3] =
 // class offsets counts[0], counts[nb], counts[2nb], counts[3nb]; out[4 + m] =
 // first entry of map m in the large list (particles of map m are
@@ -55,14 +100,25 @@ template <typename R>
 void launch_pairs(const int32_t *large, const R *rec, const PairChunk *chunks, int nchunks,
                   const TileMap *tmaps, int max_tiles, int64_t *cnt, int64_t ncnt,
                   int64_t *scan_tmp, int32_t *pairs_or_null, bool fill, hipStream_t s,
-                  const int64_t *lbase, int64_t cap = INT64_MAX);
+                  const int64_t *lbase, int64_t cap = INT64_MAX, bool scan = true);
 // small-footprint buckets as per-tile lists (fill == false: counts per
 // (tile, chunk) + scan into cnt; fill == true: out = the particles, tile t of
 // map m at cnt[cbase + t nch] ..), chunk ranges from lbase as for the pairs
-void launch_anchor_lists(const int32_t *list, const Rec2 *rec, const PairChunk *chunks,
+template <typename R>
+void launch_anchor_lists(const int32_t *list, const R *rec, const PairChunk *chunks,
                          int nchunks, const TileMap *tmaps, int max_tiles, int64_t *cnt,
                          int64_t ncnt, int64_t *scan_tmp, int32_t *out, bool fill,
-                         const int64_t *lbase, hipStream_t s);
+                         const int64_t *lbase, hipStream_t s, bool scan = true);
+// The scan of the counts of launch_pairs / launch_anchor_lists (called with
+// scan == false) and both steps of launch_items in one block, for counts of a
+// small pass: ncnt <= kListsLight and totals below 2^31 (three launches and
+// more otherwise, each a few microseconds).  items: at most item_cap are
+// written; nitems[ntiles] is the item total.
+constexpr int64_t kListsLight = 131072;
+void launch_lists_light(int64_t *cnt, int64_t ncnt, const TileMap *tmaps, int nmaps, int ntiles,
+                        int64_t gmin, int64_t target, int64_t gmax, int64_t tmax,
+                        const int64_t *total, int64_t *nitems, int4 *items, int64_t item_cap,
+                        int64_t *tile_items, hipStream_t s);
 // flag = (a map's large list outgrew nch * csz entries) | 2 * (pair total >
 // pair_cap), for a replayed pass sized at creation
 void launch_plan_check(const int64_t *lbase, int nmaps, const TileMap *tmaps,

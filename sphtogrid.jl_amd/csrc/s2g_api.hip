@@ -38,6 +38,8 @@ struct s2g_ctx {
     // explicit normalisation and the small-footprint scatter run there beside
     // the pair lists and the gather, ordered by the fork / join events
     hipStream_t side = nullptr;
+    // of a light pass: the small-footprint scatter beside the normalisation too
+    hipStream_t side2 = nullptr;
     hipEvent_t fork = nullptr, normed = nullptr, smalled = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     static constexpr int kNumStageEvents = 80;
@@ -54,7 +56,7 @@ struct s2g_ctx {
     DevBuf skeys, svals, sort_tmp, soff, snitems, sitems, stile, sscan_tmp;
     // mass_density: particles, bounding-box partials, particles in cell order
     DevBuf md_P, md_bbox, md_S, md_tab;
-    PinnedBuf h_tab, h_bounds, h_tiles;
+    PinnedBuf h_tab, h_bounds, h_tiles, h_stage;
     // all-sky deposit
     DevBuf hp_rec, hp_nunits, hp_units, hp_part, hp_ring, hp_list, hp_rtab;
     // TSC: brick offsets, sorted grid coordinates + quantity, packed cells
@@ -166,7 +168,8 @@ float elapsed(hipEvent_t a, hipEvent_t b)
 // Shared large-particle stage: per-tile pair lists and work items.
 // ---------------------------------------------------------------------------
 struct TilePlan {
-    int64_t npairs = 0, nitems = 0;
+    int64_t npairs = 0, nitems = 0;  // nitems: with d_nitems its upper bound
+    const int64_t *d_npairs = nullptr, *d_nitems = nullptr;  // light pass: totals on the device
     int32_t *pairs = nullptr;
     int4 *items = nullptr;
     int64_t *tile_items = nullptr;
@@ -182,7 +185,7 @@ struct TilePlan {
 // ms; 4096-pair items, about 260 per CU, 246.2 ms).
 TilePlan build_tile_lists(s2g_ctx *c, const int32_t *large, const void *rec, bool rec3,
                           std::vector<TileMap> &tm, const std::vector<int64_t> &lbase,
-                          const int64_t *d_lbase, int ntiles, hipStream_t s, double *ms_sort,
+                          const int64_t *d_lbase, int ntiles, hipStream_t s, bool timed,
                           int64_t gmin = 64, int64_t per_cu = 16, int64_t gmax = 0)
 {
     hipEvent_t *E = c->stage;
@@ -230,7 +233,8 @@ TilePlan build_tile_lists(s2g_ctx *c, const int32_t *large, const void *rec, boo
     // larger when maps of the pass have no large particle) share it
     const int64_t nscan = ncnt > (int64_t)ntiles + 1 ? ncnt : (int64_t)ntiles + 1;
     int64_t *tmp = (int64_t *)c->scan_tmp.get(sizeof(int64_t) * scan_tmp_elems(nscan));
-    S2G_HIP(hipEventRecord(E[4], s));
+    if (timed)
+        S2G_HIP(hipEventRecord(E[4], s));
     if (rec3)
         launch_pairs<Rec3>(large, (const Rec3 *)rec, d_ch, nchunks, d_tm, max_tiles, cnt, ncnt,
                            tmp, nullptr, false, s, d_lbase);
@@ -244,7 +248,8 @@ TilePlan build_tile_lists(s2g_ctx *c, const int32_t *large, const void *rec, boo
     int64_t *nit = (int64_t *)c->nitems.get(sizeof(int64_t) * (ntiles + 1));
     launch_items(cnt, d_tm, nmaps, ntiles, gmin, target, d_npairs, nit, tmp, nullptr, nullptr,
                  false, s, gmax);
-    S2G_HIP(hipEventRecord(E[5], s));
+    if (timed)
+        S2G_HIP(hipEventRecord(E[5], s));
     int64_t tot[2];
     read_i64(c, s, {d_npairs, nit + ntiles}, tot);
     tp.npairs = tot[0];
@@ -254,7 +259,8 @@ TilePlan build_tile_lists(s2g_ctx *c, const int32_t *large, const void *rec, boo
     tp.pairs = (int32_t *)c->pairs.get(sizeof(int32_t) * (tp.npairs ? tp.npairs : 1));
     tp.items = (int4 *)c->items.get(sizeof(int4) * (tp.nitems ? tp.nitems : 1));
     tp.tile_items = (int64_t *)c->tile_items.get(sizeof(int64_t) * 2 * ntiles);
-    S2G_HIP(hipEventRecord(E[6], s));
+    if (timed)
+        S2G_HIP(hipEventRecord(E[6], s));
     if (rec3)
         launch_pairs<Rec3>(large, (const Rec3 *)rec, d_ch, nchunks, d_tm, max_tiles, cnt, ncnt,
                            tmp, tp.pairs, true, s, d_lbase);
@@ -263,10 +269,164 @@ TilePlan build_tile_lists(s2g_ctx *c, const int32_t *large, const void *rec, boo
                            tmp, tp.pairs, true, s, d_lbase);
     launch_items(cnt, d_tm, nmaps, ntiles, gmin, target, d_npairs, nit, tmp, tp.items,
                  tp.tile_items, true, s, gmax);
-    S2G_HIP(hipEventRecord(E[7], s));
-    S2G_HIP(hipEventSynchronize(E[7]));
-    *ms_sort = elapsed(E[4], E[5]) + elapsed(E[6], E[7]);
+    if (timed)
+        S2G_HIP(hipEventRecord(E[7], s));
     return tp;
+}
+
+// ---------------------------------------------------------------------------
+// Light passes: of few particles and tiles, where the launches and the host's
+// round trips take longer than the kernels.  One launch partitions the classes
+// (launch_partition_light), one scans each list's counts and cuts its items
+// (launch_lists_light), the small footprints are bucketed by the counting sort
+// instead of the radix sort, and the pair and item counts stay on the device
+// (capacities from true bounds), so the host reads back once, the class
+// sizes.  Measured whole calls: 65,536 particles on 256^2 @L1@ us; 4,096 on
+// 64^2 through sphMapping @L2@ us.
+// ---------------------------------------------------------------------------
+constexpr int64_t kLightPairs = (int64_t)1 << 24;     // pair capacity
+constexpr int64_t kLightPartial = (int64_t)1 << 29;   // bytes of item partials
+
+// Chunk size of a counting sort over `len` list entries and `ntl` tiles in a
+// light pass: at least `least` entries, grown until the counters are few
+int64_t light_chunk(int64_t len, int64_t ntl, int64_t least)
+{
+    int64_t csz = least;
+    while (ntl * ((len + csz - 1) / csz) >= kListsLight / 2 && csz < len)
+        csz *= 2;
+    return csz;
+}
+
+// A counting sort's tables for a light pass: per map the chunks of its list
+// segment lens[m]; returns the counter count, or -1 if it is no light one
+int64_t light_tables(std::vector<TileMap> &tm, const std::vector<int64_t> &lbase, int64_t least,
+                     std::vector<PairChunk> &chunks, int *max_tiles)
+{
+    int64_t cb = 0;
+    *max_tiles = 1;
+    for (size_t m = 0; m < tm.size(); ++m) {
+        const int64_t len = lbase[m + 1] - lbase[m];
+        if (tm[m].ntiles > kMaxTiles)
+            return -1;
+        *max_tiles = tm[m].ntiles > *max_tiles ? tm[m].ntiles : *max_tiles;
+        const int64_t csz = light_chunk(len, tm[m].ntiles, least);
+        const int64_t nch = (len + csz - 1) / csz;
+        tm[m].cbase = cb;
+        tm[m].nch = (int32_t)nch;
+        tm[m].csz = (int32_t)csz;
+        cb += tm[m].ntiles * nch;
+        for (int64_t k = 0; k < nch; ++k)
+            chunks.push_back(PairChunk{(int32_t)m, (int32_t)k});
+    }
+    return cb + 1 <= kListsLight ? cb + 1 : -1;
+}
+
+// Both lists' tables of a light pass, uploaded together on `s`.
+struct LightTables {
+    bool ok = false;
+    int64_t ncnt = 0, sncnt = 0, pair_cap = 0, item_cap = 0;
+    int nchunks = 0, snchunks = 0, max_tiles = 1, smax_tiles = 1;
+    const TileMap *d_tm = nullptr, *d_stm = nullptr;
+    const PairChunk *d_ch = nullptr, *d_sch = nullptr;
+};
+
+// tm / stm: tile grids of the large and of the small lists' maps (the small
+// ones may be empty: the caller buckets them otherwise); lbase / sbase: the
+// maps' list starts.  planes x plane_elems doubles of partials per item.
+LightTables light_lists(s2g_ctx *c, std::vector<TileMap> tm, const std::vector<int64_t> &lbase,
+                        std::vector<TileMap> stm, const std::vector<int64_t> &sbase, int ntiles,
+                        int64_t gmin, int64_t per_cu, int64_t partial_bytes, hipStream_t s)
+{
+    LightTables lt;
+    std::vector<PairChunk> ch, sch;
+    lt.ncnt = light_tables(tm, lbase, 64, ch, &lt.max_tiles);
+    lt.sncnt = light_tables(stm, sbase, 512, sch, &lt.smax_tiles);
+    for (size_t m = 0; m < tm.size(); ++m)
+        lt.pair_cap += (lbase[m + 1] - lbase[m]) * tm[m].ntiles;
+    const int64_t target = (int64_t)c->ncu * per_cu;
+    const int64_t byp = (lt.pair_cap + gmin - 1) / gmin;
+    lt.item_cap = ntiles + (byp < target ? byp : target);
+    if (lt.ncnt < 0 || lt.sncnt < 0 || lt.pair_cap > kLightPairs ||
+        lt.item_cap * partial_bytes > kLightPartial)
+        return lt;
+    const size_t b0 = sizeof(TileMap) * tm.size(), b1 = sizeof(TileMap) * stm.size();
+    const size_t b2 = sizeof(PairChunk) * ch.size(), b3 = sizeof(PairChunk) * sch.size();
+    char *h = (char *)c->h_tiles.get(b0 + b1 + b2 + b3);
+    std::memcpy(h, tm.data(), b0);
+    std::memcpy(h + b0, stm.data(), b1);
+    std::memcpy(h + b0 + b1, ch.data(), b2);
+    std::memcpy(h + b0 + b1 + b2, sch.data(), b3);
+    char *d = (char *)c->tiles.get_roomy(b0 + b1 + b2 + b3);
+    S2G_HIP(hipMemcpyAsync(d, h, b0 + b1 + b2 + b3, hipMemcpyHostToDevice, s));
+    lt.d_tm = (const TileMap *)d;
+    lt.d_stm = (const TileMap *)(d + b0);
+    lt.d_ch = (const PairChunk *)(d + b0 + b1);
+    lt.d_sch = (const PairChunk *)(d + b0 + b1 + b2);
+    lt.nchunks = (int)ch.size();
+    lt.snchunks = (int)sch.size();
+    lt.ok = true;
+    return lt;
+}
+
+// The pair lists and items of a light pass, sized by the tables' bounds.
+template <typename R>
+TilePlan light_tile_lists(s2g_ctx *c, const int32_t *large, const R *rec, const LightTables &lt,
+                          int nmaps, const int64_t *d_lbase, int ntiles, hipStream_t s,
+                          bool timed, int64_t gmin, int64_t per_cu, int64_t gmax)
+{
+    hipEvent_t *E = c->stage;
+    TilePlan tp;
+    int64_t *cnt = (int64_t *)c->cnt.get_roomy(sizeof(int64_t) * lt.ncnt);
+    int64_t *nit = (int64_t *)c->nitems.get(sizeof(int64_t) * (ntiles + 1));
+    tp.pairs = (int32_t *)c->pairs.get_roomy(sizeof(int32_t) * (lt.pair_cap ? lt.pair_cap : 1));
+    tp.items = (int4 *)c->items.get_roomy(sizeof(int4) * lt.item_cap);
+    tp.tile_items = (int64_t *)c->tile_items.get(sizeof(int64_t) * 2 * ntiles);
+    tp.nitems = lt.item_cap;
+    tp.d_npairs = cnt + lt.ncnt - 1;
+    tp.d_nitems = nit + ntiles;
+    if (timed)
+        S2G_HIP(hipEventRecord(E[4], s));
+    launch_pairs<R>(large, rec, lt.d_ch, lt.nchunks, lt.d_tm, lt.max_tiles, cnt, lt.ncnt, nullptr,
+                    nullptr, false, s, d_lbase, INT64_MAX, false);
+    // item_cap covers every item: ntiles + ceil(total / G) with G >= gmin
+    // and G >= total / target (gmax applies within that: tmax)
+    const int64_t target = (int64_t)c->ncu * per_cu;
+    launch_lists_light(cnt, lt.ncnt, lt.d_tm, nmaps, ntiles, gmin, target, gmax, target,
+                       tp.d_npairs, nit, tp.items, lt.item_cap, tp.tile_items, s);
+    launch_pairs<R>(large, rec, lt.d_ch, lt.nchunks, lt.d_tm, lt.max_tiles, cnt, lt.ncnt, nullptr,
+                    tp.pairs, true, s, d_lbase, lt.pair_cap, false);
+    if (timed) {
+        S2G_HIP(hipEventRecord(E[5], s));
+        S2G_HIP(hipEventRecord(E[6], s));
+        S2G_HIP(hipEventRecord(E[7], s));
+    }
+    return tp;
+}
+
+// The small list's buckets and items (at most max_items) of a light pass;
+// returns the particles in bucket order.
+struct SmallItems {
+    const int32_t *plist = nullptr;
+    const int4 *items = nullptr;
+    const int64_t *d_nitems = nullptr;
+};
+template <typename R>
+SmallItems light_small_lists(s2g_ctx *c, const int32_t *list, int64_t ns, const R *rec,
+                             const LightTables &lt, int nmaps, const int64_t *d_sbase,
+                             int nstiles, int64_t Gs, int64_t max_items, hipStream_t s)
+{
+    int64_t *cnt = (int64_t *)c->soff.get_roomy(sizeof(int64_t) * lt.sncnt);
+    int32_t *out = (int32_t *)c->svals.get_roomy(sizeof(int32_t) * 2 * ns);
+    int64_t *nit = (int64_t *)c->snitems.get(sizeof(int64_t) * (nstiles + 1));
+    int4 *items = (int4 *)c->sitems.get_roomy(sizeof(int4) * max_items);
+    int64_t *stile = (int64_t *)c->stile.get(sizeof(int64_t) * 2 * nstiles);
+    launch_anchor_lists<R>(list, rec, lt.d_sch, lt.snchunks, lt.d_stm, lt.smax_tiles, cnt,
+                           lt.sncnt, nullptr, nullptr, false, d_sbase, s, false);
+    launch_lists_light(cnt, lt.sncnt, lt.d_stm, nmaps, nstiles, Gs, 1, 0, 0, nullptr, nit, items,
+                       max_items, stile, s);
+    launch_anchor_lists<R>(list, rec, lt.d_sch, lt.snchunks, lt.d_stm, lt.smax_tiles, cnt,
+                           lt.sncnt, nullptr, out, true, d_sbase, s, false);
+    return SmallItems{out, items, nit + nstiles};
 }
 
 struct ClassLists {
@@ -274,32 +434,48 @@ struct ClassLists {
     int32_t *l0 = nullptr, *l1 = nullptr, *l2 = nullptr;
     std::vector<int64_t> lbase;  // per-map first large-list entry (+ the total)
     const int64_t *d_lbase = nullptr;  // the same on the device
+    std::vector<int64_t> sbase;  // the same of the small list
+    const int64_t *d_sbase = nullptr;
 };
 
-// stable class partition of the pass's particles and one read-back of the
-// class sizes and of the per-map large-list bounds
-ClassLists partition_classes(s2g_ctx *c, const int32_t *cls, int64_t n, const int64_t *d_pbase,
-                             int nmaps, hipStream_t s)
+// the per-block class counts that the setup kernels write
+int64_t *class_counts(s2g_ctx *c, int64_t n)
+{
+    return (int64_t *)c->counts.get(sizeof(int64_t) * (3 * partition_blocks(n) + 1));
+}
+
+// stable class partition of the pass's particles (counts: class_counts, filled
+// by the setup) and one read-back of the class sizes and of the per-map list
+// bounds
+ClassLists partition_classes(s2g_ctx *c, const int32_t *cls, int64_t n, int64_t *counts,
+                             const int64_t *d_pbase, int nmaps, hipStream_t s, bool timed)
 {
     ClassLists cl;
     const int64_t nb = partition_blocks(n);
-    int64_t *counts = (int64_t *)c->counts.get(sizeof(int64_t) * (3 * nb + 1));
     cl.l0 = (int32_t *)c->lists[0].get(sizeof(int32_t) * n);
     cl.l1 = (int32_t *)c->lists[1].get(sizeof(int32_t) * n);
     cl.l2 = (int32_t *)c->lists[2].get(sizeof(int32_t) * n);
-    int64_t *tmp = (int64_t *)c->scan_tmp.get(sizeof(int64_t) * scan_tmp_elems(3 * nb + 1));
-    launch_partition(cls, n, counts, tmp, cl.l0, cl.l1, cl.l2, s);
     int64_t *bounds = (int64_t *)c->bounds.get(sizeof(int64_t) * (2 * nmaps + 6));
-    launch_class_bounds(counts, nb, cl.l0, cl.l1, d_pbase, nmaps, bounds, s);
-    S2G_HIP(hipEventRecord(c->stage[1], s));
-    int64_t *h = (int64_t *)c->h_bounds.get(sizeof(int64_t) * (nmaps + 5));
-    S2G_HIP(hipMemcpyAsync(h, bounds, sizeof(int64_t) * (nmaps + 5), hipMemcpyDeviceToHost, s));
+    if (nb <= kPartLight) {
+        launch_partition_light(cls, n, counts, d_pbase, nmaps, cl.l0, cl.l1, cl.l2, bounds, s);
+    } else {
+        int64_t *tmp = (int64_t *)c->scan_tmp.get(sizeof(int64_t) * scan_tmp_elems(3 * nb + 1));
+        launch_partition(cls, n, counts, tmp, cl.l0, cl.l1, cl.l2, s);
+        launch_class_bounds(counts, nb, cl.l0, cl.l1, d_pbase, nmaps, bounds, s);
+    }
+    if (timed)
+        S2G_HIP(hipEventRecord(c->stage[1], s));
+    int64_t *h = (int64_t *)c->h_bounds.get(sizeof(int64_t) * (2 * nmaps + 6));
+    S2G_HIP(hipMemcpyAsync(h, bounds, sizeof(int64_t) * (2 * nmaps + 6), hipMemcpyDeviceToHost,
+                           s));
     S2G_HIP(hipStreamSynchronize(s));
     cl.ns = h[1] - h[0];
     cl.nl = h[2] - h[1];
     cl.ne = h[3] - h[2];
     cl.lbase.assign(h + 4, h + 5 + nmaps);
     cl.d_lbase = bounds + 4;
+    cl.sbase.assign(h + 5 + nmaps, h + 6 + 2 * nmaps);
+    cl.d_sbase = bounds + 5 + nmaps;
     return cl;
 }
 
@@ -331,7 +507,7 @@ struct PassTables {
     const Map2D *d_maps = nullptr;
     const int64_t *d_pbase = nullptr;
     const TileMap *d_stm = nullptr;
-    std::vector<TileMap> tm;
+    std::vector<TileMap> tm, stm;
     int64_t ntot = 0;
     int ntiles = 0, nstiles = 0;
     bool any_out = false;
@@ -383,6 +559,7 @@ PassTables pass_tables(s2g_ctx *c, const MapIn *mi, int nmaps, hipStream_t s)
             throw Error(S2G_EUNSUPPORTED, "deposit pass too large (2^31 particles or tiles)");
     }
     pb[nmaps] = ntot;
+    pt.stm.assign(stm, stm + nmaps);
     char *d = (char *)c->tab.get(btab + bpb + bst);
     pt.d_maps = (const Map2D *)d;
     pt.d_pbase = (const int64_t *)(d + btab);
@@ -426,7 +603,12 @@ void deposit2d_pass(s2g_ctx *c, const MapIn *mi, int nmaps, hipStream_t s, s2g_s
         std::memset(st, 0, sizeof(*st));
     }
     hipEvent_t *E = c->stage;
-    S2G_HIP(hipEventRecord(E[0], s));
+    // stage events only for a caller that asks for the times
+    auto mark = [&](int e, hipStream_t q) {
+        if (st)
+            S2G_HIP(hipEventRecord(E[e], q));
+    };
+    mark(0, s);
     PassTables pt = pass_tables(c, mi, nmaps, s);
     const Map2D *d_maps = pt.d_maps;
     const int64_t *d_pbase = pt.d_pbase;
@@ -443,12 +625,25 @@ void deposit2d_pass(s2g_ctx *c, const MapIn *mi, int nmaps, hipStream_t s, s2g_s
     if (ntot > 0) {
         rec = (Rec2 *)c->rec.get(sizeof(Rec2) * ntot);
         int32_t *cls = (int32_t *)c->cls.get(sizeof(int32_t) * ntot);
-        launch_2d_setup(dtype, d_maps, nmaps, ntot, nq, kernel, rec, cls, s);
-        cl = partition_classes(c, cls, ntot, d_pbase, nmaps, s);
+        int64_t *counts = class_counts(c, ntot);
+        launch_2d_setup(dtype, d_maps, nmaps, ntot, nq, kernel, rec, cls, counts, s);
+        cl = partition_classes(c, cls, ntot, counts, d_pbase, nmaps, s, st != nullptr);
         fill_class_stats(st, ntot, cl);
     } else {
-        S2G_HIP(hipEventRecord(E[1], s));
+        mark(1, s);
     }
+
+    const int gstep = c->tune.gather_planes;
+    // three or four FP64 planes run two blocks per CU: items of twice the
+    // least size halve their partials for little balance (777^2, four planes:
+    // gather 229 -> 243 us, finalize 111 -> 42 us)
+    const int np0 = nplanes < gstep ? nplanes : gstep;
+    const int64_t gmin = c->tune.gather_item_min * (np0 > 2 && !fp32acc ? 2 : 1);
+    LightTables lt;
+    if (ntot > 0 && partition_blocks(ntot) <= kPartLight)
+        lt = light_lists(c, tm, cl.lbase, pt.stm, cl.sbase, ntiles, gmin,
+                         c->tune.gather_items_per_cu,
+                         (int64_t)sizeof(double) * np0 * kGT * kGT, s);
 
     // Side stream: the explicit normalisation, then the small-footprint
     // scatter, beside the pair lists and the gather on s.  The gather waits
@@ -457,65 +652,82 @@ void deposit2d_pass(s2g_ctx *c, const MapIn *mi, int nmaps, hipStream_t s, s2g_s
     // waits for it and adds the large particles' sums (2^24 cluster set on
     // 4096^2: the 5.7 ms normalisation runs beside the 5.7 ms pair lists and
     // the 6.4 ms small scatter beside the gather; 288 -> 284 ms per step).
-    hipStream_t s2 = c->side;
+    // A light pass leaves CUs idle in every stage: there the small scatter
+    // has a stream of its own.
+    hipStream_t s2 = c->side, s3 = lt.ok ? c->side2 : s2;
     S2G_HIP(hipEventRecord(c->fork, s));
     S2G_HIP(hipStreamWaitEvent(s2, c->fork, 0));
-    S2G_HIP(hipEventRecord(E[2], s2));
+    if (s3 != s2)
+        S2G_HIP(hipStreamWaitEvent(s3, c->fork, 0));
+    mark(2, s2);
     launch_2d_norm(kernel, cl.l2, cl.ne, d_maps, rec, s2);
-    S2G_HIP(hipEventRecord(E[3], s2));
+    mark(3, s2);
     S2G_HIP(hipEventRecord(c->normed, s2));
     const int eS = s2g_ctx::kNumStageEvents - 3;
-    S2G_HIP(hipEventRecord(E[eS], s2));
+    mark(eS, s3);
     const bool add = cl.ns > 0;  // finalize adds to the small scatter's image
     if (add) {
         for (int m = 0; m < nmaps; ++m) {
             const int64_t nd = mi[m].a.npix * mi[m].a.npix;
-            S2G_HIP(hipMemsetAsync(mi[m].image, 0, sizeof(double) * nplanes * nd, s2));
+            S2G_HIP(hipMemsetAsync(mi[m].image, 0, sizeof(double) * nplanes * nd, s3));
         }
         const int64_t ns = cl.ns;
-        int64_t *soff = nullptr;
-        const int32_t *sorted = bucket_small(c, cl, rec, d_maps, nstiles, &soff, s2);
         // work items of <= Gs particles; the item count stays on the device and
         // the grid is its upper bound nstiles + ns / Gs
         const int64_t starget = (int64_t)c->ncu * c->tune.small_items_per_cu;
         int64_t Gs = (ns + starget - 1) / starget;
-        if (Gs < c->tune.small_item_min)
-            Gs = c->tune.small_item_min;
+        // a light pass halves the least item, to spread over the CUs (65,536
+        // particles on 256^2: scatter 97 -> 70 us; quartered 78 us, the
+        // windows' own cost)
+        const int64_t smin = lt.ok ? (c->tune.small_item_min + 1) / 2 : c->tune.small_item_min;
+        if (Gs < smin)
+            Gs = smin;
         const int64_t max_items = nstiles + (ns + Gs - 1) / Gs;
         if (max_items > ((int64_t)1 << 31) / 1024)  // blocks x threads (up to 1024)
             throw Error(S2G_EUNSUPPORTED, "too many small-footprint work items");
-        int64_t *snit = (int64_t *)c->snitems.get(sizeof(int64_t) * (nstiles + 1));
-        int4 *sitems = (int4 *)c->sitems.get(sizeof(int4) * max_items);
-        int64_t *stile = (int64_t *)c->stile.get(sizeof(int64_t) * 2 * nstiles);
-        int64_t *tmp =
-            (int64_t *)c->sscan_tmp.get(sizeof(int64_t) * scan_tmp_elems(nstiles + 1));
-        launch_items(soff, d_stm, nmaps, nstiles, Gs, 1, nullptr, snit, tmp, nullptr, nullptr,
-                     false, s2);
-        launch_items(soff, d_stm, nmaps, nstiles, Gs, 1, nullptr, snit, tmp, sitems, stile,
-                     true, s2);
+        SmallItems si;
+        if (lt.ok) {
+            si = light_small_lists<Rec2>(c, cl.l0, ns, rec, lt, nmaps, cl.d_sbase, nstiles, Gs,
+                                         max_items, s3);
+        } else {
+            int64_t *soff = nullptr;
+            si.plist = bucket_small(c, cl, rec, d_maps, nstiles, &soff, s3);
+            int64_t *snit = (int64_t *)c->snitems.get(sizeof(int64_t) * (nstiles + 1));
+            int4 *sitems = (int4 *)c->sitems.get(sizeof(int4) * max_items);
+            int64_t *stile = (int64_t *)c->stile.get(sizeof(int64_t) * 2 * nstiles);
+            int64_t *tmp =
+                (int64_t *)c->sscan_tmp.get(sizeof(int64_t) * scan_tmp_elems(nstiles + 1));
+            launch_items(soff, d_stm, nmaps, nstiles, Gs, 1, nullptr, snit, tmp, nullptr, nullptr,
+                         false, s3);
+            launch_items(soff, d_stm, nmaps, nstiles, Gs, 1, nullptr, snit, tmp, sitems, stile,
+                         true, s3);
+            si.items = sitems;
+            si.d_nitems = snit + nstiles;
+        }
         const int sstep = c->tune.small_planes;
         for (int plane0 = 0; plane0 < nplanes; plane0 += sstep) {
             const int np = nplanes - plane0 < sstep ? nplanes - plane0 : sstep;
-            launch_2d_small_tile(dtype, kernel, np, sitems, snit + nstiles, max_items, sorted,
-                                 rec, d_maps, nq, plane0, s2);
+            launch_2d_small_tile(dtype, kernel, np, si.items, si.d_nitems, max_items, si.plist,
+                                 rec, d_maps, nq, plane0, s3);
         }
     }
-    S2G_HIP(hipEventRecord(E[eS + 1], s2));
-    S2G_HIP(hipEventRecord(c->smalled, s2));
+    mark(eS + 1, s3);
+    S2G_HIP(hipEventRecord(c->smalled, s3));
 
-    double ms_sort = 0.0, ms_gather = 0.0, ms_fin = 0.0;
     int64_t launches = 0;
     TilePlan tp;
     if (cl.nl > 0) {
-        tp = build_tile_lists(c, cl.l1, rec, false, tm, cl.lbase, cl.d_lbase, ntiles, s,
-                              &ms_sort, c->tune.gather_item_min, c->tune.gather_items_per_cu,
-                              c->tune.gather_item_max);
-        if (st)
-            st->n_pairs = tp.npairs;
+        if (lt.ok)
+            tp = light_tile_lists<Rec2>(c, cl.l1, rec, lt, nmaps, cl.d_lbase, ntiles, s,
+                                        st != nullptr, gmin, c->tune.gather_items_per_cu,
+                                        c->tune.gather_item_max);
+        else
+            tp = build_tile_lists(c, cl.l1, rec, false, tm, cl.lbase, cl.d_lbase, ntiles, s,
+                                  st != nullptr, gmin, c->tune.gather_items_per_cu,
+                                  c->tune.gather_item_max);
     }
     S2G_HIP(hipStreamWaitEvent(s, c->normed, 0));
     int ev = 10;
-    const int gstep = c->tune.gather_planes;
     for (int plane0 = 0; plane0 < nplanes; plane0 += gstep) {
         const int np = nplanes - plane0 < gstep ? nplanes - plane0 : gstep;
         GatherArgs g;
@@ -528,18 +740,20 @@ void deposit2d_pass(s2g_ctx *c, const MapIn *mi, int nmaps, hipStream_t s, s2g_s
         g.nmaps = nmaps;
         g.ntiles = ntiles;
         g.nitems = tp.nitems;
+        g.d_nitems = tp.d_nitems;
         g.items = tp.items;
         g.pairs = tp.pairs;
         g.rec = rec;
         g.maps = d_maps;
-        g.partial = tp.nitems > 0 ? (double *)c->partial.get(sizeof(double) * tp.nitems * np *
-                                                             kGT * kGT)
-                                  : nullptr;
+        const size_t bpart = sizeof(double) * tp.nitems * np * kGT * kGT;
+        g.partial = tp.nitems == 0 ? nullptr
+                    : lt.ok        ? (double *)c->partial.get_roomy(bpart)
+                                   : (double *)c->partial.get(bpart);
         g.tile_items = tp.tile_items;
         g.add = add;
         // events per plane group: gather start / end, finalize start (after
         // the join with the side stream) / end
-        const bool timed = ev + 3 < s2g_ctx::kNumStageEvents - 3;
+        const bool timed = st && ev + 3 < s2g_ctx::kNumStageEvents - 3;
         if (timed)
             S2G_HIP(hipEventRecord(E[ev], s));
         if (tp.nitems > 0) {
@@ -562,17 +776,22 @@ void deposit2d_pass(s2g_ctx *c, const MapIn *mi, int nmaps, hipStream_t s, s2g_s
     if (any_out)
         launch_2d_reduce_maps(d_maps, nmaps, ntiles, nq, s);
     S2G_HIP(hipGetLastError());
-    S2G_HIP(hipEventRecord(E[eS + 2], s));
-    S2G_HIP(hipEventSynchronize(E[eS + 2]));
+    mark(eS + 2, s);
+    if (st && tp.d_npairs)
+        S2G_HIP(hipMemcpyAsync(c->h_small, tp.d_npairs, sizeof(int64_t), hipMemcpyDeviceToHost,
+                               s));
+    S2G_HIP(hipStreamSynchronize(s));
     if (st) {
+        double ms_gather = 0.0, ms_fin = 0.0;
         for (int k = 10; k < ev; k += 4) {
             ms_gather += elapsed(E[k], E[k + 1]);
             ms_fin += elapsed(E[k + 2], E[k + 3]);
         }
+        st->n_pairs = tp.d_npairs ? c->h_small[0] : tp.npairs;
         st->ms_device = elapsed(E[0], E[eS + 2]);
         st->ms_setup = elapsed(E[0], E[1]);
         st->ms_norm = elapsed(E[2], E[3]);
-        st->ms_sort = ms_sort;
+        st->ms_sort = cl.nl > 0 ? elapsed(E[4], E[5]) + elapsed(E[6], E[7]) : 0.0;
         st->ms_gather = ms_gather;
         st->ms_finalize = ms_fin;
         st->ms_small = elapsed(E[eS], E[eS + 1]);
@@ -614,11 +833,15 @@ void deposit3d_device(s2g_ctx *c, const Map3DArgs &a, double *d_image, hipStream
         st->n_particles = n;
     }
     hipEvent_t *E = c->stage;
-    S2G_HIP(hipEventRecord(E[0], s));
+    // stage events only for a caller that asks for the times
+    auto mark = [&](int e, hipStream_t q) {
+        if (st)
+            S2G_HIP(hipEventRecord(E[e], q));
+    };
+    mark(0, s);
     if (n == 0) {
         S2G_HIP(hipMemsetAsync(d_image, 0, sizeof(double) * nd * 2, s));
-        S2G_HIP(hipEventRecord(E[1], s));
-        S2G_HIP(hipEventSynchronize(E[1]));
+        S2G_HIP(hipStreamSynchronize(s));
         return;
     }
     Rec3 *rec = (Rec3 *)c->rec.get(sizeof(Rec3) * n);
@@ -626,35 +849,47 @@ void deposit3d_device(s2g_ctx *c, const Map3DArgs &a, double *d_image, hipStream
     // pass table: the particle range and the grid of the small-footprint tiles
     const int64_t nst = (npix + kST3 - 1) / kST3;
     const int64_t nstiles = nst * nst * nst;
+    const TileMap stm{0, 0, (int32_t)(nstiles < INT32_MAX ? nstiles : 0), (int32_t)nst,
+                      (int32_t)nst, 1, 0};
     const size_t btab = 2 * sizeof(int64_t) + sizeof(TileMap);
     char *htab = (char *)c->h_tab.get(btab);
     int64_t *hpb = (int64_t *)htab;
     hpb[0] = 0;
     hpb[1] = n;
-    *(TileMap *)(htab + 2 * sizeof(int64_t)) =
-        TileMap{0, 0, (int32_t)(nstiles < INT32_MAX ? nstiles : 0), (int32_t)nst, (int32_t)nst,
-                1, 0};
+    *(TileMap *)(htab + 2 * sizeof(int64_t)) = stm;
     int64_t *d_pbase = (int64_t *)c->tab.get(btab);
     const TileMap *d_stm = (const TileMap *)(d_pbase + 2);
     S2G_HIP(hipMemcpyAsync(d_pbase, htab, btab, hipMemcpyHostToDevice, s));
-    launch_3d_setup(a, rec, cls, s);
-    const ClassLists cl = partition_classes(c, cls, n, d_pbase, 1, s);
+    int64_t *counts = class_counts(c, n);
+    launch_3d_setup(a, rec, cls, counts, s);
+    const ClassLists cl = partition_classes(c, cls, n, counts, d_pbase, 1, s, st != nullptr);
     fill_class_stats(st, n, cl);
 
-    // Side stream, as in the 2D pass: the explicit normalisation, then the
+    const int nb = (int)((npix + kBT - 1) / kBT);
+    const int ntiles = nb * nb * nb;
+    const std::vector<TileMap> tm0{TileMap{0, 0, ntiles, nb, nb, 0, 0}};
+    const bool windowed = small3_windowed(cl.ns, nstiles);
+    LightTables lt;
+    if (partition_blocks(n) <= kPartLight && nstiles <= kMaxTiles)
+        lt = light_lists(c, tm0, cl.lbase, {stm}, cl.sbase, ntiles, 64, 16,
+                         (int64_t)sizeof(double) * 2 * kBT * kBT * kBT, s);
+
+    // Side streams, as in the 2D pass: the explicit normalisation and the
     // small-footprint scatter into the zeroed image, beside the pair lists
     // and the gather; the gather waits for the normalisation and the
     // finalize for the scatter, to whose sums it adds.
-    hipStream_t s2 = c->side;
+    hipStream_t s2 = c->side, s3 = lt.ok ? c->side2 : s2;
     S2G_HIP(hipEventRecord(c->fork, s));
     S2G_HIP(hipStreamWaitEvent(s2, c->fork, 0));
-    S2G_HIP(hipEventRecord(E[2], s2));
+    if (s3 != s2)
+        S2G_HIP(hipStreamWaitEvent(s3, c->fork, 0));
+    mark(2, s2);
     launch_3d_norm(a.kernel, cl.l2, cl.ne, a.npix, a.flags, rec, s2);
-    S2G_HIP(hipEventRecord(E[3], s2));
+    mark(3, s2);
     S2G_HIP(hipEventRecord(c->normed, s2));
     const int eS = s2g_ctx::kNumStageEvents - 3;
-    S2G_HIP(hipMemsetAsync(d_image, 0, sizeof(double) * nd * 2, s2));
-    S2G_HIP(hipEventRecord(E[eS], s2));
+    S2G_HIP(hipMemsetAsync(d_image, 0, sizeof(double) * nd * 2, s3));
+    mark(eS, s3);
     Small3Args sa;
     sa.dtype = a.dtype;
     sa.kernel = a.kernel;
@@ -664,50 +899,59 @@ void deposit3d_device(s2g_ctx *c, const Map3DArgs &a, double *d_image, hipStream
     sa.rec = rec;
     sa.binq = a.binq;
     sa.image = d_image;
-    if (small3_windowed(cl.ns, nstiles)) {
+    if (windowed) {
         const int64_t ns = cl.ns;
         const int nt3 = (int)nst, ntl = (int)nstiles;
-        uint32_t *keys = (uint32_t *)c->skeys.get(sizeof(uint32_t) * 2 * ns);
-        int32_t *vals = (int32_t *)c->svals.get(sizeof(int32_t) * 2 * ns);
-        launch_3d_small_keys(cl.l0, ns, rec, nt3, keys, vals, s2);
-        int end_bit = 1;
-        while (end_bit < 32 && ((int64_t)1 << end_bit) < nstiles)
-            ++end_bit;
-        const size_t tb = sort_pairs_tmp_bytes(ns, end_bit);
-        void *stmp = c->sort_tmp.get(tb ? tb : 1);
-        sort_pairs(stmp, tb, keys, keys + ns, vals, vals + ns, ns, end_bit, s2);
-        int64_t *soff = (int64_t *)c->soff.get(sizeof(int64_t) * (nstiles + 1));
-        launch_tile_offsets(keys + ns, ns, ntl, soff, s2);
         const int64_t Gs = kSmall3Item;
         const int64_t max_items = nstiles + ns / Gs;
-        int64_t *snit = (int64_t *)c->snitems.get(sizeof(int64_t) * (nstiles + 1));
-        int4 *sitems = (int4 *)c->sitems.get(sizeof(int4) * max_items);
-        int64_t *stile = (int64_t *)c->stile.get(sizeof(int64_t) * 2 * nstiles);
-        int64_t *tmp =
-            (int64_t *)c->sscan_tmp.get(sizeof(int64_t) * scan_tmp_elems(nstiles + 1));
-        launch_items(soff, d_stm, 1, ntl, Gs, 1, nullptr, snit, tmp, nullptr, nullptr, false, s2);
-        launch_items(soff, d_stm, 1, ntl, Gs, 1, nullptr, snit, tmp, sitems, stile, true, s2);
-        launch_3d_small_window(sa, sitems, snit + nstiles, max_items, vals + ns, nt3, s2);
+        SmallItems si;
+        if (lt.ok) {
+            si = light_small_lists<Rec3>(c, cl.l0, ns, rec, lt, 1, cl.d_sbase, ntl, Gs, max_items,
+                                         s3);
+        } else {
+            uint32_t *keys = (uint32_t *)c->skeys.get(sizeof(uint32_t) * 2 * ns);
+            int32_t *vals = (int32_t *)c->svals.get(sizeof(int32_t) * 2 * ns);
+            launch_3d_small_keys(cl.l0, ns, rec, nt3, keys, vals, s3);
+            int end_bit = 1;
+            while (end_bit < 32 && ((int64_t)1 << end_bit) < nstiles)
+                ++end_bit;
+            const size_t tb = sort_pairs_tmp_bytes(ns, end_bit);
+            void *stmp = c->sort_tmp.get(tb ? tb : 1);
+            sort_pairs(stmp, tb, keys, keys + ns, vals, vals + ns, ns, end_bit, s3);
+            int64_t *soff = (int64_t *)c->soff.get(sizeof(int64_t) * (nstiles + 1));
+            launch_tile_offsets(keys + ns, ns, ntl, soff, s3);
+            int64_t *snit = (int64_t *)c->snitems.get(sizeof(int64_t) * (nstiles + 1));
+            int4 *sitems = (int4 *)c->sitems.get(sizeof(int4) * max_items);
+            int64_t *stile = (int64_t *)c->stile.get(sizeof(int64_t) * 2 * nstiles);
+            int64_t *tmp =
+                (int64_t *)c->sscan_tmp.get(sizeof(int64_t) * scan_tmp_elems(nstiles + 1));
+            launch_items(soff, d_stm, 1, ntl, Gs, 1, nullptr, snit, tmp, nullptr, nullptr, false,
+                         s3);
+            launch_items(soff, d_stm, 1, ntl, Gs, 1, nullptr, snit, tmp, sitems, stile, true, s3);
+            si = SmallItems{vals + ns, sitems, snit + nstiles};
+        }
+        launch_3d_small_window(sa, si.items, si.d_nitems, max_items, si.plist, nt3, s3);
     } else {
-        launch_3d_small(sa, s2);
+        launch_3d_small(sa, s3);
     }
-    S2G_HIP(hipEventRecord(E[eS + 1], s2));
-    S2G_HIP(hipEventRecord(c->smalled, s2));
+    mark(eS + 1, s3);
+    S2G_HIP(hipEventRecord(c->smalled, s3));
 
-    const int nb = (int)((npix + kBT - 1) / kBT);
-    const int ntiles = nb * nb * nb;
-    double ms_sort = 0.0, ms_gather = 0.0, ms_fin = 0.0;
     int64_t launches = 0;
+    TilePlan tp;
     if (cl.nl > 0) {
-        std::vector<TileMap> tm{TileMap{0, 0, ntiles, nb, nb, 0, 0}};
         // brick items of at most 4096 pairs (2^24 cluster set on 256^3: 16
         // items per CU of about 20k pairs, gather 69.0 ms; capped at 1024 /
         // 4096 / 8192 pairs: 60.2 / 60.9 / 63.9 ms, 1024 with a longer
         // finalize)
-        const TilePlan tp = build_tile_lists(c, cl.l1, rec, true, tm, cl.lbase, cl.d_lbase,
-                                             ntiles, s, &ms_sort, 64, 16, 4096);
-        if (st)
-            st->n_pairs = tp.npairs;
+        if (lt.ok) {
+            tp = light_tile_lists<Rec3>(c, cl.l1, rec, lt, 1, cl.d_lbase, ntiles, s,
+                                        st != nullptr, 64, 16, 4096);
+        } else {
+            std::vector<TileMap> tm = tm0;
+            tp = build_tile_lists(c, cl.l1, rec, true, tm, cl.lbase, cl.d_lbase, ntiles, s,
+                                  st != nullptr, 64, 16, 4096);
+        }
         Gather3Args g;
         g.dtype = a.dtype;
         g.kernel = a.kernel;
@@ -717,43 +961,47 @@ void deposit3d_device(s2g_ctx *c, const Map3DArgs &a, double *d_image, hipStream
         g.nb = nb;
         g.ntiles = ntiles;
         g.nitems = tp.nitems;
+        g.d_nitems = tp.d_nitems;
         g.npix = npix;
         g.items = tp.items;
         g.pairs = tp.pairs;
         g.rec = rec;
         g.binq = a.binq;
-        g.partial = (double *)c->partial.get(sizeof(double) * (tp.nitems ? tp.nitems : 1) * 2 *
-                                             kBT * kBT * kBT);
+        const size_t bpart = sizeof(double) * (tp.nitems ? tp.nitems : 1) * 2 * kBT * kBT * kBT;
+        g.partial = (double *)(lt.ok ? c->partial.get_roomy(bpart) : c->partial.get(bpart));
         g.tile_items = tp.tile_items;
         g.image = d_image;
         g.add = 1;
         S2G_HIP(hipStreamWaitEvent(s, c->normed, 0));
-        S2G_HIP(hipEventRecord(E[10], s));
+        mark(10, s);
         if (tp.nitems > 0) {
             launch_3d_gather(g, s);
             ++launches;
         }
-        S2G_HIP(hipEventRecord(E[11], s));
+        mark(11, s);
         S2G_HIP(hipStreamWaitEvent(s, c->smalled, 0));
-        S2G_HIP(hipEventRecord(E[12], s));
+        mark(12, s);
         launch_3d_finalize(g, s);
-        S2G_HIP(hipEventRecord(E[13], s));
+        mark(13, s);
     }
+    S2G_HIP(hipStreamWaitEvent(s, c->normed, 0));
     S2G_HIP(hipStreamWaitEvent(s, c->smalled, 0));
     S2G_HIP(hipGetLastError());
-    S2G_HIP(hipEventRecord(E[eS + 2], s));
-    S2G_HIP(hipEventSynchronize(E[eS + 2]));
+    mark(eS + 2, s);
+    if (st && tp.d_npairs)
+        S2G_HIP(hipMemcpyAsync(c->h_small, tp.d_npairs, sizeof(int64_t), hipMemcpyDeviceToHost,
+                               s));
+    S2G_HIP(hipStreamSynchronize(s));
     if (st) {
         if (cl.nl > 0) {
-            ms_gather = elapsed(E[10], E[11]);
-            ms_fin = elapsed(E[12], E[13]);
+            st->ms_gather = elapsed(E[10], E[11]);
+            st->ms_finalize = elapsed(E[12], E[13]);
+            st->ms_sort = elapsed(E[4], E[5]) + elapsed(E[6], E[7]);
         }
+        st->n_pairs = tp.d_npairs ? c->h_small[0] : tp.npairs;
         st->ms_device = elapsed(E[0], E[eS + 2]);
         st->ms_setup = elapsed(E[0], E[1]);
         st->ms_norm = elapsed(E[2], E[3]);
-        st->ms_sort = ms_sort;
-        st->ms_gather = ms_gather;
-        st->ms_finalize = ms_fin;
         st->ms_small = elapsed(E[eS], E[eS + 1]);
         st->n_gather_launches = launches;
     }
@@ -780,8 +1028,13 @@ Map2DArgs make_args(int dtype, const void *pos, const void *hsml, const void *m,
     return a;
 }
 
-// copy host inputs into the context's staging buffers
-Map2DArgs stage_inputs(s2g_ctx *c, const Map2DArgs &h, hipStream_t s, s2g_stats *st)
+// Host arrays of up to this many bytes in all cross in one copy through pinned
+// staging: each copy from pageable memory costs the host some 10 us.
+constexpr size_t kStageBytes = (size_t)4 << 20;
+
+// copy host inputs into the context's staging buffers (enqueued on `s`
+// between the events ev0 and ev1; h2d_ms once the stream has passed them)
+Map2DArgs stage_inputs(s2g_ctx *c, const Map2DArgs &h, hipStream_t s)
 {
     const size_t es = elem_size(h.dtype);
     const int64_t n = h.n;
@@ -789,22 +1042,30 @@ Map2DArgs stage_inputs(s2g_ctx *c, const Map2DArgs &h, hipStream_t s, s2g_stats 
     const size_t cnt[6] = {(size_t)(3 * n), (size_t)n, (size_t)n, (size_t)n,
                            (size_t)(n * h.nq), (size_t)n};
     void *dst[6];
-    hipEvent_t e0 = c->ev0, e1 = c->ev1;
-    S2G_HIP(hipEventRecord(e0, s));
+    size_t off[7] = {};
     for (int k = 0; k < 6; ++k) {
         if (n > 0 && !src[k])
             throw Error(S2G_EINVAL, "input array pointer is NULL");
-        dst[k] = c->in[k].get(es * (cnt[k] ? cnt[k] : 1));
+        off[k + 1] = off[k] + ((es * (cnt[k] ? cnt[k] : 1) + 255) & ~size_t(255));
+    }
+    S2G_HIP(hipEventRecord(c->ev0, s));
+    if (off[6] <= kStageBytes) {
+        char *hp = (char *)c->h_stage.get(off[6]);
+        char *d = (char *)c->in[6].get_roomy(off[6]);
+        for (int k = 0; k < 6; ++k) {
+            std::memcpy(hp + off[k], src[k], es * cnt[k]);
+            dst[k] = d + off[k];
+        }
         if (n > 0)
+            S2G_HIP(hipMemcpyAsync(d, hp, off[6], hipMemcpyHostToDevice, s));
+    } else {
+        for (int k = 0; k < 6; ++k) {
+            dst[k] = c->in[k].get(off[k + 1] - off[k]);
             S2G_HIP(hipMemcpyAsync(dst[k], src[k], es * cnt[k], hipMemcpyHostToDevice, s));
+        }
+        S2G_HIP(hipStreamSynchronize(s));  // done with the caller's arrays
     }
-    S2G_HIP(hipEventRecord(e1, s));
-    S2G_HIP(hipEventSynchronize(e1));
-    if (st) {
-        float ms = 0.f;
-        S2G_HIP(hipEventElapsedTime(&ms, e0, e1));
-        st->ms_h2d = ms;
-    }
+    S2G_HIP(hipEventRecord(c->ev1, s));
     Map2DArgs d = h;
     d.pos = dst[0];
     d.hsml = dst[1];
@@ -815,17 +1076,23 @@ Map2DArgs stage_inputs(s2g_ctx *c, const Map2DArgs &h, hipStream_t s, s2g_stats 
     return d;
 }
 
+// time of the last stage_inputs (after a synchronisation of its stream)
+double h2d_ms(s2g_ctx *c) { return elapsed(c->ev0, c->ev1); }
+
 void d2h(s2g_ctx *c, void *dst, const void *src, size_t bytes, hipStream_t s, double *ms)
 {
-    S2G_HIP(hipEventRecord(c->ev0, s));
-    S2G_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
-    S2G_HIP(hipEventRecord(c->ev1, s));
-    S2G_HIP(hipEventSynchronize(c->ev1));
-    if (ms) {
-        float t = 0.f;
-        S2G_HIP(hipEventElapsedTime(&t, c->ev0, c->ev1));
-        *ms = t;
-    }
+    const bool stage = bytes <= kStageBytes;
+    void *to = stage ? c->h_stage.get(bytes) : dst;
+    if (ms)
+        S2G_HIP(hipEventRecord(c->ev0, s));
+    S2G_HIP(hipMemcpyAsync(to, src, bytes, hipMemcpyDeviceToHost, s));
+    if (ms)
+        S2G_HIP(hipEventRecord(c->ev1, s));
+    S2G_HIP(hipStreamSynchronize(s));
+    if (stage)
+        std::memcpy(dst, to, bytes);
+    if (ms)
+        *ms = elapsed(c->ev0, c->ev1);
 }
 
 void check_dims_nq(int dims, int nq)
@@ -1128,10 +1395,16 @@ void plan_enqueue(s2g_plan *pl, PlanPass &pp, hipStream_t s, hipStream_t s2)
     int32_t *cls = (int32_t *)pp.cls.p, *l0 = (int32_t *)pp.l0.p, *l1 = (int32_t *)pp.l1.p,
             *l2 = (int32_t *)pp.l2.p;
     int64_t *tmp = (int64_t *)pp.scan_tmp.p, *bounds = (int64_t *)pp.bounds.p;
-    launch_2d_setup(pp.dtype, pp.d_maps, pp.nmaps, pp.ntot, pp.nq, pp.kernel, rec, cls, s);
-    launch_partition(cls, pp.ntot, (int64_t *)pp.counts.p, tmp, l0, l1, l2, s);
-    launch_class_bounds((const int64_t *)pp.counts.p, pp.nb, l0, l1, pp.d_pbase, pp.nmaps, bounds,
-                        s);
+    launch_2d_setup(pp.dtype, pp.d_maps, pp.nmaps, pp.ntot, pp.nq, pp.kernel, rec, cls,
+                    (int64_t *)pp.counts.p, s);
+    if (pp.nb <= kPartLight) {
+        launch_partition_light(cls, pp.ntot, (const int64_t *)pp.counts.p, pp.d_pbase, pp.nmaps,
+                               l0, l1, l2, bounds, s);
+    } else {
+        launch_partition(cls, pp.ntot, (int64_t *)pp.counts.p, tmp, l0, l1, l2, s);
+        launch_class_bounds((const int64_t *)pp.counts.p, pp.nb, l0, l1, pp.d_pbase, pp.nmaps,
+                            bounds, s);
+    }
     S2G_HIP(hipEventRecord(pl->fork, s));
     S2G_HIP(hipStreamWaitEvent(s2, pl->fork, 0));
 
@@ -1154,14 +1427,21 @@ void plan_enqueue(s2g_plan *pl, PlanPass &pp, hipStream_t s, hipStream_t s2)
     // per-tile lists over device-side chunk ranges of each map's small list
     // (bounds[5 + nmaps + m]), then items (bounds[1] = the small count)
     const int64_t *sbase = bounds + 5 + pp.nmaps;
-    launch_anchor_lists(l0, rec, pp.d_sch, pp.nschunks, pp.d_stm, pp.smax_tiles, scnt, pp.sncnt,
-                        stmp, nullptr, false, sbase, s2);
-    launch_anchor_lists(l0, rec, pp.d_sch, pp.nschunks, pp.d_stm, pp.smax_tiles, scnt, pp.sncnt,
-                        stmp, (int32_t *)pp.sorted.p, true, sbase, s2);
-    launch_items(scnt, pp.d_stm, pp.nmaps, pp.nstiles, pp.smin, pp.starget, bounds + 1, snit,
-                 stmp, nullptr, nullptr, false, s2);
-    launch_items(scnt, pp.d_stm, pp.nmaps, pp.nstiles, pp.smin, pp.starget, bounds + 1, snit,
-                 stmp, (int4 *)pp.sitems.p, (int64_t *)pp.stile.p, true, s2);
+    const bool slight = pp.sncnt <= kListsLight;
+    launch_anchor_lists<Rec2>(l0, rec, pp.d_sch, pp.nschunks, pp.d_stm, pp.smax_tiles, scnt,
+                              pp.sncnt, stmp, nullptr, false, sbase, s2, !slight);
+    if (slight) {
+        launch_lists_light(scnt, pp.sncnt, pp.d_stm, pp.nmaps, pp.nstiles, pp.smin, pp.starget, 0,
+                           0, bounds + 1, snit, (int4 *)pp.sitems.p, pp.sitem_cap,
+                           (int64_t *)pp.stile.p, s2);
+    } else {
+        launch_items(scnt, pp.d_stm, pp.nmaps, pp.nstiles, pp.smin, pp.starget, bounds + 1, snit,
+                     stmp, nullptr, nullptr, false, s2);
+        launch_items(scnt, pp.d_stm, pp.nmaps, pp.nstiles, pp.smin, pp.starget, bounds + 1, snit,
+                     stmp, (int4 *)pp.sitems.p, (int64_t *)pp.stile.p, true, s2);
+    }
+    launch_anchor_lists<Rec2>(l0, rec, pp.d_sch, pp.nschunks, pp.d_stm, pp.smax_tiles, scnt,
+                              pp.sncnt, stmp, (int32_t *)pp.sorted.p, true, sbase, s2);
     for (int plane0 = 0; plane0 < pp.nplanes; plane0 += pp.sstep) {
         const int np = pp.nplanes - plane0 < pp.sstep ? pp.nplanes - plane0 : pp.sstep;
         launch_2d_small_tile(pp.dtype, pp.kernel, np, (const int4 *)pp.sitems.p, snit + pp.nstiles,
@@ -1173,16 +1453,26 @@ void plan_enqueue(s2g_plan *pl, PlanPass &pp, hipStream_t s, hipStream_t s2)
     // large particles: pair lists over device-side chunk ranges
     int64_t *cnt = (int64_t *)pp.cnt.p, *nit = (int64_t *)pp.nitems.p;
     const int64_t *lbase = bounds + 4, *d_npairs = cnt + pp.ncnt - 1;
+    // (the pair totals of a light plan stay below 2^31: its pair capacity does,
+    // and no list is longer than the particles times the tiles)
+    const bool light = pp.ncnt <= kListsLight &&
+                       pp.ntot * (int64_t)pp.max_tiles < (int64_t)INT32_MAX;
     launch_pairs<Rec2>(l1, rec, pp.d_ch, pp.nchunks, pp.d_tm, pp.max_tiles, cnt, pp.ncnt, tmp,
-                       nullptr, false, s, lbase);
-    launch_items(cnt, pp.d_tm, pp.nmaps, pp.ntiles, pp.gmin, pp.gtarget, d_npairs, nit, tmp,
-                 nullptr, nullptr, false, s, pp.gmax, pp.item_cap - pp.ntiles - 1);
+                       nullptr, false, s, lbase, INT64_MAX, !light);
+    if (light)
+        launch_lists_light(cnt, pp.ncnt, pp.d_tm, pp.nmaps, pp.ntiles, pp.gmin, pp.gtarget,
+                           pp.gmax, pp.item_cap - pp.ntiles - 1, d_npairs, nit,
+                           (int4 *)pp.items.p, pp.item_cap, (int64_t *)pp.tile_items.p, s);
+    else
+        launch_items(cnt, pp.d_tm, pp.nmaps, pp.ntiles, pp.gmin, pp.gtarget, d_npairs, nit, tmp,
+                     nullptr, nullptr, false, s, pp.gmax, pp.item_cap - pp.ntiles - 1);
     launch_plan_check(lbase, pp.nmaps, pp.d_tm, d_npairs, pp.pair_cap, (int *)pp.flag.p, s);
     launch_pairs<Rec2>(l1, rec, pp.d_ch, pp.nchunks, pp.d_tm, pp.max_tiles, cnt, pp.ncnt, tmp,
                        (int32_t *)pp.pairs.p, true, s, lbase, pp.pair_cap);
-    launch_items(cnt, pp.d_tm, pp.nmaps, pp.ntiles, pp.gmin, pp.gtarget, d_npairs, nit, tmp,
-                 (int4 *)pp.items.p, (int64_t *)pp.tile_items.p, true, s, pp.gmax,
-                 pp.item_cap - pp.ntiles - 1);
+    if (!light)
+        launch_items(cnt, pp.d_tm, pp.nmaps, pp.ntiles, pp.gmin, pp.gtarget, d_npairs, nit, tmp,
+                     (int4 *)pp.items.p, (int64_t *)pp.tile_items.p, true, s, pp.gmax,
+                     pp.item_cap - pp.ntiles - 1);
     S2G_HIP(hipStreamWaitEvent(s, pl->normed, 0));
     for (int plane0 = 0; plane0 < pp.nplanes; plane0 += pp.gstep) {
         const int np = pp.nplanes - plane0 < pp.gstep ? pp.nplanes - plane0 : pp.gstep;
@@ -1245,7 +1535,7 @@ void plan_pass_build(s2g_ctx *c, PlanPass &pp, double headroom, hipStream_t s)
     pp.flag.get(sizeof(int) * 2);
     // creation run of the class stages: the per-map large counts
     launch_2d_setup(pp.dtype, pp.d_maps, nmaps, pp.ntot, pp.nq, pp.kernel, (Rec2 *)pp.rec.p,
-                    (int32_t *)pp.cls.p, s);
+                    (int32_t *)pp.cls.p, (int64_t *)pp.counts.p, s);
     pp.scan_tmp.get(sizeof(int64_t) * scan_tmp_elems(3 * pp.nb + 1));
     launch_partition((const int32_t *)pp.cls.p, pp.ntot, (int64_t *)pp.counts.p,
                      (int64_t *)pp.scan_tmp.p, (int32_t *)pp.l0.p, (int32_t *)pp.l1.p,
@@ -1536,6 +1826,7 @@ int s2g_create(s2g_ctx **out, int device)
             c->ncu = prop.multiProcessorCount;
         if (hipStreamCreateWithFlags(&c->stream, hipStreamDefault) != hipSuccess ||
             hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking) != hipSuccess ||
+            hipStreamCreateWithFlags(&c->side2, hipStreamNonBlocking) != hipSuccess ||
             hipEventCreateWithFlags(&c->fork, hipEventDisableTiming) != hipSuccess ||
             hipEventCreateWithFlags(&c->normed, hipEventDisableTiming) != hipSuccess ||
             hipEventCreateWithFlags(&c->smalled, hipEventDisableTiming) != hipSuccess ||
@@ -1591,6 +1882,7 @@ void s2g_destroy(s2g_ctx *c)
     c->h_tab.release();
     c->h_bounds.release();
     c->h_tiles.release();
+    c->h_stage.release();
     c->hp_rec.release();
     c->hp_nunits.release();
     c->hp_units.release();
@@ -1617,6 +1909,8 @@ void s2g_destroy(s2g_ctx *c)
             (void)hipEventDestroy(e);
     if (c->side)
         (void)hipStreamDestroy(c->side);
+    if (c->side2)
+        (void)hipStreamDestroy(c->side2);
     if (c->stream)
         (void)hipStreamDestroy(c->stream);
     delete c;
@@ -1661,15 +1955,10 @@ int s2g_deposit(s2g_ctx *c, int dims, int dtype, const void *pos, const void *hs
         s2g_stats *st = stats ? stats : &local;
         Map2DArgs h = make_args(dtype, pos, hsml, m, rho, bin_q, nq, weights, n, params,
                                 kernel, flags);
-        double h2d_ms = 0.0;
-        {
-            s2g_stats tmp;
-            h = stage_inputs(c, h, s, &tmp);
-            h2d_ms = tmp.ms_h2d;
-        }
+        h = stage_inputs(c, h, s);
         double *img = (double *)c->image.get(sizeof(double) * nd * nplanes);
         deposit_device_any(c, dims, h, img, s, st);
-        st->ms_h2d = h2d_ms;
+        st->ms_h2d = h2d_ms(c);
         d2h(c, image_out, img, sizeof(double) * nd * nplanes, s, &st->ms_d2h);
         return S2G_OK;
     });
@@ -1735,15 +2024,10 @@ int s2g_map(s2g_ctx *c, int dims, int dtype, const void *pos, const void *hsml, 
         s2g_stats *st = stats ? stats : &local;
         Map2DArgs h = make_args(dtype, pos, hsml, m, rho, bin_q, nq, weights, n, params,
                                 kernel, flags);
-        double h2d_ms = 0.0;
-        {
-            s2g_stats tmp;
-            h = stage_inputs(c, h, s, &tmp);
-            h2d_ms = tmp.ms_h2d;
-        }
+        h = stage_inputs(c, h, s);
         double *img = (double *)c->image.get(sizeof(double) * nd * (nq + 1));
         deposit_device_any(c, dims, h, img, s, st);
-        st->ms_h2d = h2d_ms;
+        st->ms_h2d = h2d_ms(c);
         double *o = (double *)c->out.get(sizeof(double) * nd * nout);
         int rc = s2g_reduce_device(c, dims, npix, nq, flags, img, o, s);
         if (rc)
@@ -2307,10 +2591,7 @@ int s2g_footprints(s2g_ctx *c, int dims, int dtype, const void *pos, const void 
         const int64_t npix = params->npixels;
         Map2DArgs h = make_args(dtype, pos, hsml, m, rho, bin_q, nq, weights, n, params, kernel,
                                 flags);
-        {
-            s2g_stats tmp;
-            h = stage_inputs(c, h, s, &tmp);
-        }
+        h = stage_inputs(c, h, s);
         ClassLists cl;
         std::vector<TileMap> tm;
         int ntiles = 0, nstiles = 1;
@@ -2326,8 +2607,9 @@ int s2g_footprints(s2g_ctx *c, int dims, int dtype, const void *pos, const void 
             if (n > 0) {
                 Rec2 *r2 = (Rec2 *)c->rec.get(sizeof(Rec2) * n);
                 int32_t *cl2 = (int32_t *)c->cls.get(sizeof(int32_t) * n);
-                launch_2d_setup(dtype, pt.d_maps, 1, n, nq, kernel, r2, cl2, s);
-                cl = partition_classes(c, cl2, n, pt.d_pbase, 1, s);
+                int64_t *cc = class_counts(c, n);
+                launch_2d_setup(dtype, pt.d_maps, 1, n, nq, kernel, r2, cl2, cc, s);
+                cl = partition_classes(c, cl2, n, cc, pt.d_pbase, 1, s, false);
                 rec = r2;
                 if (cl.ns > 0)
                     sorted = bucket_small(c, cl, r2, pt.d_maps, nstiles, &soff, s);
@@ -2345,8 +2627,9 @@ int s2g_footprints(s2g_ctx *c, int dims, int dtype, const void *pos, const void 
                 int64_t *d_pbase = (int64_t *)c->tab.get(2 * sizeof(int64_t));
                 S2G_HIP(hipMemcpyAsync(d_pbase, hpb, 2 * sizeof(int64_t), hipMemcpyHostToDevice,
                                        s));
-                launch_3d_setup(h, r3, cl3, s);
-                cl = partition_classes(c, cl3, n, d_pbase, 1, s);
+                int64_t *cc = class_counts(c, n);
+                launch_3d_setup(h, r3, cl3, cc, s);
+                cl = partition_classes(c, cl3, n, cc, d_pbase, 1, s, false);
                 rec = r3;
                 sorted = cl.l0;  // the 3D small path keeps particle order
             }
@@ -2355,9 +2638,8 @@ int s2g_footprints(s2g_ctx *c, int dims, int dtype, const void *pos, const void 
         int64_t npairs = 0;
         std::vector<int64_t> cnt;
         if (cl.nl > 0) {
-            double ms = 0.0;
             const TilePlan tp = build_tile_lists(c, cl.l1, rec, dims == 3, tm, cl.lbase,
-                                                 cl.d_lbase, ntiles, s, &ms);
+                                                 cl.d_lbase, ntiles, s, false);
             npairs = tp.npairs;
             const int64_t ncnt = (int64_t)ntiles * tm[0].nch + 1;
             cnt.resize(ncnt);

@@ -34,6 +34,8 @@ constexpr int kGT = 64;
 
 // 3D: footprint box side <= 8 voxels goes to the scatter path; bricks of 16^3.
 constexpr int kSmallSide3D = 8;
+// side of the windowed 3D scatter's tiles
+constexpr int kST3 = 9;
 constexpr int kBT = 16;
 
 // Per-particle record of the 2D deposit, built once per call.
@@ -341,6 +343,9 @@ struct DevBuf {
         }
         return p;
     }
+    // the same, grown by a quarter more than asked for: sizes that vary a
+    // little from call to call would otherwise reallocate again and again
+    void *get_roomy(size_t need) { return need > bytes ? get(need + need / 4) : p; }
     void release()
     {
         if (p)

@@ -1,0 +1,67 @@
+"""Passes of at most 2^18 particles take the light stages (one-launch class
+partition and list scans, counts kept on the device); larger ones the general
+stages.  A particle of zero quantity deposits nothing without calc_mean, so a
+set and the same set with one such particle more, on either side of the line,
+must give the same image: sums of the same FP64 terms in another order, 1e-12
+of the largest pixel."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+LINE = 1 << 18
+
+
+def _set(n, npix, seed, hmax):
+    r = np.random.default_rng(seed)
+    x = r.uniform(-0.5, 0.5, (n, 3))
+    h = np.exp(r.uniform(np.log(0.3 / npix), np.log(hmax / npix), n))
+    m, rho, w, q = (r.uniform(0.5, 2.0, n) for _ in range(4))
+    return x, h, m, rho, q, w
+
+
+@pytest.mark.parametrize("dims,npix,hmax", [(2, 200, 40.0), (2, 65, 3.0), (3, 30, 7.0),
+                                            (3, 100, 1.5)])
+def test_light_and_general_passes_agree(s2g, dims, npix, hmax):
+    x, h, m, rho, q, w = _set(LINE + 1, npix, 5 + dims + npix, hmax)
+    q[-1] = 0.0
+    img, st = [], []
+    for n in (LINE, LINE + 1):
+        s = {}
+        img.append(s2g.deposit(x[:n], h[:n], m[:n], rho[:n], q[:n], w[:n], npix=npix,
+                               len2pix=float(npix), dimensions=dims, kernel=s2g.WendlandC4(dims),
+                               calc_mean=False, stats=s))
+        st.append(s)
+    for k in ("n_small", "n_large", "n_large_exact", "n_pairs"):
+        assert st[0][k] == st[1][k], k
+    assert st[1]["n_skipped"] == st[0]["n_skipped"] + 1
+    for k in range(2):
+        np.testing.assert_allclose(img[0][:, k], img[1][:, k], rtol=0,
+                                   atol=1e-12 * np.abs(img[1][:, k]).max())
+
+
+@pytest.mark.parametrize("nq", [1, 3])
+def test_light_batch_with_empty_and_one_sided_maps(s2g, nq):
+    """Maps without particles (first, in the middle, last), with only small or
+    only large footprints and with all of one's particles skipped share a light
+    pass: each map equals its own call."""
+    import torch
+    r = np.random.default_rng(nq)
+    maps, singles = [], []
+    for n, npix, lo, hi in [(0, 40, 1, 2), (700, 70, 0.4, 3.0), (0, 33, 1, 2),
+                            (300, 130, 20.0, 60.0), (255, 64, 0.4, 40.0), (257, 129, 1.0, 30.0),
+                            (40, 20, 1.0, 3.0), (0, 64, 1, 2)]:
+        x = r.uniform(-0.5, 0.5, (n, 3))
+        h = np.exp(r.uniform(np.log(lo / npix), np.log(hi / npix), n))
+        m, rho, w = (r.uniform(0.5, 2.0, n) for _ in range(3))
+        q = r.uniform(0.5, 2.0, (n, nq)) * (n != 40)
+        t = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (x, h, m, rho, q, w)]
+        out = torch.empty((nq + 1) * npix * npix, dtype=torch.float64, device="cuda")
+        maps.append(dict(pos=t[0], hsml=t[1], m=t[2], rho=t[3], bin_q=t[4], weights=t[5], out=out,
+                         n=n, nq=nq, npix=npix, len2pix=float(npix), kernel=s2g.Cubic(2)))
+        singles.append(s2g.deposit(x, h, m, rho, q if nq > 1 else q[:, 0], w, npix=npix,
+                                   len2pix=float(npix), kernel=s2g.Cubic(2), calc_mean=False))
+    s2g.deposit_batch_device(maps, dtype="f64")
+    for d, ref in zip(maps, singles):
+        got = d["out"].cpu().numpy().reshape(ref.shape, order="F")
+        np.testing.assert_allclose(got, ref, rtol=0, atol=1e-12 * max(np.abs(ref).max(), 1e-300))
