@@ -21,6 +21,8 @@
 // relative accuracy even at pixel-scale angles.
 #include "k_healpix.h"
 
+#include <type_traits>
+
 namespace s2g {
 
 constexpr double kPi = 3.14159265358979323846;
@@ -143,15 +145,15 @@ __device__ __forceinline__ void hp_pix2ring(int64_t nside, int64_t pix, int64_t 
     }
 }
 
-// The pixel interval of ring iz inside the disc: [lo, hi] ring-local, where
-// lo may be negative (wrap: pixels lo+nr .. nr-1 and 0 .. hi).  Returns
-// false if the ring contributes no pixel.  Mirrors the per-ring step of the
-// disc query (non-inclusive: pixel centres within the radius).
-__device__ __forceinline__ bool hp_ring_interval(int64_t nside, int64_t iz, double z0,
-                                                 double xa, double cosr, double phi0,
-                                                 int64_t &lo, int64_t &hi)
+// The pixel interval of a ring (nr pixels, cosine z of its colatitude) inside
+// the disc: [lo, hi] ring-local, where lo may be negative (wrap: pixels
+// lo+nr .. nr-1 and 0 .. hi).  Returns false if the ring contributes no
+// pixel.  Mirrors the per-ring step of the disc query (non-inclusive: pixel
+// centres within the radius).
+__device__ __forceinline__ bool hp_ring_interval(int nr, double shift, double z, double z0,
+                                                 double xa, double cosr, double phi0, int &lo,
+                                                 int &hi)
 {
-    const double z = hp_ring_z(nside, iz);
     const double x = (cosr - z * z0) * xa;
     const double ysq = 1.0 - z * z - x * x;
     double dphi;
@@ -161,12 +163,9 @@ __device__ __forceinline__ bool hp_ring_interval(int64_t nside, int64_t iz, doub
         dphi = atan2(sqrt(ysq), x);
     if (!(dphi > 0.0))
         return false;
-    int64_t start, nr;
-    double shift;
-    hp_ring_info(nside, iz, start, nr, shift);
     const double inv2pi = 1.0 / (2.0 * kPi);
-    int64_t a = (int64_t)floor((double)nr * inv2pi * (phi0 - dphi) - shift) + 1;
-    int64_t b = (int64_t)floor((double)nr * inv2pi * (phi0 + dphi) - shift);
+    int a = (int)floor((double)nr * inv2pi * (phi0 - dphi) - shift) + 1;
+    int b = (int)floor((double)nr * inv2pi * (phi0 + dphi) - shift);
     if (a > b)
         return false;
     if (b >= nr) {
@@ -182,12 +181,11 @@ __device__ __forceinline__ bool hp_ring_interval(int64_t nside, int64_t iz, doub
 // the first one at or after phi0 - pi (lo may be negative, as above), so that
 // phi - phi0 stays in [-pi, pi) along the chord and the pixel loops need no
 // wrap of it.  The same set as [0, nr - 1], in another order.
-__device__ __forceinline__ void hp_full_chord(int64_t nr, double shift, double phi0,
-                                              int64_t &lo, int64_t &hi)
+__device__ __forceinline__ void hp_full_chord(int nr, double shift, double phi0, int &lo, int &hi)
 {
     const double inv2pi = 1.0 / (2.0 * kPi);
-    int64_t a = (int64_t)floor((double)nr * inv2pi * (phi0 - kPi) - shift) + 1;
-    int64_t b = a + nr - 1;
+    int a = (int)floor((double)nr * inv2pi * (phi0 - kPi) - shift) + 1;
+    int b = a + nr - 1;
     if (b >= nr) {
         a -= nr;
         b -= nr;
@@ -300,8 +298,6 @@ struct RingTerms {
     float s1, s2;      // sin^2(dtheta/2), sin(theta_ring) sin(theta0)
     double dphi_pix;   // 2 pi / nr
     double phase;      // shift * dphi_pix - phi0
-    int64_t start;
-    int64_t nr;
 };
 
 // Per-ring half-angle terms (ring iz at rtab[iz]): sin(theta_ring / 2) =
@@ -324,18 +320,16 @@ void launch_hp_ring_table(int64_t nside, double4 *rtab, hipStream_t s)
                        s, nside, rtab);
 }
 
-__device__ __forceinline__ RingTerms ring_terms(int64_t nside, int64_t iz, const HpRec &r,
-                                                const double4 *__restrict__ rtab)
+// q: the ring's table entry
+__device__ __forceinline__ RingTerms ring_terms(int nr, double shift, const HpRec &r,
+                                                const double4 &q)
 {
     RingTerms t;
-    double shift;
-    hp_ring_info(nside, iz, t.start, t.nr, shift);
     // sin((theta_ring - theta0) / 2) from the half-angle terms of both colatitudes
-    const double4 q = rtab[iz];
     const double sh = q.x * r.ch0 - q.y * r.sh0;
     t.s1 = (float)(sh * sh);
     t.s2 = (float)(q.z * r.sth0);
-    t.dphi_pix = 2.0 * kPi / (double)t.nr;
+    t.dphi_pix = 2.0 * kPi / (double)nr;
     t.phase = shift * t.dphi_pix - r.phi0;
     return t;
 }
@@ -346,7 +340,7 @@ __device__ __forceinline__ RingTerms ring_terms(int64_t nside, int64_t iz, const
 // adds -2 pi or +2 pi; the representative is taken in [-pi - 1e-9, pi / 2),
 // so a start a rounding below -pi keeps its place and the chord's offsets
 // run up to < pi (nr >= 4).
-__device__ __forceinline__ double hp_chord_start(int64_t a, const RingTerms &t)
+__device__ __forceinline__ double hp_chord_start(int a, const RingTerms &t)
 {
     double d0 = (double)a * t.dphi_pix + t.phase;
     d0 = d0 >= 0.5 * kPi ? d0 - 2.0 * kPi : d0;
@@ -367,65 +361,73 @@ __device__ __forceinline__ float hp_sin(float y)
     return fmaf(y * y2, p, y);
 }
 
-// asin(x) for 0 <= x <= 1: x (1 + x^2 P(x^2)) with P of degree 4 fitted
+// asin(x) for 0 <= x <= 1/2: x (1 + x^2 P(x^2)) with P of degree 4 fitted
 // for the least maximum relative error on [0, 1/2] (4.9e-9; the FP32
 // evaluation adds ~6e-8), which covers every pixel closer than pi/3 to the
 // particle; the library function above.  The choice is per pixel, so a
 // pixel's weight does not depend on which pixels share its wave.
-__device__ __forceinline__ float hp_asin(float x)
+__device__ __forceinline__ float hp_asin_near(float x)
 {
-    if (x <= 0.5f) {
-        const float t = x * x;
-        float p = fmaf(t, 4.216631e-02f, 2.417951e-02f);
-        p = fmaf(t, p, 4.547038e-02f);
-        p = fmaf(t, p, 7.495297e-02f);
-        p = fmaf(t, p, 1.6666752e-01f);
-        return fmaf(x * t, p, x);
-    }
-    return asinf(x);
+    const float t = x * x;
+    float p = fmaf(t, 4.216631e-02f, 2.417951e-02f);
+    p = fmaf(t, p, 4.547038e-02f);
+    p = fmaf(t, p, 7.495297e-02f);
+    p = fmaf(t, p, 1.6666752e-01f);
+    return fmaf(x * t, p, x);
 }
 
-// angular distance from the haversine: hav(d) = sin^2(dtheta / 2) +
-// sin(theta) sin(theta0) sin^2(dphi / 2), d = 2 asin(sqrt(hav)).  The one
-// formula for every pixel of the norm and deposit passes, so both see the
-// same weights.
-__device__ __forceinline__ float hp_angle(float dphi, float s1, float s2)
+// Half the angular distance from the haversine: hav(d) = sin^2(dtheta / 2) +
+// sin(theta) sin(theta0) sin^2(dphi / 2), d / 2 = asin(sqrt(hav)); hphi is
+// dphi / 2.  The one formula for every pixel of the norm and deposit passes,
+// so both see the same weights.
+// NEAR: every distance of the loop is below pi/3 (hp_near), so the angle's
+// argument needs neither the clamp to 1 nor the library branch; the same
+// value for such a pixel.
+template <bool NEAR>
+__device__ __forceinline__ float hp_half_angle(float hphi, float s1, float s2)
 {
-    const float sx = hp_sin(0.5f * dphi);
-    const float hav = fminf(fmaf(s2, sx * sx, s1), 1.0f);
-    return 2.0f * hp_asin(__builtin_amdgcn_sqrtf(hav));
+    const float sx = hp_sin(hphi);
+    const float hav = fmaf(s2, sx * sx, s1);
+    const float x = __builtin_amdgcn_sqrtf(NEAR ? hav : fminf(hav, 1.0f));
+    return NEAR || x <= 0.5f ? hp_asin_near(x) : asinf(x);
 }
 
-// angular distance (radians) from the particle to pixel k of the ring
-__device__ __forceinline__ float hp_dist(const RingTerms &t, int64_t k)
+// A disc whose pixels (centres within the radius theta) are all closer than
+// pi/3 = 1.047 by more than any rounding; false for a NaN radius.
+__device__ __forceinline__ bool hp_near(double theta) { return theta <= 1.0; }
+
+// half the angular distance (radians) from the particle to pixel k of the ring
+__device__ __forceinline__ float hp_dist(const RingTerms &t, int k)
 {
     double dphi = (double)k * t.dphi_pix + t.phase;  // phi_k - phi0
     dphi = dphi > kPi ? dphi - 2.0 * kPi : dphi;
     dphi = dphi < -kPi ? dphi + 2.0 * kPi : dphi;
-    return hp_angle((float)dphi, t.s1, t.s2);
+    return hp_half_angle<false>(0.5f * (float)dphi, t.s1, t.s2);
 }
 
 // W = shape(d / theta) and the area fraction (pixel_weights.jl:6-8, without
 // the constant 1/(ang_pix*dx)^2 that cancels):
 // A = max(0, min(ang, |theta - (d - ang / 2)|)) / ang, with thh = theta +
-// ang / 2 formed once per particle (the clamp is one v_med3_f32)
+// ang / 2 formed once per particle (the clamp is one v_med3_f32).  hd = d / 2
+// and inv2 = 2 / theta: factors of two move between the operands exactly.
 template <int K>
-__device__ __forceinline__ void hp_weights(float d, float thh, float inv_theta, float ang,
+__device__ __forceinline__ void hp_weights(float hd, float thh, float inv2, float ang,
                                            float inv_ang, float &W, float &A)
 {
-    W = shape_row<K>(d * inv_theta, 1.0f);
-    A = __builtin_amdgcn_fmed3f(fabsf(thh - d), 0.0f, ang) * inv_ang;
+    W = shape_row<K>(hd * inv2, 1.0f);
+    A = __builtin_amdgcn_fmed3f(fabsf(fmaf(-2.0f, hd, thh)), 0.0f, ang) * inv_ang;
 }
 
 // One ring of a work unit, as the pixel loop reads it (per-wave LDS table).
+// Half angles, as hp_half_angle takes them.
 struct HpRing {
-    int off;     // first position of the ring's chord in the unit's pixel list
+    float off;   // first position of the ring's chord in the unit's pixel list
+    float base;  // (phi of the chord's first pixel - phi0) / 2, in [-pi/2, pi/2)
+    float step;  // pi / nr
+    float s1, s2;
     int lo;      // ring-local index of the chord's first pixel (< 0: wraps)
     int start;   // RING index of the ring's first pixel
     int nr;      // pixels in the ring
-    float s1, s2;
-    float base;  // phi of the chord's first pixel - phi0, in [-pi, pi)
-    float step;  // 2 pi / nr
 };
 
 __device__ __forceinline__ int wave_incl_scan(int v, int ln)
@@ -438,27 +440,58 @@ __device__ __forceinline__ int wave_incl_scan(int v, int ln)
     return v;
 }
 
-// Iterate the pixels of unit `ui` of particle r: rings [ra + 64*ui, ...].
-// Phase 1: lane l computes the pixel interval and the terms of ring
-// ra + 64*ui + l and writes them to the wave's LDS table `tab`, with its
-// chord's offset in the unit's pixel list (wave prefix sum).  Phase 2: lane
-// l takes list positions l, l + 64, ..., walking forward through the table,
-// so every lane holds a pixel until the list ends.
-// F(pix, W, A) is called per pixel on every lane that holds a pixel.
-template <int K, typename F>
-__device__ __forceinline__ void hp_unit_pixels(int64_t nside, const HpRec &r, int ui, int ln,
-                                               float ang, HpRing *tab,
-                                               const double4 *__restrict__ rtab, F &&f)
+// The pixel list of a wave's table of chords: lane l takes positions l, l + 64,
+// ... < total, walking forward through the table (whose entry after the last
+// one has off = total), so every lane holds a pixel until the list ends.
+// B(cur, c, pos) is called per position: its chord, the offset c along it (in
+// FP32, exact: lists stay far below 2^24, which saves the loop a conversion)
+// and the position.
+template <typename E, typename B>
+__device__ __forceinline__ void hp_walk(const E *tab, int total, int ln, B &&body)
 {
-    const float thh = (float)r.theta + 0.5f * ang, inv_theta = (float)(1.0 / r.theta);
-    const float inv_ang = 1.0f / ang;
-    const double cosr = r.cosr;
-    const int64_t r0 = (int64_t)r.ra + (int64_t)ui * kHpRingsPerUnit;
-    const int64_t r1 = r0 + kHpRingsPerUnit - 1 < r.rb ? r0 + kHpRingsPerUnit - 1 : r.rb;
-    const int nrings = r1 >= r0 ? (int)(r1 - r0 + 1) : 0;
-    const int64_t cring = r.cring, ck = r.ck;
+    const E *next = tab;
+    float end = 0.0f, q = (float)ln;
+    int pos = ln;
+    E cur;
+    auto step = [&]() {
+        if (q >= end) {
+            do {
+                ++next;
+                end = next->off;
+            } while (q >= end);
+            cur = next[-1];
+        }
+        body(cur, q - cur.off, pos);
+    };
+    for (int k = total / kWave; k > 0; --k) {
+        step();
+        q += (float)kWave;
+        pos += kWave;
+    }
+    if (ln < total % kWave)
+        step();
+}
 
-    // phase 1: one ring per lane
+// What a work unit's pixel loop needs of its particle.
+struct HpUnit {
+    int total;                   // pixels in the unit's list
+    float thh, inv2;             // theta + ang / 2, 2 / theta (hp_weights)
+    bool centre;                 // the unit adds the centre pixel by itself
+    float centre_hd;             // half its distance
+};
+
+// Unit `ui` of particle r, rings [ra + 64*ui, ...]: lane l computes the pixel
+// interval and the terms of ring ra + 64*ui + l and writes them to the wave's
+// LDS table `tab` (65 entries), with its chord's offset in the unit's pixel
+// list (wave prefix sum).
+__device__ __forceinline__ HpUnit hp_unit_table(int nside, const HpRec &r, int ui, int ln,
+                                                float ang, HpRing *tab,
+                                                const double4 *__restrict__ rtab)
+{
+    const int r0 = r.ra + ui * kHpRingsPerUnit;
+    const int r1 = r0 + kHpRingsPerUnit - 1 < r.rb ? r0 + kHpRingsPerUnit - 1 : r.rb;
+    const int nrings = r1 >= r0 ? r1 - r0 + 1 : 0;
+    const int cring = r.cring, ck = r.ck;
     HpRing e;
     e.lo = 0;
     e.start = 0;
@@ -467,78 +500,87 @@ __device__ __forceinline__ void hp_unit_pixels(int64_t nside, const HpRec &r, in
     int len = 0;
     bool cov = false;
     if (ln < nrings) {
-        const int64_t iz = r0 + ln;
-        int64_t a = 0, b = -1;
-        bool any;
-        if (iz < r.irmin || iz > r.irmax) {  // a ring fully inside a polar cap
-            int64_t st, n_r;
-            double sh;
-            hp_ring_info(nside, iz, st, n_r, sh);
-            hp_full_chord(n_r, sh, r.phi0, a, b);
-            any = true;
-        } else {
-            any = hp_ring_interval(nside, iz, r.z0, r.xa, cosr, r.phi0, a, b);
-        }
+        const int iz = r0 + ln;
+        int64_t st, n_r;
+        double shift;
+        hp_ring_info(nside, iz, st, n_r, shift);
+        const int nr = (int)n_r;
+        const double4 q = rtab[iz];
+        int a = 0, b = -1;
+        bool any = true;
+        if (iz < r.irmin || iz > r.irmax)  // a ring fully inside a polar cap
+            hp_full_chord(nr, shift, r.phi0, a, b);
+        else
+            any = hp_ring_interval(nr, shift, q.w, r.z0, r.xa, r.cosr, r.phi0, a, b);
         if (any) {
-            const RingTerms t = ring_terms(nside, iz, r, rtab);
-            e.lo = (int)a;
-            len = (int)(b - a + 1);
-            e.start = (int)t.start;
-            e.nr = (int)t.nr;
+            const RingTerms t = ring_terms(nr, shift, r, q);
+            e.lo = a;
+            len = b - a + 1;
+            e.start = (int)st;
+            e.nr = nr;
             e.s1 = t.s1;
             e.s2 = t.s2;
-            e.base = (float)hp_chord_start(a, t);
-            e.step = (float)t.dphi_pix;
+            e.base = 0.5f * (float)hp_chord_start(a, t);
+            e.step = 0.5f * (float)t.dphi_pix;
             if (iz == cring)
-                cov = (a >= 0 && ck >= a && ck <= b) || (a < 0 && (ck <= b || ck >= a + t.nr));
+                cov = (a >= 0 && ck >= a && ck <= b) || (a < 0 && (ck <= b || ck >= a + nr));
         }
     }
     const bool covered_cp = __ballot(cov) != 0ull;
     const int incl = wave_incl_scan(len, ln);
-    const int total = __shfl(incl, kWave - 1, kWave);
-    e.off = incl - len;
+    HpUnit u;
+    u.total = __builtin_amdgcn_readfirstlane(__shfl(incl, kWave - 1, kWave));
+    u.thh = (float)r.theta + 0.5f * ang;
+    u.inv2 = 2.0f * (float)(1.0 / r.theta);
+    e.off = (float)(incl - len);
     __builtin_amdgcn_wave_barrier();
     tab[ln] = e;
-    __builtin_amdgcn_wave_barrier();
-
-    // phase 2: the unit's pixel list, 64 positions at a time
-    int j = -1, next = 0;
-    HpRing cur = e;
-    for (int q = ln; q < total; q += kWave) {
-        while (q >= next) {
-            ++j;
-            cur = tab[j];
-            next = j + 1 < kWave ? tab[j + 1].off : total;
-        }
-        const int c = q - cur.off;
-        int k = cur.lo + c;
-        k = k < 0 ? k + cur.nr : k;
-        // in [-pi, pi] up to FP32 rounding: every chord starts at or after
-        // phi0 - pi and spans less than 2 pi (hp_ring_interval, hp_full_chord)
-        const float dphi = fmaf((float)c, cur.step, cur.base);
-        const float d = hp_angle(dphi, cur.s1, cur.s2);
-        float W, A;
-        hp_weights<K>(d, thh, inv_theta, ang, inv_ang, W, A);
-        f((int64_t)cur.start + k, W, A);
-    }
+    if (ln == 0)
+        tab[kWave].off = (float)u.total;
     __builtin_amdgcn_wave_barrier();
     // constributing_pixels.jl:16-19: the pixel containing the particle is
     // added if the disc query did not return it (handled by the unit that
     // owns its ring, or by unit 0 if its ring is outside [ra, rb])
     const bool own = (cring >= r0 && cring <= r1) ||
                      (ui == 0 && (cring < r.ra || cring > r.rb || r.rb < r.ra));
-    if (own && !covered_cp && ln == 0) {
-        const RingTerms t = ring_terms(nside, cring, r, rtab);
-        const float d = hp_dist(t, ck);
+    u.centre = own && !covered_cp;
+    u.centre_hd = 0.0f;
+    if (u.centre) {
+        int64_t st, n_r;
+        double shift;
+        hp_ring_info(nside, cring, st, n_r, shift);
+        u.centre_hd = hp_dist(ring_terms((int)n_r, shift, r, rtab[cring]), ck);
+    }
+    return u;
+}
+
+// Iterate a unit's pixels: F(pix, W, A) per pixel, on every lane that holds
+// one.  In [-pi, pi] up to FP32 rounding: every chord starts at or after
+// phi0 - pi and spans less than 2 pi (hp_ring_interval, hp_full_chord).
+template <int K, bool NEAR, typename F>
+__device__ __forceinline__ void hp_unit_pixels(const HpUnit &u, const HpRec &r, int ln, float ang,
+                                               const HpRing *tab, F &&f)
+{
+    const float inv_ang = 1.0f / ang;
+    hp_walk(tab, u.total, ln, [&](const HpRing &e, float c, int) {
+        int k = e.lo + (int)c;
+        k = k < 0 ? k + e.nr : k;
         float W, A;
-        hp_weights<K>(d, thh, inv_theta, ang, inv_ang, W, A);
+        hp_weights<K>(hp_half_angle<NEAR>(fmaf(c, e.step, e.base), e.s1, e.s2), u.thh, u.inv2,
+                      ang, inv_ang, W, A);
+        f((int64_t)e.start + k, W, A);
+    });
+    if (u.centre && ln == 0) {
+        float W, A;
+        hp_weights<K>(u.centre_hd, u.thh, u.inv2, ang, inv_ang, W, A);
         f(r.cpix, W, A);
     }
 }
 
-// Per unit: sum of W*A in FP64 and of A in FP32 (A is needed only in the
-// fallback, i.e. when no pixel centre lies inside the kernel, which happens
-// only for discs of a few pixels).
+// Per unit: sum of W*A in FP64 and of A in FP32.  A's sum is needed only in
+// the fallback, i.e. when no pixel centre lies inside the kernel, which
+// happens only for discs of a few pixels; W*A >= 0, so a unit whose own sum
+// is not 0 rules it out and leaves A's at 0.
 template <int K>
 __device__ __forceinline__ void k_hp_norm_one(int64_t gw, const int2 *__restrict__ units,
                                               const HpRec *__restrict__ rec, int64_t nside,
@@ -547,29 +589,40 @@ __device__ __forceinline__ void k_hp_norm_one(int64_t gw, const int2 *__restrict
 {
     const int ln = threadIdx.x % kWave;
     const int2 u = units[gw];
-    const HpRec r = rec[u.x];
+    const HpRec r = rec[__builtin_amdgcn_readfirstlane(u.x)];
     const float ang = (float)sqrt(4.0 * kPi / (double)(12 * nside * nside));
-    double swa = 0.0;
-    float sa = 0.0f;
-    hp_unit_pixels<K>(nside, r, u.y, ln, ang, tab, rtab, [&](int64_t, float W, float A) {
-        swa += (double)(W * A);
-        sa += A;
-    });
+    const HpUnit t = hp_unit_table((int)nside, r, __builtin_amdgcn_readfirstlane(u.y), ln, ang,
+                                   tab, rtab);
+    double swa = 0.0, sad = 0.0;
+    const auto add = [&](int64_t, float W, float A) { swa += (double)(W * A); };
+    if (hp_near(r.theta))
+        hp_unit_pixels<K, true>(t, r, ln, ang, tab, add);
+    else
+        hp_unit_pixels<K, false>(t, r, ln, ang, tab, add);
     swa = wave_sum(swa);
-    const double sad = wave_sum((double)sa);
+    if (__ballot(swa == 0.0)) {
+        float sa = 0.0f;
+        hp_unit_pixels<K, false>(t, r, ln, ang, tab, [&](int64_t, float, float A) { sa += A; });
+        sad = wave_sum((double)sa);
+    }
+    __builtin_amdgcn_wave_barrier();
     if (ln == 0)
         part[gw] = make_double4(swa, sad, 0.0, 0.0);
 }
-// Held to 128 VGPRs (four waves per SIMD): the spills sit in the per-unit
-// ring set-up, and the pixel loop gains more from the occupancy (norm pass
-// 87 -> 61 ms per map on the all-sky workload).
+// Bound by VALU issue (0.99 of the rate before), so the loop is cut to what a
+// pixel's value needs: chord tables in half angles with an end mark, list
+// positions kept in FP32, no clamp or library branch for discs below 1 radian
+// and no sum of A where the fallback is ruled out take 45 VALU instructions
+// per 64 pixels to 34; the unit's particle in scalar registers and 32-bit ring
+// indexes take the set-up out of scratch (96 VGPRs, five waves per SIMD).
+// 2^22 particles at Nside 1024 (7,600 pixels each): 36.0 -> 23.3 ms.
 template <int K>
 __global__ __launch_bounds__(256, 4) void k_hp_norm(const int2 *__restrict__ units, int64_t nu,
                                                  const HpRec *__restrict__ rec, int64_t nside,
                                                  const double4 *__restrict__ rtab,
                                                  double4 *__restrict__ part)
 {
-    __shared__ HpRing s_tab[256 / kWave][kWave];
+    __shared__ HpRing s_tab[256 / kWave][kWave + 1];
     const int64_t nw = (int64_t)gridDim.x * (blockDim.x / kWave);
     for (int64_t gw = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave; gw < nu;
          gw += nw)
@@ -631,7 +684,8 @@ __device__ __forceinline__ void k_hp_deposit_one(int64_t gw, const int2 *__restr
         hp_map_scale<T>(g, k, u.x, r.s, flags, sw[k], bq[k]);
     const float ang = (float)sqrt(4.0 * kPi / (double)(12 * nside * nside));
     const bool fb = r.fb != 0;
-    hp_unit_pixels<K>(nside, r, u.y, ln, ang, tab, g.rtab, [&](int64_t pix, float W, float A) {
+    const HpUnit t = hp_unit_table((int)nside, r, u.y, ln, ang, tab, g.rtab);
+    hp_unit_pixels<K, false>(t, r, ln, ang, tab, [&](int64_t pix, float W, float A) {
         const double wa = (double)((fb ? 1.0f : W) * A);
 #pragma unroll
         for (int k = 0; k < NM; ++k) {
@@ -642,6 +696,7 @@ __device__ __forceinline__ void k_hp_deposit_one(int64_t gw, const int2 *__restr
             }
         }
     });
+    __builtin_amdgcn_wave_barrier();
 }
 template <typename T, int K, int NM>
 __global__ __launch_bounds__(256, 4) void k_hp_deposit(const int2 *__restrict__ units, int64_t nu,
@@ -649,7 +704,7 @@ __global__ __launch_bounds__(256, 4) void k_hp_deposit(const int2 *__restrict__ 
                                                     const HpGroup g, uint32_t flags,
                                                     int64_t nside)
 {
-    __shared__ HpRing s_tab[256 / kWave][kWave];
+    __shared__ HpRing s_tab[256 / kWave][kWave + 1];
     const int64_t nw = (int64_t)gridDim.x * (blockDim.x / kWave);
     for (int64_t gw = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave; gw < nu;
          gw += nw)
@@ -667,13 +722,13 @@ __global__ __launch_bounds__(256, 4) void k_hp_deposit(const int2 *__restrict__ 
 // arithmetic), so the deposited weights sum to the normalisation.
 // ---------------------------------------------------------------------------
 constexpr int kHpRingLds = 4096;  // pixels of the longest ring held in LDS
-// One map: 8 waves per ring block, 32 chords per wave and round (two blocks
-// per CU); two maps (four rows, 128 KB): 16 waves, 28 chords per wave, one
-// block per CU.  Either way four waves per SIMD.
+// One map: 8 waves per ring block (two blocks per CU); more: 16 waves, one
+// block per CU (four rows, 128 KB).  Either way four waves per SIMD.  A wave
+// takes 62 chords a round, one per lane, and walks them in two tables of 31
+// and an end mark, which is what fits beside the rows.
 template <int NM>
 constexpr int kHpRingThreads = NM == 1 ? 512 : 1024;
-template <int NM>
-constexpr int kHpRingPairs = NM == 1 ? 32 : 28;
+constexpr int kHpRingPairs = 31;
 
 // The rings a particle deposits to: its disc's rings [ra, rb] and the ring of
 // its centre pixel (constributing_pixels.jl:16-19), which lies outside that
@@ -823,16 +878,16 @@ __global__ __launch_bounds__(256) void k_hp_ring_fill(const uint32_t *__restrict
     }
 }
 
-// one (particle, ring) chord of the ring-major deposit (per-wave LDS table)
-template <int NM>
-struct HpPair {
-    int off;    // first position of the chord in the wave's pixel list
-    int lo;     // ring-local index of the chord's first pixel (< 0: wraps)
-    int ck;     // ring-local index of the centre pixel, or -1 if not added
-    int fb;     // fallback: area weights only
-    float s1, s2, base, step;
-    float theta, inv_theta;  // theta + ang / 2 (hp_weights's thh), 1 / theta
-    double sw[NM], bq[NM];   // per map: pixel scale and quantity
+// one (particle, ring) chord of the ring-major deposit (per-wave LDS table);
+// half angles, as HpRing
+template <int NM, int NW>
+struct alignas(16) HpPair {
+    float off;        // first position of the chord in the wave's pixel list
+    float base, step;
+    float s1, s2;
+    float thh, inv2;  // theta + ang / 2, 2 / theta (hp_weights); 0: area weights only
+    int lo8;          // byte offset in the row of the list's position 0 (< 0: wraps)
+    double sw[NW], bq[NM];  // pixel scale and quantity per map
 };
 
 // Ring of block i.  The hardware hands consecutive blocks to the eight XCDs
@@ -852,136 +907,170 @@ __device__ __forceinline__ int64_t hp_xcd_ring(int64_t i, int64_t G)
     return t / kHpXcdRun * span + x * kHpXcdRun + t % kHpXcdRun;
 }
 
-template <typename T, int K, int NM>
+// one pixel of a chord into the block's rows (`row`: the pixel in the first)
+// NEAR: every scale of the table is 0, with its quantity, or neither tiny nor
+// infinite, so W*A = 0 and nothing else gives a weight of 0.
+template <int NM, int NW, bool NEAR = false>
+__device__ __forceinline__ void hp_row_add(double *row, float w, const HpPair<NM, NW> &c)
+{
+    if (NEAR && w == 0.0f)
+        return;
+    const double wa = (double)w;
+#pragma unroll
+    for (int k = 0; k < NM; ++k) {
+        const double pw = wa * c.sw[NW == 1 ? 0 : k];
+        if (NEAR || pw != 0.0) {
+            if (k < NW)
+                unsafeAtomicAdd(row + (NM + k) * kHpRingLds, pw);
+            unsafeAtomicAdd(row + k * kHpRingLds, c.bq[k] * pw);
+        }
+    }
+}
+
+// Bound by VALU issue and, with four rows, by the LDS pipe (four FP64 atomics
+// per 64 pixels, about ten cycles each per CU).  The set-up of a chord (an
+// FP64 arc cosine and the record's read) costs about as much as 20 pixels of
+// it, so it runs on 62 lanes at once and the two halves of its results take
+// turns in the table, which the rows leave too little LDS for; the centre
+// pixel is added there, out of the pixel loop, whose instructions are those
+// of the norm pass and the row offset.  Two maps of the 2^22-particle set at
+// Nside 1024: 58.4 -> 43.8 ms.
+template <typename T, int K, int NM, int NW>
 __global__ __launch_bounds__(kHpRingThreads<NM>, 4) void k_hp_ring_deposit(
     const int32_t *__restrict__ list, const int64_t *__restrict__ off,
     const HpRec *__restrict__ rec, const HpGroup g, uint32_t flags, int64_t nside)
 {
-    constexpr int kThreads = kHpRingThreads<NM>, kPairs = kHpRingPairs<NM>;
-    __shared__ double s_m[NM][kHpRingLds], s_w[NM][kHpRingLds];
-    __shared__ HpPair<NM> s_tab[kThreads / kWave][kPairs];
-    const int64_t iz = hp_xcd_ring(blockIdx.x, gridDim.x) + 1;  // ring, 1-based
-    int64_t start, nr;
+    constexpr int kThreads = kHpRingThreads<NM>, kPairs = kHpRingPairs;
+    using Pair = HpPair<NM, NW>;
+    __shared__ double s_row[NM + NW][kHpRingLds];  // the maps, then the weights
+    __shared__ Pair s_tab[kThreads / kWave][kPairs + 1];
+    const int iz = (int)hp_xcd_ring(blockIdx.x, gridDim.x) + 1;  // ring, 1-based
+    int64_t start, n_r;
     double shift;
-    hp_ring_info(nside, iz, start, nr, shift);
+    hp_ring_info(nside, iz, start, n_r, shift);
+    const int nr = (int)n_r;
     for (int k = threadIdx.x; k < nr; k += kThreads) {
 #pragma unroll
-        for (int q = 0; q < NM; ++q) {
-            s_m[q][k] = 0.0;
-            s_w[q][k] = 0.0;
-        }
+        for (int q = 0; q < NM + NW; ++q)
+            s_row[q][k] = 0.0;
     }
     __syncthreads();
     const int wv = threadIdx.x / kWave, ln = threadIdx.x % kWave;
-    HpPair<NM> *tab = s_tab[wv];
+    Pair *tab = s_tab[wv];
     const float ang = (float)sqrt(4.0 * kPi / (double)(12 * nside * nside));
     const float inv_ang = 1.0f / ang;
+    const double4 rq = g.rtab[iz];
     const int64_t b = off[iz], e = off[iz + 1];
-    for (int64_t c0 = b + (int64_t)wv * kPairs; c0 < e; c0 += (kThreads / kWave) * kPairs) {
-        // phase 1: lane l < kPairs takes pair c0 + l: its chord on this ring
-        HpPair<NM> q;
-        q.lo = 0;
-        q.ck = -1;
-        q.fb = 0;
-        q.s1 = q.s2 = q.base = q.step = q.theta = q.inv_theta = 0.0f;
+    for (int64_t c0 = b + (int64_t)wv * 2 * kPairs; c0 < e;
+         c0 += (kThreads / kWave) * 2 * kPairs) {
+        // phase 1: lane l < 2 kPairs takes pair c0 + l: its chord on this ring
+        Pair q;
+        q.base = q.step = q.s1 = q.s2 = q.thh = q.inv2 = 0.0f;
+#pragma unroll
+        for (int k = 0; k < NW; ++k)
+            q.sw[k] = 0.0;
 #pragma unroll
         for (int k = 0; k < NM; ++k)
-            q.sw[k] = q.bq[k] = 0.0;
-        int len = 0;
-        if (ln < kPairs && c0 + ln < e) {
+            q.bq[k] = 0.0;
+        int len = 0, lo = 0;
+        bool near = true;
+        if (ln < 2 * kPairs && c0 + ln < e) {
             const int p = list[c0 + ln];
             const HpRec r = rec[p];
             int64_t cring, ck;
             bool extra;
             hp_dep_rings(nside, r, cring, ck, extra);
-            int64_t a = 0, bb = -1;
+            int a = 0, bb = -1;
             bool any = false;
             if (iz >= r.ra && iz <= r.rb) {
                 if (iz < r.irmin || iz > r.irmax) {  // a ring fully inside a polar cap
                     hp_full_chord(nr, shift, r.phi0, a, bb);
                     any = true;
                 } else {
-                    any = hp_ring_interval(nside, iz, r.z0, r.xa, r.cosr, r.phi0, a, bb);
+                    any = hp_ring_interval(nr, shift, rq.w, r.z0, r.xa, r.cosr, r.phi0, a, bb);
                 }
             }
-            const RingTerms t = ring_terms(nside, iz, r, g.rtab);
+            const RingTerms t = ring_terms(nr, shift, r, rq);
             if (any) {
-                q.lo = (int)a;
-                len = (int)(bb - a + 1);
-                q.base = (float)hp_chord_start(a, t);
-                q.step = (float)t.dphi_pix;
+                lo = a;
+                len = bb - a + 1;
+                q.base = 0.5f * (float)hp_chord_start(a, t);
+                q.step = 0.5f * (float)t.dphi_pix;
             }
             q.s1 = t.s1;
             q.s2 = t.s2;
+            q.thh = (float)r.theta + 0.5f * ang;
+            // area weights only: shape(0) in place of W (1 up to the quintic's
+            // constant, see the loop)
+            q.inv2 = r.fb ? 0.0f : 2.0f * (float)(1.0 / r.theta);
+            near = hp_near(r.theta);
+#pragma unroll
+            for (int k = 0; k < NM; ++k) {
+                double sw;
+                hp_map_scale<T>(g, k, p, r.s, flags, sw, q.bq[k]);
+                if (k < NW)
+                    q.sw[k] = sw;
+                // the near loop skips a pixel by W*A alone
+                q.bq[k] = sw == 0.0 ? 0.0 : q.bq[k];
+                near = near && (sw == 0.0 || (fabs(sw) > 1e-250 && fabs(sw) < 1e300));
+            }
             // constributing_pixels.jl:16-19: the centre pixel, if the disc
-            // query did not return it
+            // query did not return it, as the norm pass computes it
             if (iz == cring) {
-                const bool cov = any && ((a >= 0 && ck >= a && ck <= bb) ||
-                                         (a < 0 && (ck <= bb || ck >= a + nr)));
+                const int k = (int)ck;
+                const bool cov = any && ((a >= 0 && k >= a && k <= bb) ||
+                                         (a < 0 && (k <= bb || k >= a + nr)));
                 if (!cov) {
-                    q.ck = (int)ck;
-                    len += 1;
+                    float W, A;
+                    hp_weights<K>(hp_dist(t, k), q.thh, q.inv2, ang, inv_ang, W, A);
+                    hp_row_add<NM, NW>(&s_row[0][k], (r.fb ? 1.0f : W) * A, q);
                 }
             }
-            q.fb = r.fb;
-            q.theta = (float)r.theta + 0.5f * ang;  // theta + ang / 2, as the norm pass
-            q.inv_theta = (float)(1.0 / r.theta);
-#pragma unroll
-            for (int k = 0; k < NM; ++k)
-                hp_map_scale<T>(g, k, p, r.s, flags, q.sw[k], q.bq[k]);
         }
         const int incl = wave_incl_scan(len, ln);
-        const int total = __shfl(incl, kWave - 1, kWave);
-        q.off = incl - len;
-        __builtin_amdgcn_wave_barrier();
-        if (ln < kPairs)
-            tab[ln] = q;
-        __builtin_amdgcn_wave_barrier();
+        const int half = __builtin_amdgcn_readlane(incl, kPairs - 1);
         // phase 2: the chords' pixels, 64 list positions at a time
-        int j = -1, next = 0;
-        HpPair<NM> cur = q;
-        int clen = 0;
-        for (int pos = ln; pos < total; pos += kWave) {
-            while (pos >= next) {
-                ++j;
-                cur = tab[j];
-                next = j + 1 < kPairs ? tab[j + 1].off : total;
-                clen = next - cur.off - (cur.ck >= 0 ? 1 : 0);
+#pragma unroll 1
+        for (int h = 0; h < 2; ++h) {
+            const int total =
+                h == 0 ? half : __builtin_amdgcn_readlane(incl, 2 * kPairs - 1) - half;
+            const int j = ln - h * kPairs, first = incl - len - (h == 0 ? 0 : half);
+            const bool mine = j >= 0 && j < kPairs;
+            __builtin_amdgcn_wave_barrier();
+            if (mine) {
+                q.off = (float)first;
+                q.lo8 = 8 * (lo - first);
+                tab[j] = q;
             }
-            const int c = pos - cur.off;
-            int k;
-            float d;
-            if (c < clen) {
-                k = cur.lo + c;
-                k = k < 0 ? k + (int)nr : k;
-                // in [-pi, pi] up to FP32 rounding, as in hp_unit_pixels
-                d = hp_angle(fmaf((float)c, cur.step, cur.base), cur.s1, cur.s2);
-            } else {
-                // the centre pixel, as the norm pass computes it
-                k = cur.ck;
-                const HpRec &r = rec[list[c0 + j]];
-                d = hp_dist(ring_terms(nside, iz, r, g.rtab), k);
-            }
-            float W, A;
-            hp_weights<K>(d, cur.theta, cur.inv_theta, ang, inv_ang, W, A);
-            const double wa = (double)((cur.fb ? 1.0f : W) * A);
-#pragma unroll
-            for (int m = 0; m < NM; ++m) {
-                const double pw = wa * cur.sw[m];
-                if (pw != 0.0) {
-                    unsafeAtomicAdd(&s_w[m][k], pw);
-                    unsafeAtomicAdd(&s_m[m][k], cur.bq[m] * pw);
-                }
-            }
+            if (ln == 0)
+                tab[kPairs].off = (float)total;
+            __builtin_amdgcn_wave_barrier();
+            const auto walk = [&](auto near_c) {
+                constexpr bool NEAR = decltype(near_c)::value;
+                hp_walk(tab, total, ln, [&](const Pair &c, float d, int pos) {
+                    // row offset, wrapped: a negative one is the larger unsigned
+                    const uint32_t k8 = (uint32_t)(c.lo8 + 8 * pos);
+                    const uint32_t o = k8 < k8 + 8u * nr ? k8 : k8 + 8u * nr;
+                    float W, A;
+                    hp_weights<K>(hp_half_angle<NEAR>(fmaf(d, c.step, c.base), c.s1, c.s2), c.thh,
+                                  c.inv2, ang, inv_ang, W, A);
+                    if constexpr (K == S2G_KERNEL_QUINTIC)
+                        W = c.inv2 == 0.0f ? 1.0f : W;
+                    hp_row_add<NM, NW, NEAR>((double *)((char *)s_row + o), W * A, c);
+                });
+            };
+            if (__ballot(mine && !near) == 0)
+                walk(std::true_type());
+            else
+                walk(std::false_type());
         }
-        __builtin_amdgcn_wave_barrier();
     }
     __syncthreads();
     for (int k = threadIdx.x; k < nr; k += kThreads) {
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
-            g.map[m][start + k] = s_m[m][k];
-            g.wmap[m][start + k] = s_w[m][k];
+            g.map[m][start + k] = s_row[m][k];
+            g.wmap[m][start + k] = s_row[NM + (NW == 1 ? 0 : m)][k];
         }
     }
 }
@@ -1102,12 +1191,14 @@ static void hp_ring_deposit_k(const HpArgs &a, const HpGroup &g, const int32_t *
                               const int64_t *off, const HpRec *rec, hipStream_t s)
 {
     const dim3 grid((unsigned)(4 * a.nside - 1));
+#define S2G_HP_RING(NM, NW)                                                     \
+    hipLaunchKernelGGL((k_hp_ring_deposit<T, K, NM, NW>), grid, dim3(kHpRingThreads<NM>), 0, s, \
+                       list, off, rec, g, a.flags, a.nside)
     if (g.nm == 1)
-        hipLaunchKernelGGL((k_hp_ring_deposit<T, K, 1>), grid, dim3(kHpRingThreads<1>), 0, s,
-                           list, off, rec, g, a.flags, a.nside);
+        S2G_HP_RING(1, 1);
     else
-        hipLaunchKernelGGL((k_hp_ring_deposit<T, K, 2>), grid, dim3(kHpRingThreads<2>), 0, s,
-                           list, off, rec, g, a.flags, a.nside);
+        S2G_HP_RING(2, 2);
+#undef S2G_HP_RING
 }
 
 void launch_hp_ring_deposit(const HpArgs &a, const HpGroup &g, const int32_t *list,

@@ -226,3 +226,34 @@ def test_maps_of_one_particle_set(s2g, orc, nside):
             e1, e2 = rel_l1(got[k][0], om), rel_l1(got[k][1], ow)
             print(f"[maps nside={nside} cm={cm} map {k}] rel_l1 {e1:.2e} {e2:.2e}", flush=True)
             assert e1 <= 1e-5 and e2 <= 1e-5
+
+
+@pytest.mark.parametrize("kname", ["quintic", "wendlandc4"])
+@pytest.mark.parametrize("n", [1, 31, 32, 62, 63, 500])
+def test_chord_tables_and_near_discs(s2g, orc, kname, n):
+    """The ring-major deposit's chord tables (31 and 62 chords a round, an end
+    mark after each) on rings that every particle touches, with discs on both
+    sides of the 1 radian up to which the pixel loops need no clamp, and some
+    that hold no pixel centre."""
+    r = np.random.default_rng(n)
+    v = np.array([0.3, 0.2, 0.5]) + 0.02 * r.standard_normal((n, 3))
+    pos = v / np.linalg.norm(v, axis=1)[:, None]
+    theta = r.uniform(0.5, 1.5, n)
+    theta[1::5] = 1e-3
+    h, m, rho, q, w = (np.sin(theta), *(r.uniform(0.5, 2.0, n) for _ in range(4)))
+    _compare(s2g, orc, pos, h, m, rho, q, w, 16, kname, tag=f"chords{n}")
+
+
+@pytest.mark.parametrize("w0,q0", [(0.0, np.inf), (1e-300, 3.0), (0.0, np.nan)])
+def test_zero_and_tiny_scales(s2g, w0, q0):
+    """A particle of zero weight adds nothing, whatever its quantity, and one
+    whose scale nearly underflows nothing that shows (below 1e-290 of the
+    others'); both beside ordinary particles of the same chord tables."""
+    pos, h, m, rho, q, w = _shell(80, 5, hmin=0.05)
+    w[7], q[7] = w0, q0
+    run = lambda s: s2g.healpix_map(pos[s].T.copy(), h[s], m[s], rho[s], q[s], w[s], Nside=32,
+                                    kernel=s2g.WendlandC4(2), show_progress=False)
+    rest = np.arange(80) != 7
+    for a, b in zip(run(slice(None)), run(rest)):
+        # two orders of at most 80 FP64 sums per pixel
+        np.testing.assert_allclose(a, b, rtol=80 * 2.3e-16, atol=1e-280)
