@@ -1,6 +1,8 @@
 // k_healpix.h -- launchers of the all-sky (HEALPix RING) deposit kernels.
 #pragma once
 
+#include <vector>
+
 #include "s2g_internal.h"
 
 namespace s2g {
@@ -33,13 +35,24 @@ struct HpArgs {
     uint32_t flags;
 };
 
-// maps [m0, m0 + nm) of an HpArgs, nm <= 2, and their outputs
+// Maps of an HpArgs that one deposit pass takes, and their outputs: one or two
+// with their own weights (nw = nm), or up to kHpGroupMaps that share them
+// (nw = 1).
+constexpr int kHpGroupMaps = 3;
 struct HpGroup {
-    const void *binq[2], *w[2];
-    double *map[2], *wmap[2];
-    int nm;
+    const void *binq[kHpGroupMaps], *w[kHpGroupMaps];
+    double *map[kHpGroupMaps], *wmap[kHpGroupMaps];
+    int nm, nw;
     const double4 *rtab;  // per-ring terms (launch_hp_ring_table)
 };
+
+// The passes of a call, its maps in order.  A run of maps given the same
+// weight array (a quantity each, all weighted by the mass, say) takes passes of
+// up to three, whose one row of weights is formed once, for the ring-major
+// deposit with calc_mean (without it a map leaves out the particles of which
+// its own quantity is 0, and the weights differ).
+std::vector<HpGroup> hp_groups(const HpArgs &a, double *const *maps, double *const *wmaps,
+                               const double4 *rtab);
 
 // nunits: n+1 int64 (last = 0, the total after an exclusive scan)
 void launch_hp_setup(const HpArgs &a, HpRec *rec, int64_t *nunits, hipStream_t s);

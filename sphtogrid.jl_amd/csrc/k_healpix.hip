@@ -443,15 +443,15 @@ __device__ __forceinline__ int wave_incl_scan(int v, int ln)
 // The pixel list of a wave's table of chords: lane l takes positions l, l + 64,
 // ... < total, walking forward through the table (whose entry after the last
 // one has off = total), so every lane holds a pixel until the list ends.
-// B(cur, c, pos) is called per position: its chord, the offset c along it (in
+// B(cur, c, pos8) is called per position: its chord, the offset c along it (in
 // FP32, exact: lists stay far below 2^24, which saves the loop a conversion)
-// and the position.
+// and eight times the position.
 template <typename E, typename B>
 __device__ __forceinline__ void hp_walk(const E *tab, int total, int ln, B &&body)
 {
     const E *next = tab;
     float end = 0.0f, q = (float)ln;
-    int pos = ln;
+    int pos8 = 8 * ln;
     E cur;
     auto step = [&]() {
         if (q >= end) {
@@ -461,12 +461,12 @@ __device__ __forceinline__ void hp_walk(const E *tab, int total, int ln, B &&bod
             } while (q >= end);
             cur = next[-1];
         }
-        body(cur, q - cur.off, pos);
+        body(cur, q - cur.off, pos8);
     };
     for (int k = total / kWave; k > 0; --k) {
         step();
         q += (float)kWave;
-        pos += kWave;
+        pos8 += 8 * kWave;
     }
     if (ln < total % kWave)
         step();
@@ -907,7 +907,8 @@ __device__ __forceinline__ int64_t hp_xcd_ring(int64_t i, int64_t G)
     return t / kHpXcdRun * span + x * kHpXcdRun + t % kHpXcdRun;
 }
 
-// one pixel of a chord into the block's rows (`row`: the pixel in the first)
+// One pixel of a chord into the block's rows (`row`: the pixel in the first):
+// NM maps and NW rows of weights, NW = NM, or 1 for maps that share theirs.
 // NEAR: every scale of the table is 0, with its quantity, or neither tiny nor
 // infinite, so W*A = 0 and nothing else gives a weight of 0.
 template <int NM, int NW, bool NEAR = false>
@@ -917,12 +918,13 @@ __device__ __forceinline__ void hp_row_add(double *row, float w, const HpPair<NM
         return;
     const double wa = (double)w;
 #pragma unroll
-    for (int k = 0; k < NM; ++k) {
-        const double pw = wa * c.sw[NW == 1 ? 0 : k];
+    for (int j = 0; j < NW; ++j) {
+        const double pw = wa * c.sw[j];
         if (NEAR || pw != 0.0) {
-            if (k < NW)
-                unsafeAtomicAdd(row + (NM + k) * kHpRingLds, pw);
-            unsafeAtomicAdd(row + k * kHpRingLds, c.bq[k] * pw);
+            unsafeAtomicAdd(row + (NM + j) * kHpRingLds, pw);
+#pragma unroll
+            for (int k = j; k < (NW == 1 ? NM : j + 1); ++k)
+                unsafeAtomicAdd(row + k * kHpRingLds, c.bq[k] * pw);
         }
     }
 }
@@ -934,7 +936,10 @@ __device__ __forceinline__ void hp_row_add(double *row, float w, const HpPair<NM
 // turns in the table, which the rows leave too little LDS for; the centre
 // pixel is added there, out of the pixel loop, whose instructions are those
 // of the norm pass and the row offset.  Two maps of the 2^22-particle set at
-// Nside 1024: 58.4 -> 43.8 ms.
+// Nside 1024: 58.4 -> 43.6 ms; 38.3 ms if they share their weights (NW = 1:
+// three atomics and one scale less per entry).  An entry that also holds its
+// chord's end, so that a lane moving on reads one entry instead of the next
+// mark and then the entry, measured 39.9 ms.
 template <typename T, int K, int NM, int NW>
 __global__ __launch_bounds__(kHpRingThreads<NM>, 4) void k_hp_ring_deposit(
     const int32_t *__restrict__ list, const int64_t *__restrict__ off,
@@ -949,6 +954,7 @@ __global__ __launch_bounds__(kHpRingThreads<NM>, 4) void k_hp_ring_deposit(
     double shift;
     hp_ring_info(nside, iz, start, n_r, shift);
     const int nr = (int)n_r;
+    const uint32_t nr8 = 8u * (uint32_t)nr;
     for (int k = threadIdx.x; k < nr; k += kThreads) {
 #pragma unroll
         for (int q = 0; q < NM + NW; ++q)
@@ -1047,10 +1053,10 @@ __global__ __launch_bounds__(kHpRingThreads<NM>, 4) void k_hp_ring_deposit(
             __builtin_amdgcn_wave_barrier();
             const auto walk = [&](auto near_c) {
                 constexpr bool NEAR = decltype(near_c)::value;
-                hp_walk(tab, total, ln, [&](const Pair &c, float d, int pos) {
+                hp_walk(tab, total, ln, [&](const Pair &c, float d, int pos8) {
                     // row offset, wrapped: a negative one is the larger unsigned
-                    const uint32_t k8 = (uint32_t)(c.lo8 + 8 * pos);
-                    const uint32_t o = k8 < k8 + 8u * nr ? k8 : k8 + 8u * nr;
+                    const uint32_t k8 = (uint32_t)(c.lo8 + pos8);
+                    const uint32_t o = k8 < k8 + nr8 ? k8 : k8 + nr8;
                     float W, A;
                     hp_weights<K>(hp_half_angle<NEAR>(fmaf(d, c.step, c.base), c.s1, c.s2), c.thh,
                                   c.inv2, ang, inv_ang, W, A);
@@ -1145,6 +1151,37 @@ void launch_hp_deposit(const HpArgs &a, const HpGroup &g, const int2 *units, int
     }
 }
 
+std::vector<HpGroup> hp_groups(const HpArgs &a, double *const *maps, double *const *wmaps,
+                               const double4 *rtab)
+{
+    std::vector<HpGroup> out;
+    const bool rings = hp_ring_deposit_fits(a.nside) && (a.flags & S2G_FLAG_CALC_MEAN);
+    for (int m0 = 0; m0 < a.nmaps;) {
+        int run = 1;
+        while (m0 + run < a.nmaps && a.w[m0 + run] == a.w[m0])
+            ++run;
+        HpGroup g = {};
+        g.rtab = rtab;
+        if (rings && run > 1) {
+            const int passes = (run + kHpGroupMaps - 1) / kHpGroupMaps;
+            g.nm = (run + passes - 1) / passes;
+            g.nw = 1;
+        } else {
+            g.nm = a.nmaps - m0 < 2 ? 1 : 2;
+            g.nw = g.nm;
+        }
+        for (int k = 0; k < g.nm; ++k) {
+            g.binq[k] = a.binq[m0 + k];
+            g.w[k] = a.w[m0 + k];
+            g.map[k] = maps[m0 + k];
+            g.wmap[k] = wmaps[m0 + k];
+        }
+        m0 += g.nm;
+        out.push_back(g);
+    }
+    return out;
+}
+
 bool hp_ring_deposit_fits(int64_t nside) { return 4 * nside <= kHpRingLds; }
 
 void launch_hp_entry_keys(const int2 *units, int64_t nu, const HpRec *rec, int64_t n,
@@ -1196,8 +1233,12 @@ static void hp_ring_deposit_k(const HpArgs &a, const HpGroup &g, const int32_t *
                        list, off, rec, g, a.flags, a.nside)
     if (g.nm == 1)
         S2G_HP_RING(1, 1);
-    else
+    else if (g.nw == 2)
         S2G_HP_RING(2, 2);
+    else if (g.nm == 2)
+        S2G_HP_RING(2, 1);
+    else
+        S2G_HP_RING(3, 1);
 #undef S2G_HP_RING
 }
 

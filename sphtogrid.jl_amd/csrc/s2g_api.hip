@@ -2057,19 +2057,7 @@ static void healpix_device(s2g_ctx *c, const HpArgs &a, double *const *maps,
     // per-ring half-angle terms, once per call
     double4 *rtab = (double4 *)c->hp_rtab.get(sizeof(double4) * 4 * nside);
     launch_hp_ring_table(nside, rtab, s);
-    auto group = [&](int m0) {
-        HpGroup g;
-        g.rtab = rtab;
-        g.nm = a.nmaps - m0 < 2 ? a.nmaps - m0 : 2;
-        for (int k = 0; k < 2; ++k) {
-            const int mk = m0 + (k < g.nm ? k : 0);
-            g.binq[k] = a.binq[mk];
-            g.w[k] = a.w[mk];
-            g.map[k] = maps[mk];
-            g.wmap[k] = wmaps[mk];
-        }
-        return g;
-    };
+    const std::vector<HpGroup> groups = hp_groups(a, maps, wmaps, rtab);
     if (n > 0) {
         HpRec *rec = (HpRec *)c->hp_rec.get(sizeof(HpRec) * n);
         int64_t *nun = (int64_t *)c->hp_nunits.get(sizeof(int64_t) * (n + 1));
@@ -2125,11 +2113,11 @@ static void healpix_device(s2g_ctx *c, const HpArgs &a, double *const *maps,
             launch_hp_ring_fill(keys + ne, vals + ne, eoff, off, nside, list, s2);
             S2G_HIP(hipEventRecord(c->smalled, s2));
             S2G_HIP(hipStreamWaitEvent(s, c->smalled, 0));
-            for (int m0 = 0; m0 < a.nmaps; m0 += 2)
-                launch_hp_ring_deposit(a, group(m0), list, off, rec, s);
+            for (const HpGroup &g : groups)
+                launch_hp_ring_deposit(a, g, list, off, rec, s);
         } else {
-            for (int m0 = 0; m0 < a.nmaps; m0 += 2)
-                launch_hp_deposit(a, group(m0), units, nu, rec, s);
+            for (const HpGroup &g : groups)
+                launch_hp_deposit(a, g, units, nu, rec, s);
         }
         S2G_HIP(hipGetLastError());
         if (st)
@@ -2266,11 +2254,14 @@ int s2g_healpix_deposit_maps(s2g_ctx *c, int dtype, const void *pos, const void 
         for (int k = 0; k < nmaps; ++k) {
             dq[k] = qw + es * cnt * (2 * k);
             dw[k] = qw + es * cnt * (2 * k + 1);
-            if (n > 0) {
-                S2G_HIP(hipMemcpyAsync((void *)dq[k], bin_q[k], es * n, hipMemcpyHostToDevice, s));
+            // maps that share their weights stage them once (hp_groups)
+            if (k > 0 && weights[k] == weights[k - 1])
+                dw[k] = dw[k - 1];
+            else if (n > 0)
                 S2G_HIP(hipMemcpyAsync((void *)dw[k], weights[k], es * n, hipMemcpyHostToDevice,
                                        s));
-            }
+            if (n > 0)
+                S2G_HIP(hipMemcpyAsync((void *)dq[k], bin_q[k], es * n, hipMemcpyHostToDevice, s));
         }
         S2G_HIP(hipEventRecord(e1, s));
         S2G_HIP(hipEventSynchronize(e1));

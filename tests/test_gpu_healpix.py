@@ -257,3 +257,36 @@ def test_zero_and_tiny_scales(s2g, w0, q0):
     for a, b in zip(run(slice(None)), run(rest)):
         # two orders of at most 80 FP64 sums per pixel
         np.testing.assert_allclose(a, b, rtol=80 * 2.3e-16, atol=1e-280)
+
+
+@pytest.mark.parametrize("nmaps,shared", [(2, 2), (3, 3), (4, 4), (5, 3), (7, 7)])
+@pytest.mark.parametrize("nside,cm", [(32, True), (32, False), (1025, True)])
+def test_maps_that_share_weights(s2g, nmaps, shared, nside, cm):
+    """Maps given one weight array (one row of weights per pass), the first
+    `shared` of them, equal the same maps given copies of it."""
+    from sph2grid import _lib
+    pos, h, m, rho, q, w = _shell(300, 17, hmax=0.2 if nside == 32 else 5e-3,
+                                  rmin=0.05 if nside == 32 else 0.5)
+    r = np.random.default_rng(3)
+    w[5] = 0.0
+    qs = [r.uniform(0.5, 2.0, 300) for _ in range(nmaps)]
+    for k in range(nmaps):
+        qs[k][k::9] = 0.0
+    ctx = _lib.default_context()
+    vp = lambda a: a.ctypes.data_as(C.c_void_p)
+    arr = lambda xs: (C.c_void_p * len(xs))(*[x.ctypes.data for x in xs])
+
+    def run(ws):
+        out = [np.full(12 * nside ** 2, np.nan) for _ in range(2 * nmaps)]
+        rc = ctx.lib.s2g_healpix_deposit_maps(
+            ctx.handle, _lib.S2G_F64, vp(pos), vp(h), vp(m), vp(rho), nmaps, arr(qs), arr(ws),
+            300, nside, s2g.WendlandC4(2).kernel_id, 2,
+            _lib.S2G_FLAG_CALC_MEAN if cm else 0, arr(out[:nmaps]), arr(out[nmaps:]), None)
+        ctx.check(rc, "s2g_healpix_deposit_maps")
+        return out
+
+    one = run([w] * shared + [w.copy() for _ in range(nmaps - shared)])
+    own = run([w.copy() for _ in range(nmaps)])
+    for a, b in zip(one, own):
+        # two orders of at most 300 FP64 sums of one sign per pixel
+        np.testing.assert_allclose(a, b, rtol=300 * 2.3e-16, atol=0)
