@@ -21,13 +21,15 @@
 //                  2. the level whose cells are between T0/2 and T0 wide and
 //                     the cube of <= 5^3 cells around the particle that covers
 //                     the ball of radius T0;
-//                  3. every particle in the cube at distance <= T goes to a
+//                  3. the particle ranges of the cells within T0, once, two
+//                     cells a lane;
+//                     every particle in the cube at distance <= T goes to a
 //                     per-wave LDS buffer (T shrinks as the buffer is cut back
 //                     to the k nearest), the cells within T0/2 first: the
 //                     k-th nearest of those gives T1, and of the other cells
 //                     only those within T1 are read; the search works on
 //                     squared distances, and the exact k-th smallest is a
-//                     radix select on their FP64 bit patterns (its square
+//                     bisection on their FP64 bit patterns (its square
 //                     root is hsml);
 //                  4. the kernel sum over the buffer and the bias correction
 //                     of Dehnen & Aly (2012, eqs. 18-19).
@@ -40,10 +42,9 @@
 
 namespace s2g {
 
-constexpr int kMdWaves = 4;     // waves per block of the search
-constexpr int kMdCap = 600;     // candidate buffer per wave
+constexpr int kMdCap = 596;     // candidate buffer per wave (20 waves of 8 KB per CU)
 constexpr int kMdBits = 21;     // Morton bits per axis
-constexpr int kMdMaxCells = 216;  // cube cells per particle (at most 6^3)
+constexpr int kMdMaxCells = 2 * kWave;  // cube cells per particle
 
 template <typename T>
 __global__ __launch_bounds__(256) void k_md_prep(const T *__restrict__ pos,
@@ -147,6 +148,19 @@ __device__ __forceinline__ int64_t md_lower_bound(const uint64_t *__restrict__ K
     return lo;
 }
 
+__device__ __forceinline__ int md_lower_bound32(const uint64_t *__restrict__ K, int lo, int hi,
+                                                uint64_t key)
+{
+    while (lo < hi) {
+        const int mid = lo + (hi - lo) / 2;
+        if (K[mid] < key)
+            lo = mid + 1;
+        else
+            hi = mid;
+    }
+    return lo;
+}
+
 // offsets of the 8^lt cells of level lt (+ the end)
 __global__ void k_md_table(const uint64_t *__restrict__ K, int64_t n, int lt,
                            int32_t *__restrict__ tab)
@@ -180,149 +194,134 @@ __device__ __forceinline__ double md_dist2(const double4 &a, const double4 &b, c
     return add_rn(add_rn(mul_rn(dx, dx), mul_rn(dy, dy)), mul_rn(dz, dz));
 }
 
-// exclusive prefix sum over the lanes of a wave
-__device__ __forceinline__ int wave_excl_scan(int v, int ln)
+// value of another lane (DPP lane pattern) on the rows of the mask, else 0
+template <int kCtrl, int kRows = 0xF>
+__device__ __forceinline__ int dpp_or_0(int v)
 {
-    int x = v;
-    for (int o = 1; o < kWave; o <<= 1) {
-        const int y = __shfl_up(x, o, kWave);
-        if (ln >= o)
-            x += y;
-    }
-    return x - v;
+    return __builtin_amdgcn_update_dpp(0, v, kCtrl, kRows, 0xF, true);
 }
 
-// value of another lane of the same 16-lane row (DPP lane pattern)
-template <int kCtrl>
-__device__ __forceinline__ double dpp_get(double v)
+// inclusive prefix sum over the lanes of a fully active wave
+__device__ __forceinline__ int wave_incl_scan(int v)
 {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), kCtrl, 0xF, 0xF, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), kCtrl, 0xF, 0xF, true);
-    return __hiloint2double(hi, lo);
+    v += dpp_or_0<0x111>(v);       // row_shr 1, 2, 4, 8
+    v += dpp_or_0<0x112>(v);
+    v += dpp_or_0<0x114>(v);
+    v += dpp_or_0<0x118>(v);
+    v += dpp_or_0<0x142, 0xA>(v);  // row_bcast 15 into rows 1 and 3
+    v += dpp_or_0<0x143, 0xC>(v);  // row_bcast 31 into rows 2 and 3
+    return v;
 }
 
-// minimum and maximum over the 64 lanes of a fully active wave, on every lane
-__device__ __forceinline__ void wave_min_max(double &mn, double &mx)
+// keys (NR a lane) below c, over the wave
+template <int NR>
+__device__ __forceinline__ int md_count_below(const uint32_t (&key)[NR], uint32_t c)
 {
-    mn = fmin(mn, dpp_get<0xB1>(mn));  // quad_perm [1, 0, 3, 2]
-    mx = fmax(mx, dpp_get<0xB1>(mx));
-    mn = fmin(mn, dpp_get<0x4E>(mn));  // quad_perm [2, 3, 0, 1]
-    mx = fmax(mx, dpp_get<0x4E>(mx));
-    mn = fmin(mn, dpp_get<0x141>(mn));  // row_half_mirror
-    mx = fmax(mx, dpp_get<0x141>(mx));
-    mn = fmin(mn, dpp_get<0x140>(mn));  // row_mirror
-    mx = fmax(mx, dpp_get<0x140>(mx));
-    double a = mn, b = mx;
+    int m = 0;
 #pragma unroll
-    for (int r = 16; r < kWave; r += 16) {
-        a = fmin(a, __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(mn), r),
-                                     __builtin_amdgcn_readlane(__double2loint(mn), r)));
-        b = fmax(b, __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(mx), r),
-                                     __builtin_amdgcn_readlane(__double2loint(mx), r)));
-    }
-    mn = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(a), 0),
-                          __builtin_amdgcn_readlane(__double2loint(a), 0));
-    mx = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(b), 0),
-                          __builtin_amdgcn_readlane(__double2loint(b), 0));
+    for (int r = 0; r < NR; ++r)
+        m += (int)__popcll(__ballot(key[r] < c));
+    return m;
 }
 
-// k-th smallest (1-based) of the doubles buf[0..cnt) (each +0 or positive),
-// exactly: most-significant-bits-first radix select on the bit patterns.
-// Zeros (the particle itself, coincident particles) are counted apart; the
-// bits above the highest one in which the smallest and largest positive
-// entries differ are common to all of them, so the first 8-bit pass starts
-// there and spreads the entries over many bins (a pass from the top byte
-// sends them all to one bin, and its LDS atomics serialise).  Once the chosen
-// bin holds a single entry, that entry is the k-th: one scan finds it.
-// kExact == false: an upper bound of the k-th smallest instead, for
-// thresholds that only have to keep at least k entries: the upper edge of
-// the bin that holds it once the bins are narrower than 1/16 of a binade
-// (the exponent and four mantissa bits chosen; entries that straddle a power
-// of two where many exponent bits flip can need a second pass for that), or
-// the largest entry if smaller.
-template <bool kExact>
-__device__ double md_select(const double *buf, int cnt, int k, int *hist, int ln)
+// The k-th smallest of the keys between lo and last, of which `under` are
+// below lo and `upto` at most last (under < k <= upto): halves the interval
+// until it is no wider than `width` or holds one key, counting with ballots:
+// NR compares and scalar additions a step, no LDS and no prefix sums.
+template <int NR>
+__device__ __forceinline__ void md_bisect(const uint32_t (&key)[NR], int k, uint32_t width,
+                                          uint32_t &lo, uint32_t &last, int &under, int &upto)
 {
-    double mn = __builtin_inf(), mx = 0.0;
-    int nz = 0;  // uniform
-    for (int e0 = 0; e0 < cnt; e0 += kWave) {
-        const int e = e0 + ln;
-        const double v = e < cnt ? buf[e] : -1.0;
-        nz += (int)__popcll(__ballot(v == 0.0));
-        if (v > 0.0) {
-            mn = fmin(mn, v);
-            mx = fmax(mx, v);
+    while (last - lo >= width && upto - under > 1) {
+        const uint32_t mid = lo + (last - lo) / 2 + 1;
+        const int m = md_count_below<NR>(key, mid);
+        if (m < k) {
+            lo = mid;
+            under = m;
+        } else {
+            last = mid - 1;
+            upto = m;
         }
     }
-    if (k <= nz)
-        return 0.0;
-    k -= nz;
-    wave_min_max(mn, mx);
-    const uint64_t lo = (uint64_t)__double_as_longlong(mn);
-    const uint64_t hi = (uint64_t)__double_as_longlong(mx);
-    if (lo == hi)
-        return mn;
-    int top = 64 - __clzll((long long)(lo ^ hi));  // bits from `top` up are common (top < 64)
-    uint64_t prefix = lo >> top << top;
-    for (;;) {
-        const int w = top < 8 ? top : 8;
-        const int shift = top - w;
-        const uint64_t mask = (1ull << w) - 1;
-        for (int b = ln; b < 256; b += kWave)
-            hist[b] = 0;
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        for (int e = ln; e < cnt; e += kWave) {
-            const uint64_t key = (uint64_t)__double_as_longlong(buf[e]);
-            if (key != 0 && (key >> top) == (prefix >> top))
-                atomicAdd(&hist[(key >> shift) & mask], 1);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        // lane l owns bins 4l .. 4l+3
-        int c4[4], loc = 0;
-        for (int j = 0; j < 4; ++j) {
-            c4[j] = hist[4 * ln + j];
-            loc += c4[j];
-        }
-        const int before = wave_excl_scan(loc, ln);
-        const bool mine = before < k && k <= before + loc;
-        const uint64_t owner = __ballot(mine);
-        const int src = __ffsll((unsigned long long)owner) - 1;
-        int bin = 0, below = 0, nbin = 0;
-        if (mine) {
-            int acc = before;
-            for (int j = 0; j < 4; ++j) {
-                if (k <= acc + c4[j]) {
-                    bin = 4 * ln + j;
-                    below = acc;
-                    nbin = c4[j];
-                    break;
-                }
-                acc += c4[j];
-            }
-        }
-        bin = __shfl(bin, src, kWave);
-        below = __shfl(below, src, kWave);
-        nbin = __shfl(nbin, src, kWave);
-        k -= below;
-        prefix |= (uint64_t)bin << shift;
-        top = shift;
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        if (!kExact && top <= 48)
-            return fmin(__longlong_as_double((long long)(prefix | ((1ull << top) - 1))), mx);
-        if (top == 0)
-            return __longlong_as_double((long long)prefix);
-        if (nbin == 1) {
-            // the one positive entry whose bits from `top` up equal the prefix's
-            for (int e0 = 0; e0 < cnt; e0 += kWave) {
-                const int e = e0 + ln;
-                const uint64_t key = e < cnt ? (uint64_t)__double_as_longlong(buf[e]) : 0;
-                const uint64_t bh = __ballot(key != 0 && (key >> top) == (prefix >> top));
-                if (bh)  // wave-uniform
-                    return __shfl(__longlong_as_double((long long)key),
-                                  __ffsll((unsigned long long)bh) - 1, kWave);
-            }
+}
+
+// k-th smallest (1-based) of the doubles buf[0..cnt) (each +0 or positive and
+// finite), cnt <= 64 NR, exactly: by the high words first (the sign is 0; keys
+// that a lane does not hold are all ones), then, if several entries share the
+// k-th's high word, by their low words.  The search starts from the two
+// binades up to T, which no entry exceeds (for T = infinity, from the three on
+// either side of a sample), and widens where the k-th is not in there.
+// kExact == false: an upper bound of it instead, within 1/16, for thresholds
+// that only have to keep at least k entries.
+template <int NR, bool kExact>
+__device__ __forceinline__ double md_select_of(const double *buf, int cnt, int k, double T, int ln)
+{
+    uint32_t hi[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+        hi[r] = r * kWave + ln < cnt ? (uint32_t)__double2hiint(buf[r * kWave + ln]) : ~0u;
+    constexpr uint32_t kInf = 0x7ff00000u, kBinade = 1u << 20;
+    uint32_t last = (uint32_t)__builtin_amdgcn_readfirstlane(__double2hiint(T));
+    uint32_t lo = last > 2 * kBinade ? last - 2 * kBinade : 0;
+    int upto = cnt;
+    if (last == kInf) {
+        const uint32_t g =
+            (uint32_t)__builtin_amdgcn_readfirstlane(__double2hiint(buf[cnt / 4]));
+        lo = g > 3 * kBinade ? g - 3 * kBinade : 0;
+        last = g + 3 * kBinade;
+        upto = md_count_below<NR>(hi, last + 1);
+        if (upto < k) {
+            last = kInf;
+            upto = cnt;
         }
     }
+    int under = md_count_below<NR>(hi, lo);
+    if (under >= k) {
+        last = lo - 1;
+        upto = under;
+        lo = 0;
+        under = 0;
+    }
+    md_bisect<NR>(hi, k, kExact ? 1 : kBinade / 16, lo, last, under, upto);
+    // the only entry for which `in` holds
+    const auto one = [&](auto &&in) -> double {
+        double v = 0.0;
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            const uint64_t bt = __ballot(in(r));
+            if (bt)  // wave-uniform
+                v = buf[r * kWave + __ffsll((unsigned long long)bt) - 1];
+        }
+        return v;
+    };
+    if (upto - under == 1)
+        return one([&](int r) { return hi[r] - lo <= last - lo; });
+    if (!kExact)
+        return __hiloint2double((int)last, -1);
+    // several with the high word lo == last
+    uint32_t low[NR], l0 = 0, l1 = ~0u;
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+        low[r] = hi[r] == lo ? (uint32_t)__double2loint(buf[r * kWave + ln]) : ~0u;
+    k -= under;
+    upto -= under;
+    under = 0;
+    md_bisect<NR>(low, k, 1, l0, l1, under, upto);
+    if (l0 == l1)
+        return __hiloint2double((int)lo, (int)l0);
+    return one([&](int r) { return hi[r] == lo && low[r] - l0 <= l1 - l0; });
+}
+
+template <bool kExact>
+__device__ __forceinline__ double md_select(const double *buf, int cnt, int k, double T, int ln)
+{
+    static_assert(kMdCap <= 10 * kWave, "the buffer in ten registers a lane");
+    const double v = cnt <= 3 * kWave   ? md_select_of<3, kExact>(buf, cnt, k, T, ln)
+                     : cnt <= 6 * kWave ? md_select_of<6, kExact>(buf, cnt, k, T, ln)
+                                        : md_select_of<10, kExact>(buf, cnt, k, T, ln);
+    // the same on every lane: keeps what follows from it in scalar registers
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(v)));
 }
 
 // keep the entries below T and, of those equal to T, as many as make k in
@@ -365,8 +364,7 @@ __device__ int md_compact(double *buf, int *jb, int cnt, double T, int k, int ln
 // d <= T to the buffer; when it is about to overflow, cut it back to the k
 // nearest.
 __device__ __forceinline__ void md_offer(bool valid, double d, int j, double &T, int &cnt,
-                                         double *buf, int *jb, int *hist, int k1, int ln,
-                                         uint64_t below)
+                                         double *buf, int *jb, int k1, int ln, uint64_t below)
 {
     const bool take = valid && d <= T;
     const uint64_t bt = __ballot(take);
@@ -378,49 +376,71 @@ __device__ __forceinline__ void md_offer(bool valid, double d, int j, double &T,
     cnt += (int)__popcll(bt);
     if (cnt > kMdCap - kWave) {
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        T = md_select<true>(buf, cnt, k1, hist, ln);
+        T = md_select<true>(buf, cnt, k1, T, ln);
         cnt = md_compact(buf, jb, cnt, T, k1, ln);
     }
 }
 
+// The hardware hands consecutive blocks to the eight XCDs in turn; here each
+// XCD takes runs of kMdXcdRun consecutive particles in key order, whose cells
+// are the same few, through its own L2 (runs of 256 to 8192 time alike).  The
+// last n mod (8 kMdXcdRun) particles keep their own order.
+constexpr int kXcds = 8, kMdXcdRun = 1024;
+__device__ __forceinline__ int64_t md_xcd_query(int64_t i, int64_t n)
+{
+    const int64_t span = (int64_t)kXcds * kMdXcdRun;
+    if (i >= n / span * span)
+        return i;
+    const int64_t x = i % kXcds, t = i / kXcds;
+    return t / kMdXcdRun * span + x * kMdXcdRun + t % kMdXcdRun;
+}
+
+// Bound by instruction issue, vector and scalar alike, and by the latency of
+// the cells' searches and candidates, so by the waves in flight: one wave a
+// block, which is replaced as soon as it ends (four in a block waited for the
+// slowest), and 8 KB of LDS, 20 waves per CU.  A particle's cell ranges are
+// searched once for both passes; the selects bisect with ballots from a guessed
+// interval in place of radix passes over LDS histograms; what is the same on
+// all lanes is kept in scalar registers.  2^20 particles in halos, 64
+// neighbours: 9.18 -> 4.95 ms (3,700 -> about 2,000 vector instructions a
+// particle).  A bound from the last particle's neighbours instead of the key
+// order's (median 1.35 times the true distance against 1.27) measured slower,
+// and so did a search of the ranges by quarters (5.57 -> 5.88 ms).
 template <int K>
-__global__ __launch_bounds__(kMdWaves * kWave, 4) void k_md_knn(
+__global__ __launch_bounds__(kWave, 4) void k_md_knn(
     const double4 *__restrict__ S, const uint64_t *__restrict__ SK,
     const int32_t *__restrict__ order, const int32_t *__restrict__ tab, int lt, int64_t n,
     MdGrid g, int k1, int dim, int nneigh, double norm, double *__restrict__ rho_out,
     double *__restrict__ hsml_out)
 {
-    __shared__ double s_d[kMdWaves][kMdCap];
-    __shared__ int s_j[kMdWaves][kMdCap];
-    __shared__ int s_h[kMdWaves][256];
-    __shared__ int s_cs[kMdWaves][kMdMaxCells];  // cube cell: first particle
-    __shared__ int s_cp[kMdWaves][kMdMaxCells + 1];  // prefix of the cells' counts
-    const int wv = threadIdx.x / kWave, ln = threadIdx.x % kWave;
-    double *buf = s_d[wv];
-    int *jb = s_j[wv];
-    int *hist = s_h[wv];
-    int *cstart = s_cs[wv];
-    int *cpre = s_cp[wv];
+    __shared__ double buf[kMdCap];
+    __shared__ int jb[kMdCap];
+    __shared__ int cstart[kMdMaxCells];  // cube cell: first particle
+    __shared__ int cpre[kMdMaxCells];    // prefix of the cells' counts
+    const int ln = threadIdx.x;
     const uint64_t below = ln == 0 ? 0ull : (~0ull >> (kWave - ln));
-    const int64_t nw = (int64_t)gridDim.x * kMdWaves;
-    for (int64_t q = (int64_t)blockIdx.x * kMdWaves + wv; q < n; q += nw) {
+    for (int64_t i = blockIdx.x; i < n; i += gridDim.x) {
+        const int64_t q = md_xcd_query(i, n);
         const double4 me = S[q];
         // 1. first bound: the k-th nearest of the particles next in key
         //    order, k on each side (where the particles on one side are far,
         //    as at the edge of a cluster in key order, the other side alone
         //    still holds k)
         int cnt = 0;
-        double T = 1e300;  // squared distances from here on
+        double T;  // squared distances from here on
         {
-            const int64_t a = q - k1 > 0 ? q - k1 : 0;
-            const int64_t b = q + k1 < n - 1 ? q + k1 : n - 1;
-            for (int64_t t0 = a; t0 <= b; t0 += kWave) {
-                const int64_t t = t0 + ln;
-                const bool valid = t <= b;
-                const double d = valid ? md_dist2(me, S[t], g) : 0.0;
-                md_offer(valid, d, (int)t, T, cnt, buf, jb, hist, k1, ln, below);
+            const int w = k1 < kMdCap / 2 ? k1 : kMdCap / 2 - 1;
+            int64_t a = q - w > 0 ? q - w : 0;
+            int64_t b = q + w < n - 1 ? q + w : n - 1;
+            if (b - a + 1 < k1) {  // a large k near either end
+                a = a < n - k1 ? a : n - k1;
+                b = a + k1 - 1;
             }
-            T = md_select<false>(buf, cnt, k1, hist, ln);  // >= the k-th of these
+            cnt = (int)(b - a) + 1;  // in [k1, kMdCap)
+            for (int t = ln; t < cnt; t += kWave)
+                buf[t] = md_dist2(me, S[a + t], g);
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            T = md_select<false>(buf, cnt, k1, __builtin_inf(), ln);  // >= the k-th of these
         }
         const double T20 = T, T0 = sqrt(T20);
         // 2. level with cells in [T0/2, T0) along the narrowest axis; per
@@ -431,34 +451,49 @@ __global__ __launch_bounds__(kMdWaves * kWave, 4) void k_md_knn(
         //    exceeds T0), so at most six cells per axis
         int lev = kMdBits;
         if (T0 > 0.0) {
-            const int l = (int)floor(log2(g.min_ext / T0)) + 1;
+            const int l = __builtin_amdgcn_frexp_exp(g.min_ext / T0);  // floor(log2) + 1
             lev = l < 0 ? 0 : (l > kMdBits ? kMdBits : l);
         }
-        const uint32_t ncl = 1u << lev;
-        const int sh = kMdBits - lev;
-        int ca[3], cl[3];  // first cell (unwrapped) and cell count per axis
+        uint32_t ncl;
+        int ca[3], cl[3], ncube;  // first cell (unwrapped) and cell count per axis
         const double mv[3] = {me.x, me.y, me.z};
+        int qlo[3], qhi[3];
         for (int d = 0; d < 3; ++d) {
             const double qs = (double)(1u << kMdBits);
-            const int64_t qlo = (int64_t)floor((mv[d] - T0 - g.lo[d]) * g.inv_ext[d] * qs) - 1;
-            const int64_t qhi = (int64_t)floor((mv[d] + T0 - g.lo[d]) * g.inv_ext[d] * qs) + 1;
-            int64_t clo = qlo >> sh, chi = qhi >> sh;  // floor division
-            if (g.periodic) {
-                if (chi - clo + 1 >= (int64_t)ncl) {
-                    clo = 0;
-                    chi = (int64_t)ncl - 1;
+            // far outside the domain (a narrow axis) means all of its cells:
+            // the clamp to 2^28 quanta, 128 domains, keeps that
+            const double far = 268435456.0;
+            const double l = (mv[d] - T0 - g.lo[d]) * g.inv_ext[d] * qs;
+            const double h = (mv[d] + T0 - g.lo[d]) * g.inv_ext[d] * qs;
+            qlo[d] = (int)floor(fmax(l, -far)) - 1;
+            qhi[d] = (int)floor(fmin(h, far)) + 1;
+        }
+        for (;; --lev) {
+            ncl = 1u << lev;
+            const int sh = kMdBits - lev;
+            for (int d = 0; d < 3; ++d) {
+                int clo = qlo[d] >> sh, chi = qhi[d] >> sh;  // floor division
+                if (g.periodic) {
+                    if (chi - clo + 1 >= (int)ncl) {
+                        clo = 0;
+                        chi = (int)ncl - 1;
+                    }
+                } else {
+                    clo = clo < 0 ? 0 : clo;
+                    chi = chi > (int)ncl - 1 ? (int)ncl - 1 : chi;
                 }
-            } else {
-                clo = clo < 0 ? 0 : clo;
-                chi = chi > (int64_t)ncl - 1 ? (int64_t)ncl - 1 : chi;
+                ca[d] = clo;
+                cl[d] = chi - clo + 1;
             }
-            ca[d] = (int)clo;
-            cl[d] = (int)(chi - clo + 1);
+            ncube = cl[0] * cl[1] * cl[2];
+            // two cells a lane: 6 x 6 x 4 cells and more take the next
+            // coarser level, at most 4^3
+            if (ncube <= kMdMaxCells)
+                break;
         }
         // cells whose nearest point is farther than T0 (with a margin of two
         // quanta per axis) hold no candidate
         const double T0m = T0 * (1.0 + 1e-12);
-        const int ncube = cl[0] * cl[1] * cl[2];
         // 3. the cube's particles; cells are ranges of the sorted order.  The
         //    cells whose nearest point lies within T0/2 go first: the k-th
         //    nearest of their particles is a bound T1 close to the true k-th
@@ -471,66 +506,84 @@ __global__ __launch_bounds__(kMdWaves * kWave, 4) void k_md_knn(
         for (int d = 0; d < 3; ++d) {
             const double eps = 2.0 * g.ext[d] / (double)(1u << kMdBits);
             const double xr = mv[d] - g.lo[d];
-            cw[d] = g.ext[d] / (double)ncl;
+            cw[d] = ldexp(g.ext[d], -lev);
             xlo[d] = xr + eps;
             xhi[d] = xr - eps;
             rcl[d] = 1.0f / (float)cl[d];
         }
-        int ncells = 0;  // uniform
-        auto gather_cells = [&](double lo2, double hi2) -> int {
-            // the non-empty cells with lo2 < (nearest distance)^2 <= hi2, in
-            // cube order, into cstart/cpre (first particle, number of the
-            // first candidate) and ncells; returns their particle count
-            // (uniform)
-            int C = 0, nc = 0;
-            for (int t0 = 0; t0 < ncube; t0 += kWave) {
-                const int t = t0 + ln;
-                int s = 0, e = 0;
-                bool near = false;
+        // the cube's cells, two a lane: squared nearest distance (above T0's:
+        // not read), first particle and count
+        double cdd[2];
+        int cs[2], cn[2];
+#pragma unroll
+        for (int z = 0; z < 2; ++z) {
+            const int t = z * kWave + ln;
+            cdd[z] = 1e300;
+            cs[z] = cn[z] = 0;
+            if (z * kWave < ncube && t < ncube) {
                 uint32_t cc[3];
-                if (t < ncube) {
-                    int r = t;
-                    double dd = 0.0;
-                    for (int d = 0; d < 3; ++d) {
-                        // r = q cl + rem with r < 216, cl <= 6: the float
-                        // quotient of r + 1/2 is at least 1/12 from an integer
-                        const int qd = d < 2 ? (int)(((float)r + 0.5f) * rcl[d]) : 0;
-                        int o = ca[d] + (r - qd * cl[d]);
-                        r = qd;
-                        if (cl[d] < (int)ncl || !g.periodic) {
-                            const double a = (double)o * cw[d] - xlo[d];
-                            const double b = xhi[d] - (double)(o + 1) * cw[d];
-                            const double dx = a > 0.0 ? a : (b > 0.0 ? b : 0.0);
-                            dd += dx * dx;
-                        }
-                        o = o < 0 ? o + (int)ncl : (o >= (int)ncl ? o - (int)ncl : o);
-                        cc[d] = (uint32_t)o;
+                int r = t;
+                double dd = 0.0;
+                for (int d = 0; d < 3; ++d) {
+                    // r = q cl + rem with r < 216, cl <= 6: the float
+                    // quotient of r + 1/2 is at least 1/12 from an integer
+                    const int qd = d < 2 ? (int)(((float)r + 0.5f) * rcl[d]) : 0;
+                    int o = ca[d] + (r - qd * cl[d]);
+                    r = qd;
+                    if (cl[d] < (int)ncl || !g.periodic) {
+                        const double a = (double)o * cw[d] - xlo[d];
+                        const double b = xhi[d] - (double)(o + 1) * cw[d];
+                        const double dx = a > 0.0 ? a : (b > 0.0 ? b : 0.0);
+                        dd += dx * dx;
                     }
-                    near = dd > lo2 && dd <= hi2;
+                    o = o < 0 ? o + (int)ncl : (o >= (int)ncl ? o - (int)ncl : o);
+                    cc[d] = (uint32_t)o;
                 }
-                if (near) {
+                if (dd <= T0m * T0m) {
                     const uint64_t pre = md_morton(cc[0], cc[1], cc[2]);  // 3*lev bits
+                    int s, e;
                     if (lev <= lt) {
                         s = tab[pre << (3 * (lt - lev))];
                         e = tab[(pre + 1) << (3 * (lt - lev))];
                     } else {
                         const uint64_t par = pre >> (3 * (lev - lt));
-                        const int64_t ps = tab[par], pe = tab[par + 1];
                         const int ksh = 3 * (kMdBits - lev);
-                        s = (int)md_lower_bound(SK, ps, pe, pre << ksh);
-                        e = (int)md_lower_bound(SK, s, pe, (pre + 1) << ksh);
+                        s = tab[par];
+                        e = tab[par + 1];
+                        s = md_lower_bound32(SK, s, e, pre << ksh);
+                        // the cell holds few of the parent's particles
+                        const uint64_t end = (pre + 1) << ksh;
+                        const bool more = s + 32 < e && SK[s + 32] < end;
+                        e = md_lower_bound32(SK, more ? s + 33 : s,
+                                            more || e < s + 32 ? e : s + 32, end);
                     }
+                    cdd[z] = dd;
+                    cs[z] = s;
+                    cn[z] = e - s;
                 }
-                const int len = e - s;
-                const int ex = wave_excl_scan(len, ln);
+            }
+        }
+        int ncells = 0;  // uniform
+        auto list_cells = [&](double lo2, double hi2) -> int {
+            // the non-empty cells with lo2 < (nearest distance)^2 <= hi2, in
+            // cube order, into cstart/cpre (first particle, number of the
+            // first candidate) and ncells; returns their particle count
+            // (uniform)
+            int C = 0, nc = 0;
+#pragma unroll
+            for (int z = 0; z < 2; ++z) {
+                if (z * kWave >= ncube)
+                    break;
+                const int len = cdd[z] > lo2 && cdd[z] <= hi2 ? cn[z] : 0;
+                const int in = wave_incl_scan(len);
                 const uint64_t bne = __ballot(len > 0);
                 if (len > 0) {
                     const int at = nc + (int)__popcll(bne & below);
-                    cstart[at] = s;
-                    cpre[at] = C + ex;
+                    cstart[at] = cs[z];
+                    cpre[at] = C + in - len;
                 }
                 nc += (int)__popcll(bne);
-                C += __shfl(ex + len, kWave - 1, kWave);
+                C += __builtin_amdgcn_readlane(in, kWave - 1);
             }
             ncells = nc;
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -540,21 +593,22 @@ __global__ __launch_bounds__(kMdWaves * kWave, 4) void k_md_knn(
             // candidate u lies in the last cell c with cpre[c] <= u.  Of a
             // chunk of 64 candidates from u0, the cells after cp (the cell
             // of u0 - 1) that start in it are the next ones in the list:
-            // their starts are flagged (in the histogram's first 64 ints,
-            // free here), and a lane's cell is cp plus the flags at or
-            // below its position
+            // their starts are flagged (in the 64 entries of jb that the
+            // chunk may fill afterwards), and a lane's cell is cp plus the
+            // flags at or below its position
             int cp = -1;  // uniform
             for (int u0 = 0; u0 < C; u0 += kWave) {
-                hist[ln] = 0;
+                int *start = jb + cnt;
+                start[ln] = 0;
                 __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
                 const int ci = cp + 1 + ln;
                 if (ci < ncells) {
                     const int st = cpre[ci] - u0;  // >= 0
                     if (st < kWave)
-                        hist[st] = 1;
+                        start[st] = 1;
                 }
                 __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                const uint64_t bf = __ballot(hist[ln] != 0);
+                const uint64_t bf = __ballot(start[ln] != 0);
                 const int u = u0 + ln;
                 const bool valid = u < C;
                 double d = 0.0;
@@ -565,7 +619,7 @@ __global__ __launch_bounds__(kMdWaves * kWave, 4) void k_md_knn(
                     d = md_dist2(me, S[j], g);
                 }
                 cp += (int)__popcll(bf);
-                md_offer(valid, d, j, T, cnt, buf, jb, hist, k1, ln, below);
+                md_offer(valid, d, j, T, cnt, buf, jb, k1, ln, below);
             }
             // the next pass rewrites cstart/cpre
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -580,13 +634,13 @@ __global__ __launch_bounds__(kMdWaves * kWave, 4) void k_md_knn(
                 lo2 = inner2;
                 hi2 = T1m * T1m;
             }
-            offer_cells(gather_cells(lo2, hi2));
+            offer_cells(list_cells(lo2, hi2));
             // after the inner cells a bound T1 <= T0 of the k-th (at least
             // k entries are within it); at the end the exact k-th, with
             // every particle nearer than it in the buffer, each once
             if (cnt >= k1)
-                T = pass == 0 ? md_select<false>(buf, cnt, k1, hist, ln)
-                              : md_select<true>(buf, cnt, k1, hist, ln);
+                T = pass == 0 ? md_select<false>(buf, cnt, k1, T, ln)
+                              : md_select<true>(buf, cnt, k1, T, ln);
         }
         // 4. mass_density.jl:70-86: kernel sum over the neighbours, bias correction
         const double h = sqrt(T), h_inv = 1.0 / h;
@@ -619,7 +673,12 @@ __global__ __launch_bounds__(kMdWaves * kWave, 4) void k_md_knn(
 // ---------------------------------------------------------------------------
 int64_t md_prep_blocks(int64_t n) { return (n + 255) / 256; }
 
-int md_max_neighbours() { return kMdCap - 2 * kWave - 1; }
+
+int md_max_neighbours()
+{
+    static_assert(471 + 1 <= kMdCap - kWave, "k entries and a chunk of candidates fit");
+    return 471;
+}
 
 int md_bits() { return kMdBits; }
 
@@ -660,10 +719,10 @@ void launch_md_knn(int kernel, const double4 *S, const uint64_t *SK, const int32
                    const int32_t *tab, int lt, int64_t n, const MdGrid &g, int k1, int dim,
                    int nneigh, double norm, double *rho, double *hsml, hipStream_t s)
 {
-    int64_t blocks = (n + kMdWaves - 1) / kMdWaves;
+    int64_t blocks = n;
     if (blocks > (1 << 18))
         blocks = 1 << 18;
-    const dim3 grid((unsigned)blocks), blk(kMdWaves * kWave);
+    const dim3 grid((unsigned)blocks), blk(kWave);
 #define S2G_MD_CASE(KK)                                                                      \
     hipLaunchKernelGGL(k_md_knn<KK>, grid, blk, 0, s, S, SK, order, tab, lt, n, g, k1, dim, \
                        nneigh, norm, rho, hsml)

@@ -122,3 +122,24 @@ def test_errors(s2g):
     with pytest.raises(_lib.LibraryError) as e:
         s2g.mass_density(bad, m, Nneighbors=4)
     assert e.value.code == _lib.S2G_EINVAL
+
+
+@pytest.mark.parametrize("n,k", [(3, 1), (70, 63), (200, 190), (700, 191), (900, 383), (500, 471),
+                                 (9000, 40)])
+@pytest.mark.parametrize("kind", ["random", "lattice", "binades"])
+def test_select_sizes(s2g, orc, n, k, kind):
+    """The k-th smallest distance over the register counts of the select (3, 6
+    and 10 a lane), the largest k near both ends of the key order, more
+    particles than one round of the XCDs' runs, and distances that tie in all,
+    some or none of their bits or span many binades."""
+    r = np.random.default_rng(n + k)
+    if kind == "lattice":
+        L = int(np.ceil(n ** (1 / 3)))
+        pos = np.stack(np.meshgrid(*[np.arange(L) + 0.5] * 3, indexing="ij")).reshape(3, -1)[:, :n]
+    elif kind == "binades":
+        v = r.standard_normal((3, n))
+        pos = v / np.linalg.norm(v, axis=0) * 2.0 ** r.uniform(-12, 0, n)
+    else:
+        pos = r.random((3, n)) * 4.0
+    _check(s2g, orc, np.ascontiguousarray(pos), r.uniform(0.5, 2.0, n), s2g.WendlandC4(3),
+           "wendlandc4", k, (8.0, 8.0, 8.0) if kind == "random" else None)
