@@ -135,6 +135,13 @@ __global__ __launch_bounds__(kPartBlock) void k3d_setup(
 // overlap as an FP64 factor), so the sum and the deposited weights agree.
 // ---------------------------------------------------------------------------
 
+// Voxels farther than this beyond h are not visited by the norm and the gather:
+// they have u >= 1 and weight 0.  It covers the FP32 rounding of the tests (a
+// centre at 2^11 voxels is off by 1e-4, a radius by 1e-7 of itself).  A margin
+// of one voxel, 1.4 times the volume at h = 8, measured 13.4 ms in the norm
+// and 57 ms in the gather of the 2^24 cluster set at 256^3, against 10.9 and
+// 52.1 ms.
+constexpr float kMargin3 = 1.0f / 16.0f;
 constexpr int kNX3 = 128;  // x terms tabulated per pass (per wave, in LDS)
 
 struct NRow3 {
@@ -176,8 +183,8 @@ __device__ __forceinline__ float wave_max_nonneg(float x)
 
 // This lane's share of the sum over the box [ia, ib] x [ja, jb] x [ka, kb]
 // (any integers; voxels outside the grid follow the same formulas).  Only
-// voxels within h + 1 voxel of the centre are visited (the others have
-// u >= 1 in FP32 too, and weight 0); a fallback footprint keeps its whole
+// voxels within h + kMargin3 of the centre are visited (the others have
+// u >= 1 and weight 0); a fallback footprint keeps its whole
 // box.  Per 64 rows j the (j, k) pairs inside that ball's section are listed
 // (per-row k ranges, wave prefix sum) and taken 64 at a time, a pair per
 // lane; each 64 pairs run over the x range of their union, with the x terms
@@ -188,7 +195,7 @@ __device__ __forceinline__ double norm_box3(const Rec3 &r, double hinv, int ia, 
                                             NRow3 *rows)
 {
     const float xc = (float)r.x, yc = (float)r.y, zc = (float)r.z;
-    const float hr = (float)r.h + 1.0f;
+    const float hr = (float)r.h + kMargin3;
     const bool all = r.fb != 0;
     double acc = 0.0;
     for (int xa = ia; xa <= ib; xa += kNX3) {
@@ -209,8 +216,8 @@ __device__ __forceinline__ double norm_box3(const Rec3 &r, double hinv, int ia, 
                     const float dy = fabsf((float)j + 0.5f - yc);
                     if (dy < hr) {
                         const float wz = sqrtf(hr * hr - dy * dy);
-                        const int a = (int)floorf(zc - 0.5f - wz);
-                        const int c = (int)ceilf(zc - 0.5f + wz);
+                        const int a = (int)ceilf(zc - 0.5f - wz);
+                        const int c = (int)floorf(zc - 0.5f + wz);
                         lo = a > lo ? a : lo;
                         hi = c < hi ? c : hi;
                     } else {
@@ -257,8 +264,8 @@ __device__ __forceinline__ double norm_box3(const Rec3 &r, double hinv, int ia, 
                 int ra = xa, rb = xb;
                 if (!all) {
                     const float wm = wave_max_nonneg(wx);
-                    const int a = (int)floorf(xc - 0.5f - wm);
-                    const int c = (int)ceilf(xc - 0.5f + wm);
+                    const int a = (int)ceilf(xc - 0.5f - wm);
+                    const int c = (int)floorf(xc - 0.5f + wm);
                     ra = a > ra ? a : ra;
                     rb = c < rb ? c : rb;
                 }
@@ -361,18 +368,22 @@ __global__ __launch_bounds__(256) void k3d_norm(const int32_t *__restrict__ list
 // 4 bj + ((l >> 2) & 3), 4w + (l & 3)) of sub-brick m.  Per batch of
 // particles the block tabulates per axis the 16 offset terms (offset / h)^2
 // and overlaps, and one bit per sub-brick that can reach the kernel sphere
-// (voxel-centre box within h + 1 voxel of the centre, inside the footprint
-// box); a wave evaluates only its sub-bricks with that bit set.  The x
+// (voxel-centre box within h + kMargin3 of the centre, inside the footprint
+// box); a wave evaluates only its sub-bricks with that bit set, two whose
+// bits are both set side by side.  The x
 // overlap enters shape_row as ax^(1/n), the y overlap multiplies the FP32
 // weight and the z overlap (fixed per lane) folds into the FP64 plane
 // multipliers: one instruction per voxel more than the 2D gather's per
 // pixel, and a per-particle set-up of one FP64 multiplier per plane.
 // ---------------------------------------------------------------------------
-constexpr int kGBatch3 = 32;
-// sub-bricks per uniform test (1, 2 or 4: one bi per test; 4 was slower on
-// the 2^24 cluster set at 256^3, 64.3 -> 69.6 ms, more sub-bricks outside
-// the footprint evaluated)
-constexpr int kG3 = 2;
+// Issue takes three quarters of the time, the rest are waits: the chain of a
+// sub-brick, which four waves per SIMD (64 accumulator registers) do not
+// cover, and the barriers, so batches are as long as the four blocks of a CU
+// have LDS for and the records of two are read at once.  Cluster set at 256^3,
+// two planes: tests of pairs, batches of 32: 52.1 ms; pairs picked by masks:
+// 51.6; batches of 64: 48.9; records of 128: 47.3.  All four x terms read
+// ahead: 54.0 (against 51.6).
+constexpr int kGBatch3 = 64, kGStage3 = 2 * kGBatch3;  // 64: one particle a lane
 
 template <typename T, int K, int NP>
 __global__ __launch_bounds__(256, 4) void k3d_gather(const int4 *__restrict__ items,
@@ -388,11 +399,12 @@ __global__ __launch_bounds__(256, 4) void k3d_gather(const int4 *__restrict__ it
         return;  // the whole block
     __shared__ float2 s_tab[3][kGBatch3][kBT];
     __shared__ uint32_t s_hit[kGBatch3][2];
-    __shared__ double s_c[kGBatch3][3], s_h[kGBatch3];
-    __shared__ double s_hinvd[kGBatch3];
-    __shared__ float s_dd[kGBatch3][3][4];  // per axis: squared sub-brick distance
-    __shared__ float s_rr[kGBatch3];        // (h + 1)^2
-    __shared__ double s_mult[NP][kGBatch3];
+    // the records of two batches
+    __shared__ double s_c[kGStage3][3], s_h[kGStage3];
+    __shared__ double s_hinvd[kGStage3];
+    __shared__ float s_dd[kGStage3][3][4];  // per axis: squared sub-brick distance
+    __shared__ float s_rr[kGStage3];        // (h + margin)^2
+    __shared__ double s_mult[NP][kGStage3];
 
     const int4 it = items[blockIdx.x];
     const int t = it.x;
@@ -412,7 +424,8 @@ __global__ __launch_bounds__(256, 4) void k3d_gather(const int4 *__restrict__ it
 
     for (int base = 0; base < it.z; base += kGBatch3) {
         const int cnt = it.z - base < kGBatch3 ? it.z - base : kGBatch3;
-        if (threadIdx.x < cnt) {
+        const int sb = base % kGStage3;  // the batch in the staged records
+        if (sb == 0 && (int)threadIdx.x < kGStage3 && (int)threadIdx.x < it.z - base) {
             const int p = pairs[it.y + base + threadIdx.x];
             const Rec3 r = rec[p];
             s_c[threadIdx.x][0] = r.x;
@@ -423,8 +436,7 @@ __global__ __launch_bounds__(256, 4) void k3d_gather(const int4 *__restrict__ it
             // sub-brick test terms: per axis and sub-brick the squared
             // distance from the centre to its voxel centres, infinite
             // outside the footprint box (0 inside it for a fallback
-            // footprint, which keeps its whole box); one voxel of margin on
-            // h, so FP32 rounding cannot drop a voxel with u < 1
+            // footprint, which keeps its whole box)
             const int lo[3] = {r.i0 - b0[0], r.j0 - b0[1], r.k0 - b0[2]};
             const int hi[3] = {r.i1 - b0[0], r.j1 - b0[1], r.k1 - b0[2]};
             const double cc[3] = {r.x, r.y, r.z};
@@ -439,7 +451,7 @@ __global__ __launch_bounds__(256, 4) void k3d_gather(const int4 *__restrict__ it
                     s_dd[threadIdx.x][ax][sb] = !inbox ? __builtin_inff() : r.fb ? 0.0f : dd * dd;
                 }
             }
-            const float rr = (float)r.h + 1.0f;
+            const float rr = (float)r.h + kMargin3;
             s_rr[threadIdx.x] = rr * rr;
 #pragma unroll
             for (int q = 0; q < NP; ++q) {
@@ -449,7 +461,8 @@ __global__ __launch_bounds__(256, 4) void k3d_gather(const int4 *__restrict__ it
                 s_mult[q][threadIdx.x] = mult * r.s;
             }
         }
-        __syncthreads();
+        if (sb == 0)
+            __syncthreads();
         // per axis the 16 terms ((offset / h)^2, overlap); offset / h in FP64,
         // rounded once; the x overlap as its n-th root.  One axis per wave.
         for (int e = threadIdx.x; e < 3 * kGBatch3 * kBT; e += 256) {
@@ -457,27 +470,30 @@ __global__ __launch_bounds__(256, 4) void k3d_gather(const int4 *__restrict__ it
             if (b >= cnt)
                 continue;
             const double f = (double)(b0[ax] + v);
-            const double c = s_c[b][ax];
-            const float os = (float)(coff1(c, f) * s_hinvd[b]);
-            const float ov = fmaxf((float)overlap1(c, s_h[b], f), 0.0f);
+            const double c = s_c[sb + b][ax];
+            const float os = (float)(coff1(c, f) * s_hinvd[sb + b]);
+            const float ov = fmaxf((float)overlap1(c, s_h[sb + b], f), 0.0f);
             s_tab[ax][b][v] = make_float2(os * os, ax == 0 ? overlap_root<K>(ov) : ov);
         }
         // sub-brick bits: lane = 16 bk + 4 bi + bj
         const int sbx = (ln >> 2) & 3, sby = ln & 3, sbz = ln >> 4;
         for (int b = wv; b < cnt; b += 4) {
-            const float d2 = s_dd[b][0][sbx] + s_dd[b][1][sby] + s_dd[b][2][sbz];
-            const uint64_t bits = __ballot(d2 < s_rr[b]);
+            const float d2 = s_dd[sb + b][0][sbx] + s_dd[sb + b][1][sby] + s_dd[sb + b][2][sbz];
+            const uint64_t bits = __ballot(d2 < s_rr[sb + b]);
             if (ln == 0) {
                 s_hit[b][0] = (uint32_t)bits;
                 s_hit[b][1] = (uint32_t)(bits >> 32);
             }
         }
         __syncthreads();
-        for (int b = 0; b < cnt; ++b) {
-            const uint32_t word = __builtin_amdgcn_readfirstlane(s_hit[b][wv >> 1]);
-            const uint32_t wm = (word >> (16 * (wv & 1))) & 0xffffu;
-            if (wm == 0)
-                continue;
+        // this wave's sub-bricks of particle lane b; the particles with any are
+        // taken in order
+        const int mk = ln < cnt ? (int)((s_hit[ln][wv >> 1] >> (16 * (wv & 1))) & 0xffffu) : 0;
+        uint64_t live = __ballot(mk != 0);
+        while (live) {
+            const int b = __builtin_ctzll(live);
+            live &= live - 1;
+            const int wm = __builtin_amdgcn_readlane(mk, b);
             const float2 zt = s_tab[2][b][4 * wv + dk];
             const double az = (double)zt.y;
             // the z overlap is common to the lane's voxels: fold it into the
@@ -487,35 +503,46 @@ __global__ __launch_bounds__(256, 4) void k3d_gather(const int4 *__restrict__ it
             double mult[NP];
 #pragma unroll
             for (int q = 0; q < NP; ++q)
-                mult[q] = s_mult[q][b] * az;
+                mult[q] = s_mult[q][sb + b] * az;
             float yz[4], ay[4];
 #pragma unroll
             for (int bj = 0; bj < 4; ++bj) {
-                if (!(wm & (((1u << kG3) - 1u) * 0x1111u << (bj / kG3 * kG3))))
+                if (!(wm & (0x3333 << (bj & 2))))
                     continue;
                 const float2 yt = s_tab[1][b][4 * bj + dj];
                 yz[bj] = yt.x + zt.x;
                 ay[bj] = yt.y;
             }
+            // pairs of sub-bricks (bj, bj + 1) that are both reached (bit of
+            // the first) run side by side, so that their dependency chains
+            // overlap; then the ones reached alone
+            int both = wm & (wm >> 1) & 0x5555;
+            int one = wm & ~(both * 3);
+            asm("" : "+s"(both), "+s"(one));  // keep the tests below apart
+            auto weight = [&](float2 xt, int m) {
+                const int bj = m & 3;
+                return (double)(shape_row<K>(__builtin_amdgcn_sqrtf(xt.x + yz[bj]), xt.y) *
+                                ay[bj]);
+            };
 #pragma unroll
-            for (int m = 0; m < 16; m += kG3) {
-                if (!((wm >> m) & ((1u << kG3) - 1u)))
-                    continue;
-                // the kG3 sub-bricks of one test share bi
-                const float2 xt = s_tab[0][b][4 * (m >> 2) + di];
-                float wk[kG3];
+            for (int m = 0; m < 16; m += 2) {
+                if (both & (1 << m)) {
+                    const float2 xt = s_tab[0][b][4 * (m >> 2) + di];
+                    const double f0 = weight(xt, m), f1 = weight(xt, m + 1);
 #pragma unroll
-                for (int g = 0; g < kG3; ++g) {
-                    const int bj = (m + g) & 3;
-                    wk[g] = shape_row<K>(__builtin_amdgcn_sqrtf(xt.x + yz[bj]), xt.y) * ay[bj];
+                    for (int q = 0; q < NP; ++q) {
+                        acc[m][q] = fma(f0, mult[q], acc[m][q]);
+                        acc[m + 1][q] = fma(f1, mult[q], acc[m + 1][q]);
+                    }
                 }
 #pragma unroll
-                for (int g = 0; g < kG3; ++g) {
-                    const double f = (double)wk[g];
+                for (int d = 0; d < 2; ++d)
+                    if (one & (1 << (m + d))) {
+                        const double f = weight(s_tab[0][b][4 * (m >> 2) + di], m + d);
 #pragma unroll
-                    for (int q = 0; q < NP; ++q)
-                        acc[m + g][q] = fma(f, mult[q], acc[m + g][q]);
-                }
+                        for (int q = 0; q < NP; ++q)
+                            acc[m + d][q] = fma(f, mult[q], acc[m + d][q]);
+                    }
             }
         }
         __syncthreads();

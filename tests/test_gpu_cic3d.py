@@ -142,6 +142,35 @@ def test_small_window_scatter(s2g, orc, kernel, npix, n):
         assert rel_l1(gpu[:, k], ref[:, k]) <= 1e-12, k
 
 
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 128, 129, 300])
+@pytest.mark.parametrize("kernel,hpix", [("cubic", 4.7), ("wendlandc6", 13.2)])
+def test_gather_batches_and_reach(s2g, orc, kernel, hpix, n):
+    """Work items of one and several gather batches (64) and record stages
+    (128), and the voxels next to the kernel sphere: an offset from a voxel
+    centre puts voxels at u just below 1, which neither the gather's
+    sub-brick tests nor the norm's sections may leave out.  A voxel at u <
+    0.98 has a weight above 1e-12 of the peak for both kernels."""
+    npix = 48
+    r = np.random.default_rng(n)
+    x = (np.floor(r.uniform(-6.0, 6.0, (n, 3))) + 0.5 + 1e-3) / npix
+    h = np.full(n, hpix / npix) * r.uniform(0.99, 1.01, n)
+    m, rho, w, q = (r.uniform(0.5, 2.0, n) for _ in range(4))
+    st = {}
+    gpu = s2g.deposit(x, h, m, rho, q, w, npix=npix, len2pix=float(npix), dimensions=3,
+                      kernel=_kernel(s2g, kernel), calc_mean=False, stats=st)
+    assert st["n_large"] == n
+    ref = orc.cic_mapping_3D(x, h, m, rho, q, w, npix, float(npix), kernel, 3, False)
+    _check(gpu, ref, f"batches {kernel} {n}")
+    c = np.arange(npix) + 0.5 - npix / 2
+    X, Y, Z = np.meshgrid(c, c, c, indexing="ij")
+    near = np.zeros((npix,) * 3, bool)
+    for p in range(n):
+        d2 = ((np.stack([X, Y, Z], -1) - x[p] * npix) ** 2).sum(-1)
+        near |= d2 < (0.98 * h[p] * npix) ** 2
+    got = gpu[:, 1].reshape((npix,) * 3)
+    assert (got[near] > 0).all() and ((ref[:, 1].reshape(got.shape) > 0) >= (got > 0)).all()
+
+
 def test_large_only_is_deterministic(s2g):
     npix, n = 48, 150
     x, h, m, rho, q, w = _particles(n, npix, 8, hmin=4.0, hmax=12.0)
