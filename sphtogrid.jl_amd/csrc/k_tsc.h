@@ -18,15 +18,17 @@ int64_t tsc_nbricks(int64_t npix);
 // bits [tsc_key_begin_bit(), tsc_key_bits(npix))
 int tsc_key_begin_bit();
 int tsc_key_bits(int64_t npix);
-void launch_tsc_keys(int dtype, const void *pos, int64_t n, int64_t npix, double len2pix,
-                     int periodic, uint32_t *keys, int32_t *vals, hipStream_t s);
+// rec: null, or n records (grid coordinates, quantity) for launch_tsc_prep
+void launch_tsc_keys(int dtype, const void *pos, const void *binq, int64_t n, int64_t npix,
+                     double len2pix, int periodic, uint32_t *keys, int32_t *vals, double4 *rec,
+                     hipStream_t s);
 // off[b] = first sorted particle of brick b, b in [0, nbricks] (off[nbricks] =
 // the particles that are not dropped)
 void launch_tsc_offsets(const uint32_t *sorted_keys, int64_t n, int64_t npix, int64_t *off,
                         hipStream_t s);
 // sorted grid coordinates + quantity and packed nearest cells
-void launch_tsc_prep(int dtype, const void *pos, const void *binq, const int32_t *order,
-                     const int64_t *off, int64_t n, int64_t npix, double len2pix, int periodic,
+void launch_tsc_prep(int dtype, const void *pos, const void *binq, const double4 *rec,
+                     const int32_t *order, const int64_t *off, int64_t n, int64_t npix, double len2pix, int periodic,
                      double4 *gq, uint64_t *cell, hipStream_t s);
 // every cell of both planes (grid: 2 x npix^3 doubles)
 void launch_tsc_gather(const double4 *gq, const uint64_t *cell, const uint32_t *sorted_keys,

@@ -2357,14 +2357,25 @@ static void check_tsc(int dtype, int64_t n, const s2g_params *params)
 static void tsc_run(int dtype, const void *d_pos, const void *d_q, int64_t n, int64_t npix,
              double len2pix, int periodic, const TscWork &w, double *d_grid, hipStream_t s)
 {
+    // The particles' records in input order, for the prep's random reads, lie
+    // in the grid until the gather overwrites all of it: where they fit (at
+    // most one particle per two cells), are aligned, and the grid is apart
+    // from the inputs, which the same kernel reads.
+    const uintptr_t g0 = (uintptr_t)d_grid, g1 = g0 + 16 * (uintptr_t)(npix * npix * npix);
+    const auto apart = [&](const void *p, int64_t m) {
+        return (uintptr_t)p + elem_size(dtype) * (uintptr_t)m <= g0 || (uintptr_t)p >= g1;
+    };
+    const bool fits = 2 * n <= npix * npix * npix && g0 % alignof(double4) == 0 &&
+                      apart(d_pos, 3 * n) && apart(d_q, n);
+    double4 *rec = fits ? (double4 *)d_grid : nullptr;
     if (n > 0) {
-        launch_tsc_keys(dtype, d_pos, n, npix, len2pix, periodic, w.keys, w.vals, s);
+        launch_tsc_keys(dtype, d_pos, d_q, n, npix, len2pix, periodic, w.keys, w.vals, rec, s);
         sort_pairs(w.sort_tmp, w.sort_bytes, w.keys, w.keys + n, w.vals, w.vals + n, n,
                    tsc_key_bits(npix), s, tsc_key_begin_bit());
     }
     // n == 0: every offset is 0 (no key is read)
     launch_tsc_offsets(w.keys + n, n, npix, w.off, s);
-    launch_tsc_prep(dtype, d_pos, d_q, w.vals + n, w.off, n, npix, len2pix, periodic, w.gq,
+    launch_tsc_prep(dtype, d_pos, d_q, rec, w.vals + n, w.off, n, npix, len2pix, periodic, w.gq,
                     w.cell, s);
     launch_tsc_gather(w.gq, w.cell, w.keys + n, w.off, npix, periodic, d_grid, s);
 }

@@ -108,3 +108,32 @@ def test_tsc_brick_edges(s2g, orc, N, periodic):
     ref = orc.tsc_3d(pos, q, N, float(N), periodic)
     # n weights of order one per cell at most: 3000 roundings of 1.1e-16
     np.testing.assert_allclose(got, ref, rtol=1e-12, atol=1e-12)
+
+
+@pytest.mark.parametrize("periodic", [False, True])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [1, 2047, 2048, 2049])
+def test_records_in_the_grid(s2g, n, dtype, periodic):
+    """A 16^3 grid holds the records of up to 2048 particles until it is
+    written; a grid that is not aligned for them, and more particles, take
+    the inputs directly: the same grid bit for bit."""
+    import torch
+    from sph2grid import _lib
+    N, ctx = 16, s2g.default_context()
+    r = np.random.default_rng(n)
+    pos, q = r.uniform(-0.7, 0.7, (n, 3)), r.uniform(-1, 3, n)
+    pos[: n // 9, 1] = np.nan
+    x, qq = (torch.tensor(a.astype(dtype), device="cuda") for a in (pos, q))
+    par = _lib.Params(npixels=N, len2pix=float(N))
+    out = []
+    for shift in (0, 1):
+        g = torch.full((2 * N ** 3 + 4,), np.nan, dtype=torch.float64, device="cuda")[shift:]
+        torch.cuda.synchronize()
+        rc = ctx.lib.s2g_tsc3d_device(
+            ctx.handle, _lib.S2G_F32 if dtype == np.float32 else _lib.S2G_F64,
+            C.c_void_p(x.data_ptr()), C.c_void_p(qq.data_ptr()), n, C.byref(par),
+            _lib.S2G_FLAG_PERIODIC if periodic else 0, C.c_void_p(g.data_ptr()), None)
+        ctx.check(rc, "s2g_tsc3d_device")
+        torch.cuda.synchronize()
+        out.append(g[: 2 * N ** 3].cpu().numpy())
+    assert np.isfinite(out[0]).all() and np.array_equal(out[0], out[1])
