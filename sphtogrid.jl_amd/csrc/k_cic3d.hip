@@ -107,23 +107,46 @@ __device__ __forceinline__ Rec3 setup3d(const T *__restrict__ pos, const T *__re
     return r;
 }
 
-// counts: the partition's per-block class counts
+// counts: the partition's per-block class counts.  box (or null): of every
+// `stride`-th block the small particles: Small3Sample.
 template <typename T>
 __global__ __launch_bounds__(kPartBlock) void k3d_setup(
     const T *__restrict__ pos, const T *__restrict__ hsml, const T *__restrict__ m,
     const T *__restrict__ rho, const T *__restrict__ binq, const T *__restrict__ w, int64_t n,
     int64_t npix, double len2pix, int kernel, uint32_t flags, Rec3 *__restrict__ rec,
-    int32_t *__restrict__ cls, int64_t *__restrict__ counts)
+    int32_t *__restrict__ cls, int64_t *__restrict__ counts, Small3Sample *__restrict__ box,
+    int stride)
 {
+    __shared__ int s_box[4];
     const int64_t p = (int64_t)blockIdx.x * kPartBlock + threadIdx.x;
-    int c = kClsSkip;
+    int c = kClsSkip, vox = 0, tile = -1;
     if (p < n) {
         const Rec3 r = setup3d(pos, hsml, m, rho, binq, w, npix, len2pix, kernel, flags, p);
         rec[p] = r;
         c = r.cls;
         cls[p] = c;
+        if (c == kClsSmall) {
+            vox = (r.i1 - r.i0 + 1) * (r.j1 - r.j0 + 1) * (r.k1 - r.k0 + 1);
+            tile = (r.i0 / kST3) << 20 | (r.j0 / kST3) << 10 | r.k0 / kST3;
+        }
     }
-    block_class_counts(c, counts);
+    if (threadIdx.x < 4)
+        s_box[threadIdx.x] = 0;
+    block_class_counts(c, counts);  // holds a barrier
+    if (!box || blockIdx.x % stride)
+        return;  // the whole block
+    const int other = __shfl_xor(tile, 32, kWave);
+    if (vox) {
+        atomicAdd(&s_box[0], vox);
+        atomicAdd(&s_box[1], 1);
+        if (other >= 0)
+            atomicAdd(&s_box[2], 1);
+        if (other == tile)
+            atomicAdd(&s_box[3], 1);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0)
+        box[blockIdx.x / stride] = Small3Sample{s_box[0], s_box[1], s_box[2], s_box[3]};
 }
 
 
@@ -723,8 +746,8 @@ __global__ __launch_bounds__(256) void k3d_small_flat(const int32_t *__restrict_
 }
 
 
-// Windowed small scatter, for grids with enough small particles per tile
-// (small3_windowed).  Particles are sorted by the kST3^3 tile that holds their
+// Windowed small scatter, for grids with enough small particles per tile and
+// voxels per particle (small3_windowed).  Particles are sorted by the kST3^3 tile that holds their
 // box's first voxel; a block takes a work item of one tile, accumulates it in
 // an LDS window (the tile and the largest box, both planes) with ds_add_f64
 // and adds the window to the image once, so the global FP64 atomics that
@@ -932,7 +955,8 @@ __global__ void k3d_reduce(const double *__restrict__ image, int64_t nd, int red
     default: { constexpr int KK = S2G_KERNEL_WENDLAND_C8; CALL; } break;       \
     }
 
-void launch_3d_setup(const Map3DArgs &a, Rec3 *rec, int32_t *cls, int64_t *counts, hipStream_t s)
+void launch_3d_setup(const Map3DArgs &a, Rec3 *rec, int32_t *cls, int64_t *counts,
+                     Small3Sample *box, int stride, hipStream_t s)
 {
     if (a.n == 0)
         return;
@@ -941,12 +965,12 @@ void launch_3d_setup(const Map3DArgs &a, Rec3 *rec, int32_t *cls, int64_t *count
         hipLaunchKernelGGL(k3d_setup<float>, g, blk, 0, s, (const float *)a.pos,
                            (const float *)a.hsml, (const float *)a.m, (const float *)a.rho,
                            (const float *)a.binq, (const float *)a.w, a.n, a.npix, a.len2pix,
-                           a.kernel, a.flags, rec, cls, counts);
+                           a.kernel, a.flags, rec, cls, counts, box, stride);
     else
         hipLaunchKernelGGL(k3d_setup<double>, g, blk, 0, s, (const double *)a.pos,
                            (const double *)a.hsml, (const double *)a.m, (const double *)a.rho,
                            (const double *)a.binq, (const double *)a.w, a.n, a.npix,
-                           a.len2pix, a.kernel, a.flags, rec, cls, counts);
+                           a.len2pix, a.kernel, a.flags, rec, cls, counts, box, stride);
 }
 
 void launch_3d_norm(int kernel, const int32_t *list, int64_t ne, int64_t npix, uint32_t flags,

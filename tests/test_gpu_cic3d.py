@@ -142,6 +142,30 @@ def test_small_window_scatter(s2g, orc, kernel, npix, n):
         assert rel_l1(gpu[:, k], ref[:, k]) <= 1e-12, k
 
 
+@pytest.mark.parametrize("npix,n,hpix,clump", [
+    (18, 3000, 0.4, 1.0),     # many per tile, few voxels each
+    (18, 3000, 3.4, 1.0),
+    (27, 300000, 0.4, 1.0),   # more than the light lists take
+    (27, 300000, 2.0, 1.0),
+    (48, 300000, 0.5, 0.05),  # few cells hold most
+])
+def test_small_scatter_rule(s2g, orc, npix, n, hpix, clump):
+    """Dense small footprints on either side of the rule between the flat and
+    the windowed scatter.  FP64 throughout: as test_small_window_scatter, with
+    up to 3e5 sums of one sign in a voxel, 3e5 * 1.1e-16 < 1e-10."""
+    r = np.random.default_rng(n + npix)
+    x = clump * r.uniform(-0.5, 0.5, (n, 3))
+    h = hpix / npix * r.uniform(0.9, 1.0, n)
+    m, rho, w, q = (r.uniform(0.5, 2.0, n) for _ in range(4))
+    st = {}
+    gpu = s2g.deposit(x, h, m, rho, q, w, npix=npix, len2pix=float(npix), dimensions=3,
+                      kernel=s2g.WendlandC6(3), calc_mean=False, stats=st)
+    assert st["n_small"] == n
+    ref = orc.cic_mapping_3D(x, h, m, rho, q, w, npix, float(npix), "wendlandc6", 3, False)
+    for k in range(2):
+        assert rel_l1(gpu[:, k], ref[:, k]) <= 1e-10, k
+
+
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 128, 129, 300])
 @pytest.mark.parametrize("kernel,hpix", [("cubic", 4.7), ("wendlandc6", 13.2)])
 def test_gather_batches_and_reach(s2g, orc, kernel, hpix, n):
