@@ -1,12 +1,13 @@
 // k_cic2d.hip -- the 2D Smac pixel-overlap deposit (cic_interpolation/cic_2D.jl)
 // on gfx950.
 //
-// Pipeline of one pass (all on one stream).  A pass deposits one map or a
-// batch of maps; the maps' particles and tiles are concatenated and every
-// stage reads the per-map table (Map2D) where it needs map data.
+// Pipeline of one pass (the normalisation and the small footprints beside the
+// lists and the gather, on the context's side streams).  A pass deposits one
+// map or a batch of maps; the maps' particles and tiles are concatenated and
+// every stage reads the per-map table (Map2D) where it needs map data.
 //   k2d_setup        per particle, FP64: pixel coordinates, integer footprint,
 //                    zero-quantity skip, fallback decision, class
-//   k2d_partition    stable (particle-order) lists of small / large / exact
+//   k_part_*         stable (particle-order) lists of small / large / exact
 //   k2d_norm         explicit FP64 normalisation sum of large clipped footprints
 //                    (closed form minus the border-cut part when smaller)
 //   k_pair_count     counting sort of (tile, particle) pairs: per-chunk counts
