@@ -150,7 +150,8 @@ typedef struct s2g_tuning {
                                     weights need FP64, in the scatter) */
     int32_t small_item_min;      /* least particles per small-footprint work item;
                                     16..4096, default 256 (half of it in a pass of at
-                                    most 2^18 particles) */
+                                    most 2^18 particles, a quarter where half
+                                    would not give every CU an item) */
     int32_t small_items_per_cu;  /* small-footprint work items per CU aimed at;
                                     1..64, default 16 */
     int32_t gather_item_min;     /* least (tile, particle) pairs per gather work item;

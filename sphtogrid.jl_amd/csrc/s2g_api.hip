@@ -678,8 +678,13 @@ void deposit2d_pass(s2g_ctx *c, const MapIn *mi, int nmaps, hipStream_t s, s2g_s
         int64_t Gs = (ns + starget - 1) / starget;
         // a light pass halves the least item, to spread over the CUs (65,536
         // particles on 256^2: scatter 97 -> 70 us; quartered 78 us, the
-        // windows' own cost)
-        const int64_t smin = lt.ok ? (c->tune.small_item_min + 1) / 2 : c->tune.small_item_min;
+        // windows' own cost), and quarters it where half would not give every
+        // CU one (whole calls, half / quarter: 4,096 particles on 64^2 151 /
+        // 133 us, 8,000 of a blast on 128^2 170 / 136, 30,000 on 128^2 187 / 173)
+        const int64_t half = (c->tune.small_item_min + 1) / 2;
+        const int64_t smin = !lt.ok               ? c->tune.small_item_min
+                             : ns < half * c->ncu ? (half + 1) / 2
+                                                  : half;
         if (Gs < smin)
             Gs = smin;
         const int64_t max_items = nstiles + (ns + Gs - 1) / Gs;

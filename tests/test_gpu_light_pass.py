@@ -65,3 +65,21 @@ def test_light_batch_with_empty_and_one_sided_maps(s2g, nq):
     for d, ref in zip(maps, singles):
         got = d["out"].cpu().numpy().reshape(ref.shape, order="F")
         np.testing.assert_allclose(got, ref, rtol=0, atol=1e-12 * max(np.abs(ref).max(), 1e-300))
+
+
+@pytest.mark.parametrize("n", [63, 64, 65, 1000, 40000])
+def test_small_item_floor(s2g, orc, n):
+    """Small footprints piled on one tile, so that its list is cut into items
+    of a quarter of the least item (few particles) or half of it (40,000).
+    Tolerance: the 2D deposit's (rel-L1 1e-5, conservation 1e-6)."""
+    npix = 64
+    r = np.random.default_rng(n)
+    x = r.uniform(-0.2, 0.0, (n, 3))
+    h = r.uniform(0.5, 6.0, n) / npix
+    m, rho, w, q = (r.uniform(0.5, 2.0, n) for _ in range(4))
+    gpu = s2g.deposit(x, h, m, rho, q, w, npix=npix, len2pix=float(npix), dimensions=2,
+                      kernel=s2g.WendlandC4(2), calc_mean=False)
+    ref = orc.cic_mapping_2D(x, h, m, rho, q, w, npix, float(npix), "wendlandc4", 2, False)
+    for k in range(2):
+        assert np.abs(gpu[:, k] - ref[:, k]).sum() <= 1e-5 * np.abs(ref[:, k]).sum(), k
+    assert abs(gpu[:, 1].sum() / ref[:, 1].sum() - 1) <= 1e-6
