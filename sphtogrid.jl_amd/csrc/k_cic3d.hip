@@ -763,9 +763,6 @@ __global__ __launch_bounds__(256) void k3d_small_flat(const int32_t *__restrict_
 // windowed 4.2 ms.
 constexpr int kS3Waves = 8;
 constexpr int kS3Batch = 8 * kS3Waves;  // eight particles per wave and batch
-// window strides: one voxel of padding against bank conflicts
-constexpr int kSW3 = kST3 + kSmallSide3D - 1;
-constexpr int kSW3y = kSW3 + 1, kSW3x = kSW3 * kSW3y;
 
 template <typename T, int K>
 __global__ __launch_bounds__(kS3Waves *kWave) void k3d_small_window(
@@ -849,13 +846,8 @@ __global__ __launch_bounds__(kS3Waves *kWave) void k3d_small_window(
                     const int4 bs = s_box[es];
                     const int dims = __builtin_amdgcn_readfirstlane(bs.w);
                     const int iws = dims & 0xff, jws = (dims >> 8) & 0xff, kws = dims >> 16;
-                    const int jk = jws * kws;
-                    const float ijk = 1.0f / (float)jk, ikw = 1.0f / (float)kws;
-                    const int ri = (int)(((float)ln + 0.5f) * ijk), rem = ln - ri * jk;
-                    const int dj = (int)(((float)rem + 0.5f) * ikw), dk = rem - dj * kws;
-                    int R = __builtin_amdgcn_readfirstlane((int)(((float)kWave + 0.5f) * ijk));
-                    R = R < kSmallSide3D ? R : kSmallSide3D;
-                    const bool on = ri < R;
+                    const int R = __builtin_amdgcn_readfirstlane(small3_planes(jws * kws));
+                    const Small3Lane l = small3_lane(ln, iws, jws, kws);
                     const double x = s_x[es], y = s_y[es], z = s_z[es], h = s_h[es];
                     const double hinv = s_hinv[es];
                     if (ln < 2 * kSmallSide3D) {
@@ -863,10 +855,11 @@ __global__ __launch_bounds__(kS3Waves *kWave) void k3d_small_window(
                         const double xd = coff1(x, fi);
                         s_xt[wv][ln] = make_double2(xd * xd, ln < iws ? overlap1(x, h, fi) : 0.0);
                     }
-                    const double fj = (double)(bs.y + dj), fk = (double)(bs.z + dk);
+                    const double fj = (double)(bs.y + l.dj), fk = (double)(bs.z + l.dk);
                     const double yd = coff1(y, fj), zd = coff1(z, fk);
-                    const double ayz = on ? overlap1(y, h, fj) * overlap1(z, h, fk) : 0.0;
-                    const double2 *xt = s_xt[wv] + (on ? ri : 0);
+                    const double ayz =
+                        l.left > 0 ? overlap1(y, h, fj) * overlap1(z, h, fk) : 0.0;
+                    const double2 *xt = s_xt[wv] + (l.left > 0 ? l.ri : 0);
                     double wk[kSmallSide3D];
                     double ws = 0.0;
                     __builtin_amdgcn_wave_barrier();
@@ -882,12 +875,13 @@ __global__ __launch_bounds__(kS3Waves *kWave) void k3d_small_window(
                     ws = wave_sum(ws);
                     const double scale = ws != 0.0 ? s_s[es] / ws : 0.0;
                     const double bq = s_bq[es];
-                    int cl = (bs.x - oi + ri) * kSW3x + (bs.y + dj - oj) * kSW3y + (bs.z + dk - ok);
+                    int cl = (bs.x - oi + l.ri) * kSW3x + (bs.y + l.dj - oj) * kSW3y +
+                             (bs.z + l.dk - ok);
 #pragma unroll
                     for (int st = 0; st < kSmallSide3D; ++st)
                         if (st * R < iws) {
                             const double pw = wk[st] * scale;
-                            if (pw != 0.0) {
+                            if (st * R < l.left && pw != 0.0) {
                                 unsafeAtomicAdd(&acc[0][cl], bq * pw);
                                 unsafeAtomicAdd(&acc[1][cl], pw);
                             }

@@ -8,6 +8,7 @@
 #include <string>
 
 #include "../../include/sph2grid.h"
+#include "k_small3.h"
 
 namespace s2g {
 
@@ -32,10 +33,7 @@ constexpr int kST = 32;
 // 2D gather tile: 64 x 64 pixels.
 constexpr int kGT = 64;
 
-// 3D: footprint box side <= 8 voxels goes to the scatter path; bricks of 16^3.
-constexpr int kSmallSide3D = 8;
-// side of the windowed 3D scatter's tiles
-constexpr int kST3 = 9;
+// 3D: bricks of 16^3.
 constexpr int kBT = 16;
 
 // Per-particle record of the 2D deposit, built once per call.
