@@ -815,7 +815,7 @@ __global__ __launch_bounds__(kS3Waves *kWave) void k3d_small_window(
                 const bool tiny = e < cnt && iw <= 2 && jw <= 2 && kw <= 2;
                 uint64_t rest = __ballot(e < cnt && !tiny);
                 double wv3 = 0.0;
-                int cell = 0;
+                int cell = -1;  // in the box: its window cell
                 if (tiny) {
                     const int di = v >> 2, dj = (v >> 1) & 1, dk = v & 1;
                     if (di < iw && dj < jw && dk < kw) {
@@ -834,10 +834,13 @@ __global__ __launch_bounds__(kS3Waves *kWave) void k3d_small_window(
                 double sum = dpp_add<0xB1>(wv3);
                 sum = dpp_add<0x4E>(sum);
                 sum = dpp_add<0x141>(sum);
-                if (wv3 != 0.0) {
-                    const double pw = wv3 * (s_s[e] / sum);
-                    unsafeAtomicAdd(&acc[0][cell], s_bq[e] * pw);
-                    unsafeAtomicAdd(&acc[1][cell], pw);
+                if (cell >= 0) {
+                    // as the flat scatter: nothing where the deposited weight is 0
+                    const double pw = wv3 * (sum != 0.0 ? s_s[e] / sum : 0.0);
+                    if (pw != 0.0) {
+                        unsafeAtomicAdd(&acc[0][cell], s_bq[e] * pw);
+                        unsafeAtomicAdd(&acc[1][cell], pw);
+                    }
                 }
                 while (rest) {
                     const int b = __builtin_ctzll(rest) / 8;

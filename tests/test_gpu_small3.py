@@ -61,3 +61,19 @@ def test_scale_that_is_not_finite(s2g, centre, h, side, bad):
         # two orders of at most 3000 FP64 sums of one sign: 3000 * 1.1e-16
         np.testing.assert_allclose(got[~inside, c], ref[~inside, c], rtol=0,
                                    atol=1e-12 * ref[:, c].max())
+
+
+@pytest.mark.parametrize("q0", [np.inf, -np.inf, np.nan])
+def test_zero_weight_of_a_small_box(s2g, q0):
+    """Particles of weight 0 in boxes of one to eight voxels (eight to a wave)
+    add nothing, whatever their quantity, among large boxes that share their
+    voxels."""
+    p = _set(3000, 12)
+    p[1][::5] = 0.4 / NPIX
+    p[5][::10], p[4][::10] = 0.0, q0
+    got = _deposit(s2g, p)
+    keep = np.arange(3000) % 10 != 0
+    ref = _deposit(s2g, [a[keep] for a in p])
+    for c in range(2):
+        # two orders of at most 3000 FP64 sums of one sign: 3000 * 1.1e-16
+        np.testing.assert_allclose(got[:, c], ref[:, c], rtol=0, atol=1e-12 * ref[:, c].max())
