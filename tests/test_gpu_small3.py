@@ -77,3 +77,21 @@ def test_zero_weight_of_a_small_box(s2g, q0):
     for c in range(2):
         # two orders of at most 3000 FP64 sums of one sign: 3000 * 1.1e-16
         np.testing.assert_allclose(got[:, c], ref[:, c], rtol=0, atol=1e-12 * ref[:, c].max())
+
+
+def test_weights_that_cancel(s2g, orc):
+    """Two particles of equal geometry and opposite weights: their voxels' sum
+    of weights is exactly 0, their sum of quantities is not.  (The rest of the
+    set stays clear of them, so that no other sum rounds theirs.)"""
+    p = _set(3000, 13, 0.0, 8.0)
+    c, h = (14.4, 14.3, 14.6), 2.0
+    for k, w, q in ((700, 1.0, 3.0), (2100, -1.0, 1.0)):
+        p[0][k] = (np.array(c) - 0.5 * NPIX) / NPIX
+        p[1][k], p[2][k], p[3][k], p[4][k], p[5][k] = h / NPIX, 1.0, 1.0, q, w
+    inside, _ = _box(c, h)
+    got = _deposit(s2g, p)
+    ref = orc.cic_mapping_3D(*p, NPIX, float(NPIX), "wendlandc4", 3, False)
+    assert (got[inside, 1] == 0.0).all() and ref[inside, 0].max() > 0.0
+    # FP64 in both, boxes of 125 voxels: a few hundred roundings of 1.1e-16
+    np.testing.assert_allclose(got[inside, 0], ref[inside, 0], rtol=0,
+                               atol=1e-12 * ref[inside, 0].max())
