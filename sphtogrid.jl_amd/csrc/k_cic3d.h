@@ -31,12 +31,6 @@ struct Small3Args {
 };
 
 // counts: the partition's per-block class counts
-// A set-up block's small particles: voxels of their boxes, particles, those
-// whose partner (32 particles on) is small too, and those whose partner starts
-// in the same kST3^3 tile.
-struct Small3Sample {
-    int voxels, n, pairs, same;
-};
 // box: null, or a sample of every stride-th block of partition_blocks(a.n)
 void launch_3d_setup(const Map3DArgs &a, Rec3 *rec, int32_t *cls, int64_t *counts,
                      Small3Sample *box, int stride, hipStream_t s);

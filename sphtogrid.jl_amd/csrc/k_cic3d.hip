@@ -117,7 +117,9 @@ __global__ __launch_bounds__(kPartBlock) void k3d_setup(
     int32_t *__restrict__ cls, int64_t *__restrict__ counts, Small3Sample *__restrict__ box,
     int stride)
 {
-    __shared__ int s_box[4];
+    constexpr int kRun = kPartBlock / kSmall3Tiles;  // threads that give a tile
+    static_assert(kRun == 16, "four runs per wave");
+    __shared__ int s_box[2], s_tile[kSmall3Tiles];
     const int64_t p = (int64_t)blockIdx.x * kPartBlock + threadIdx.x;
     int c = kClsSkip, vox = 0, tile = -1;
     if (p < n) {
@@ -130,23 +132,27 @@ __global__ __launch_bounds__(kPartBlock) void k3d_setup(
             tile = (r.i0 / kST3) << 20 | (r.j0 / kST3) << 10 | r.k0 / kST3;
         }
     }
-    if (threadIdx.x < 4)
+    if (threadIdx.x < 2)
         s_box[threadIdx.x] = 0;
     block_class_counts(c, counts);  // holds a barrier
     if (!box || blockIdx.x % stride)
         return;  // the whole block
-    const int other = __shfl_xor(tile, 32, kWave);
+    const int ln = threadIdx.x % kWave;
+    const uint32_t small = (uint32_t)(__ballot(vox != 0) >> (ln & -kRun)) & 0xffffu;
+    const int first = __shfl(tile, small ? (ln & -kRun) + __builtin_ctz(small) : ln, kWave);
+    if (ln % kRun == 0)
+        s_tile[threadIdx.x / kRun] = small ? first : -1;
     if (vox) {
         atomicAdd(&s_box[0], vox);
         atomicAdd(&s_box[1], 1);
-        if (other >= 0)
-            atomicAdd(&s_box[2], 1);
-        if (other == tile)
-            atomicAdd(&s_box[3], 1);
     }
     __syncthreads();
-    if (threadIdx.x == 0)
-        box[blockIdx.x / stride] = Small3Sample{s_box[0], s_box[1], s_box[2], s_box[3]};
+    if (threadIdx.x == 0) {
+        Small3Sample o{s_box[0], s_box[1], {}};
+        for (int k = 0; k < kSmall3Tiles; ++k)
+            o.tile[k] = s_tile[k];
+        box[blockIdx.x / stride] = o;
+    }
 }
 
 

@@ -1,6 +1,10 @@
-// k_small3.h -- index arithmetic of the windowed 3D small scatter, in plain
-// C++ so that it can be checked on the host.
+// k_small3.h -- index arithmetic of the windowed 3D small scatter and the rule
+// between it and the flat one, in plain C++ so that it can be checked on the
+// host.
 #pragma once
+
+#include <algorithm>
+#include <cstdint>
 
 namespace s2g {
 
@@ -35,6 +39,102 @@ constexpr Small3Lane small3_lane(int ln, int iw, int jw, int kw)
     const int ri = (int)(((float)ln + 0.5f) * (1.0f / (float)jk)), rem = ln - ri * jk;
     const int dj = (int)(((float)rem + 0.5f) * (1.0f / (float)kw));
     return Small3Lane{ri, dj, rem - dj * kw, ri < small3_planes(jk) ? iw - ri : 0};
+}
+
+// A sampled set-up block's small particles: voxels of their boxes, particles,
+// and the kST3^3 tile in which the first one of each run of 16 starts (-1: a
+// run without any).
+constexpr int kSmall3Blocks = 64, kSmall3Tiles = 16;
+struct Small3Sample {
+    int voxels, n, tile[kSmall3Tiles];
+};
+
+// The chance that two small particles start in the same tile: over the pairs
+// of sampled particles of different blocks, each standing for its share of its
+// block.  (Particles near each other in the caller's order are left out: in a
+// spatially ordered set they share a tile however sparse the set is.)
+inline double small3_share(const Small3Sample *sample, int64_t nsample)
+{
+    // the tiles' weights, of all blocks and of the block in hand
+    constexpr uint32_t kSlots = 2 * kSmall3Blocks * kSmall3Tiles;
+    static_assert((kSlots & (kSlots - 1)) == 0, "a power of two");
+    struct Slot {
+        int tile = -1;
+        double all = 0.0, block = 0.0;
+    };
+    Slot slots[kSlots];
+    double all = 0.0, same = 0.0, pairs = 0.0;
+    for (int64_t b = 0; b < nsample && b < kSmall3Blocks; ++b) {
+        const Small3Sample &s = sample[b];
+        int held = 0;
+        for (int t : s.tile)
+            held += t >= 0;
+        if (held == 0)
+            continue;
+        const double w = (double)s.n / held;
+        Slot *of[kSmall3Tiles];
+        int m = 0;
+        for (int t : s.tile) {
+            if (t < 0)
+                continue;
+            uint32_t k = (uint32_t)t * 2654435761u >> 20 & (kSlots - 1);
+            while (slots[k].tile >= 0 && slots[k].tile != t)
+                k = (k + 1) & (kSlots - 1);
+            slots[k].tile = t;
+            // pairs with the blocks before, then into this block's weight
+            same += 2.0 * w * slots[k].all;
+            slots[k].block += w;
+            of[m++] = &slots[k];
+        }
+        pairs += 2.0 * (double)s.n * all;
+        all += (double)s.n;
+        for (int i = 0; i < m; ++i) {
+            of[i]->all += of[i]->block;
+            of[i]->block = 0.0;
+        }
+    }
+    return pairs > 0.0 ? same / pairs : 0.0;
+}
+
+// The rule between the windowed and the flat scatter.  At least 32 particles
+// per tile, so that adding a window to the image costs less than their own
+// atomics (10^5 of the cluster set on 200^3, 7 per tile: 887 / 737 us), and
+// boxes large enough that their voxels' atomics outweigh the sort (`light`:
+// the lists that need none) and the work per particle.  The times are fitted to
+// whole calls: flat 12.5 ps per voxel, 0.8 us for every voxel of a wave's chain
+// of boxes, and 0.75 us for every voxel added to the same cell past 240, where
+// many share few (as many as the chance that two particles share a tile says);
+// windowed 0.2 ms for a sort (50 us without), 0.25 ns per particle (0.09 for
+// boxes of at most 2^3) and 4.6 ps per voxel.  Whole calls, windowed / flat,
+// us: uniform sets, 10^6 particles of 29 voxels on 48^3 762 / 488, in Morton
+// order 721 / 497, 4 10^5 of 14 on 24^3 435 / 183, 10^6 of 150 on 96^3 963 /
+// 1846, 2.5 10^5 of 85 on 48^3 330 / 370; the cluster set, 2 10^6 on 48^3 1169
+// / 2015, 3 10^4 on 24^3 145 / 107.  Over 176 such sets, shuffled and ordered,
+// the choice costs 2 % on average; the most, 1.29 times, where a cluster's
+// few densest voxels hold up the flat scatter by more than the chance of a
+// shared tile shows (2 10^6 on 128^3: 3.2 / 4.2 ms).
+inline bool small3_dense(int64_t ns, int64_t nstiles)
+{
+    return ns > 0 && nstiles < ((int64_t)1 << 30) && ns >= 32 * nstiles;
+}
+inline bool small3_windowed(int64_t ns, int64_t nstiles, const Small3Sample *sample,
+                            int64_t nsample, int64_t nd, bool light)
+{
+    if (!small3_dense(ns, nstiles))
+        return false;
+    double voxels = 0.0, boxes = 0.0;
+    for (int64_t k = 0; k < nsample; ++k) {
+        voxels += sample[k].voxels;
+        boxes += sample[k].n;
+    }
+    const double n = (double)ns, box = boxes > 0.0 ? voxels / boxes : 1.0, vox = box * n;
+    const double win = (light ? 50e-6 : 200e-6) + (box <= 8.0 ? 0.09e-9 : 0.25e-9) * n +
+                       4.6e-12 * vox;
+    if (win < std::max(12.5e-12 * vox, 0.8e-6 * box))
+        return true;
+    const double share = std::max(small3_share(sample, nsample), 1.0 / (double)nstiles);
+    const double cells = (double)nd / ((double)nstiles * share);
+    return win < 0.75e-6 * vox / cells - 180e-6;
 }
 
 }  // namespace s2g

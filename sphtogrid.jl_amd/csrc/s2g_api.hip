@@ -812,48 +812,8 @@ void deposit2d_device(s2g_ctx *c, const Map2DArgs &a, double *d_image, hipStream
     deposit2d_pass(c, &m, 1, s, st);
 }
 
-// Particles per work item of the windowed 3D scatter (heavy tiles are split),
-// and the rule between it and the flat scatter.  At least 32 particles per
-// tile, so that adding a window to the image costs less than their own atomics
-// (whole calls, windowed against flat: 20,000 particles of 8-voxel boxes on
-// 40^3, 160 per tile, 339 / 443 us; 10^6 of the cluster set on 101^3, 416 per
-// tile, 1.54 / 1.92 ms; on 256^3, 30 per tile, 5.76 / 5.82 ms; 10^5 on 200^3,
-// 7 per tile, 887 / 737 us); and boxes large enough that their voxels' atomics
-// outweigh the sort (`light`: the lists that need none) and the work per
-// particle.  The times are fitted to whole calls: flat 12.5 ps per voxel,
-// 0.8 us for every voxel of a wave's chain of boxes, and 0.6 us for every
-// voxel added to the same cell past 200, where many share few (as many as the
-// chance that two particles share a tile says); windowed 0.2 ms for a sort
-// (50 us without), 0.25 ns per particle (0.09 for boxes of at most 2^3) and
-// 4.6 ps per voxel.  Whole calls, windowed / flat, us: uniform sets, 10^6
-// particles of 29 voxels on 48^3 737 / 511, 4 10^5 of 14 on 24^3 419 / 215, 10^6
-// of 150 on 96^3 995 / 1706, 2.5 10^5 of 85 on 48^3 364 / 460; the cluster set,
-// 2 10^6 on 48^3 1179 / 1995, 3 10^4 on 24^3 158 / 128.
+// particles per work item of the windowed 3D scatter (heavy tiles are split)
 constexpr int64_t kSmall3Item = 512;
-bool small3_dense(int64_t ns, int64_t nstiles)
-{
-    return ns > 0 && nstiles < ((int64_t)1 << 30) && ns >= 32 * nstiles;
-}
-bool small3_windowed(int64_t ns, int64_t nstiles, const Small3Sample *sample, int64_t nsample,
-                     int64_t nd, bool light)
-{
-    if (!small3_dense(ns, nstiles))
-        return false;
-    double voxels = 0.0, boxes = 0.0, pairs = 0.0, same = 0.0;
-    for (int64_t k = 0; k < nsample; ++k) {
-        voxels += sample[k].voxels;
-        boxes += sample[k].n;
-        pairs += sample[k].pairs;
-        same += sample[k].same;
-    }
-    const double n = (double)ns, box = boxes > 0.0 ? voxels / boxes : 1.0, vox = box * n;
-    const double share = std::max(pairs > 0.0 ? same / pairs : 0.0, 1.0 / (double)nstiles);
-    const double cells = (double)nd / ((double)nstiles * share);
-    const double flat = std::max({12.5e-12 * vox, 0.8e-6 * box, 0.6e-6 * vox / cells - 120e-6});
-    const double win = (light ? 50e-6 : 200e-6) + (box <= 8.0 ? 0.09e-9 : 0.25e-9) * n +
-                       4.6e-12 * vox;
-    return win < flat;
-}
 
 // ---------------------------------------------------------------------------
 // 3D deposit on device pointers (image: npix^3 x 2, plane 0 = q, 1 = weights)
@@ -887,18 +847,17 @@ void deposit3d_device(s2g_ctx *c, const Map3DArgs &a, double *d_image, hipStream
     const TileMap stm{0, 0, (int32_t)(nstiles < INT32_MAX ? nstiles : 0), (int32_t)nst,
                       (int32_t)nst, 1, 0};
     const size_t btab = 2 * sizeof(int64_t) + (sizeof(TileMap) + 7) / 8 * 8;
-    // the small particles of at most 64 blocks of the set-up, for the rule
-    // between the small scatters
+    // a sample of the small particles, for the rule between the small scatters
     const int64_t nblk = partition_blocks(n);
-    const int stride = (int)((nblk + 63) / 64);
+    const int stride = (int)((nblk + kSmall3Blocks - 1) / kSmall3Blocks);
     const int64_t nsample = small3_dense(n, nstiles) ? (nblk + stride - 1) / stride : 0;
-    char *htab = (char *)c->h_tab.get(btab + sizeof(Small3Sample) * 64);
+    char *htab = (char *)c->h_tab.get(btab + sizeof(Small3Sample) * kSmall3Blocks);
     int64_t *hpb = (int64_t *)htab;
     Small3Sample *hbox = (Small3Sample *)(htab + btab);
     hpb[0] = 0;
     hpb[1] = n;
     *(TileMap *)(htab + 2 * sizeof(int64_t)) = stm;
-    int64_t *d_pbase = (int64_t *)c->tab.get(btab + sizeof(Small3Sample) * 64);
+    int64_t *d_pbase = (int64_t *)c->tab.get(btab + sizeof(Small3Sample) * kSmall3Blocks);
     Small3Sample *d_box = (Small3Sample *)((char *)d_pbase + btab);
     const TileMap *d_stm = (const TileMap *)(d_pbase + 2);
     S2G_HIP(hipMemcpyAsync(d_pbase, htab, btab, hipMemcpyHostToDevice, s));

@@ -1,9 +1,10 @@
-"""The index arithmetic of the windowed 3D small scatter (csrc/k_small3.h),
-compiled for the host.  CPU only."""
+"""The index arithmetic of the windowed 3D small scatter and the rule between it
+and the flat one (csrc/k_small3.h), compiled for the host.  CPU only."""
 import ctypes as C
 import os
 import subprocess
 
+import numpy as np
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -44,6 +45,13 @@ extern "C" int bad_cells(int iw, int jw, int kw)
     return bad;
 }
 extern "C" int side() { return kSmallSide3D; }
+extern "C" int blocks() { return kSmall3Blocks; }
+extern "C" int tiles() { return kSmall3Tiles; }
+extern "C" double share(const int *s, int64_t n) { return small3_share((const Small3Sample *)s, n); }
+extern "C" int windowed(int64_t ns, int64_t nt, const int *s, int64_t n, int64_t nd, int light)
+{
+    return small3_windowed(ns, nt, (const Small3Sample *)s, n, nd, light != 0);
+}
 """
 
 
@@ -54,7 +62,11 @@ def lib(tmp_path_factory):
     so = str(d / "t.so")
     subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-o", so, str(d / "t.cpp"),
                     "-I", os.path.join(ROOT, "sphtogrid.jl_amd", "csrc")], check=True)
-    return C.CDLL(so)
+    L = C.CDLL(so)
+    L.share.restype = C.c_double
+    L.share.argtypes = [C.c_void_p, C.c_int64]
+    L.windowed.argtypes = [C.c_int64, C.c_int64, C.c_void_p, C.c_int64, C.c_int64, C.c_int]
+    return L
 
 
 def test_lanes_cover_the_box_and_nothing_else(lib):
@@ -66,3 +78,41 @@ def test_lanes_cover_the_box_and_nothing_else(lib):
         for jw in range(1, n + 1):
             for kw in range(1, n + 1):
                 assert lib.bad_cells(iw, jw, kw) == 0, (iw, jw, kw)
+
+
+def _sample(lib, tile, vox):
+    """What the set-up samples of particles in this order (blocks of 256, the
+    first particle of every run of 16)."""
+    nblk = -(-len(tile) // 256)
+    stride = -(-nblk // lib.blocks())
+    out = []
+    for b in range(0, nblk, stride):
+        t, v = tile[256 * b: 256 * (b + 1)], vox[256 * b: 256 * (b + 1)]
+        first = np.full(lib.tiles(), -1)
+        first[: -(-len(t) // 16)] = t[::16]
+        out.append([v.sum(), len(t), *first])
+    return np.ascontiguousarray(out, dtype=np.int32)
+
+
+@pytest.mark.parametrize("npix,n,box,clump,want", [
+    (48, 1000000, 29, 1.0, 0),    # flat 450 us, windowed 720
+    (33, 400000, 25, 1.0, 0),     # 262, 450
+    (96, 1000000, 150, 1.0, 1),   # 1820, 960
+    (48, 1000000, 35, 0.3, 1),    # many in few cells
+    (18, 3000, 300, 1.0, 1),
+])
+def test_rule_does_not_depend_on_the_order(lib, npix, n, box, clump, want):
+    """The same set shuffled, tile by tile, and with its crowded part first."""
+    r = np.random.default_rng(n + npix)
+    x = r.random((n, 3))
+    x[: n // 2] = 0.5 + clump * (x[: n // 2] - 0.5)
+    c = (x * npix).astype(np.int64) // 9
+    nt = -(-npix // 9)
+    tile = (c[:, 0] * nt + c[:, 1]) * nt + c[:, 2]
+    vox = np.full(n, box)
+    true = ((np.bincount(tile) / n) ** 2).sum()
+    for order in (np.arange(n), r.permutation(n), np.argsort(tile, kind="stable")):
+        s = _sample(lib, tile[order], vox)
+        # systematic samples of 192 to 1024 particles: the chance within a half
+        assert 0.5 * true < max(lib.share(s.ctypes.data, len(s)), 1 / nt ** 3) < 1.5 * true
+        assert lib.windowed(n, nt ** 3, s.ctypes.data, len(s), npix ** 3, n <= 1 << 18) == want
