@@ -31,7 +31,7 @@ struct Small3Args {
 };
 
 // counts: the partition's per-block class counts
-// box: null, or a sample of every stride-th block of partition_blocks(a.n)
+// box: null, or a sample of one of every stride blocks of partition_blocks(a.n)
 void launch_3d_setup(const Map3DArgs &a, Rec3 *rec, int32_t *cls, int64_t *counts,
                      Small3Sample *box, int stride, hipStream_t s);
 // explicit normalisation sums (flags: S2G_FLAG_EXACT_NORM turns off the

@@ -107,8 +107,8 @@ __device__ __forceinline__ Rec3 setup3d(const T *__restrict__ pos, const T *__re
     return r;
 }
 
-// counts: the partition's per-block class counts.  box (or null): of every
-// `stride`-th block the small particles: Small3Sample.
+// counts: the partition's per-block class counts.  box (or null): of one block
+// of every `stride` the small particles: Small3Sample.
 template <typename T>
 __global__ __launch_bounds__(kPartBlock) void k3d_setup(
     const T *__restrict__ pos, const T *__restrict__ hsml, const T *__restrict__ m,
@@ -135,7 +135,8 @@ __global__ __launch_bounds__(kPartBlock) void k3d_setup(
     if (threadIdx.x < 2)
         s_box[threadIdx.x] = 0;
     block_class_counts(c, counts);  // holds a barrier
-    if (!box || blockIdx.x % stride)
+    const int group = (int)blockIdx.x / stride;
+    if (!box || (int)blockIdx.x != small3_block(group, stride, gridDim.x))
         return;  // the whole block
     const int ln = threadIdx.x % kWave;
     const uint32_t small = (uint32_t)(__ballot(vox != 0) >> (ln & -kRun)) & 0xffffu;
@@ -151,7 +152,7 @@ __global__ __launch_bounds__(kPartBlock) void k3d_setup(
         Small3Sample o{s_box[0], s_box[1], {}};
         for (int k = 0; k < kSmall3Tiles; ++k)
             o.tile[k] = s_tile[k];
-        box[blockIdx.x / stride] = o;
+        box[group] = o;
     }
 }
 

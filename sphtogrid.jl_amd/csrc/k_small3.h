@@ -49,6 +49,15 @@ struct Small3Sample {
     int voxels, n, tile[kSmall3Tiles];
 };
 
+// The block sampled of group i, blocks [i stride, (i + 1) stride) of nblk: not
+// the same one of each group, since a lattice's rows may be as long as a group.
+constexpr int small3_block(int i, int stride, int64_t nblk)
+{
+    const int64_t left = nblk - (int64_t)i * stride;
+    const uint32_t size = (uint32_t)(left < stride ? left : stride);
+    return i * stride + (int)(((uint32_t)i * 2654435769u >> 8) % size);
+}
+
 // The chance that two small particles start in the same tile: over the pairs
 // of sampled particles of different blocks, each standing for its share of its
 // block.  (Particles near each other in the caller's order are left out: in a
@@ -99,28 +108,30 @@ inline double small3_share(const Small3Sample *sample, int64_t nsample)
 // The rule between the windowed and the flat scatter.  At least 32 particles
 // per tile, so that adding a window to the image costs less than their own
 // atomics (10^5 of the cluster set on 200^3, 7 per tile: 887 / 737 us), and
-// boxes large enough that their voxels' atomics outweigh the sort (`light`:
-// the lists that need none) and the work per particle.  The times are fitted to
-// whole calls: flat 12.5 ps per voxel, 0.8 us for every voxel of a wave's chain
-// of boxes, and 0.75 us for every voxel added to the same cell past 240, where
-// many share few (as many as the chance that two particles share a tile says);
-// windowed 0.2 ms for a sort (50 us without), 0.25 ns per particle (0.09 for
-// boxes of at most 2^3) and 4.6 ps per voxel.  Whole calls, windowed / flat,
-// us: uniform sets, 10^6 particles of 29 voxels on 48^3 762 / 488, in Morton
-// order 721 / 497, 4 10^5 of 14 on 24^3 435 / 183, 10^6 of 150 on 96^3 963 /
-// 1846, 2.5 10^5 of 85 on 48^3 330 / 370; the cluster set, 2 10^6 on 48^3 1169
-// / 2015, 3 10^4 on 24^3 145 / 107.  Over 176 such sets, shuffled and ordered,
-// the choice costs 2 % on average; the most, 1.29 times, where a cluster's
-// few densest voxels hold up the flat scatter by more than the chance of a
-// shared tile shows (2 10^6 on 128^3: 3.2 / 4.2 ms).
+// then the difference of the two, fitted to whole calls: a window saves 6.9 ps
+// of global atomics per voxel, 0.97 us for every voxel of a mean box (a wave's
+// chain), and what the flat scatter waits where many particles share few
+// voxels; it costs the sort (165 us, 79 us for the lists that need none,
+// `light`) and 0.23 ns per particle (0.09 for boxes of at most 2^3).  The
+// crowding is the chance of a shared tile over that of a uniform set: beyond 1
+// it costs the flat scatter 0.28 us for every deposit on a mean voxel and 18 ps
+// per particle (up to 20 times).
+// Whole calls, windowed / flat, us: uniform sets, 10^6 particles of 29 voxels on
+// 48^3 762 / 488, in Morton order 721 / 497, 4 10^5 of 14 on 24^3 435 / 183,
+// 10^6 of 150 on 96^3 963 / 1846, 2.5 10^5 of 85 on 48^3 330 / 370; the cluster
+// set, 2 10^6 on 48^3 1169 / 2015, on 128^3 3198 / 4036, 3 10^4 on 24^3 145 /
+// 107.  Over 392 sets (uniform, lattices, clusters; shuffled and in Morton
+// order) the choice loses 1.7 % on average and 1.5 times at most (2 10^6 in 20
+// clumps on 48^3, Morton order, 657 / 999).
 inline bool small3_dense(int64_t ns, int64_t nstiles)
 {
     return ns > 0 && nstiles < ((int64_t)1 << 30) && ns >= 32 * nstiles;
 }
-inline bool small3_windowed(int64_t ns, int64_t nstiles, const Small3Sample *sample,
-                            int64_t nsample, int64_t nd, bool light)
+inline bool small3_windowed(int64_t ns, int64_t npix, const Small3Sample *sample,
+                            int64_t nsample, bool light)
 {
-    if (!small3_dense(ns, nstiles))
+    const int64_t nt = (npix + kST3 - 1) / kST3;
+    if (!small3_dense(ns, nt * nt * nt))
         return false;
     double voxels = 0.0, boxes = 0.0;
     for (int64_t k = 0; k < nsample; ++k) {
@@ -128,13 +139,15 @@ inline bool small3_windowed(int64_t ns, int64_t nstiles, const Small3Sample *sam
         boxes += sample[k].n;
     }
     const double n = (double)ns, box = boxes > 0.0 ? voxels / boxes : 1.0, vox = box * n;
-    const double win = (light ? 50e-6 : 200e-6) + (box <= 8.0 ? 0.09e-9 : 0.25e-9) * n +
-                       4.6e-12 * vox;
-    if (win < std::max(12.5e-12 * vox, 0.8e-6 * box))
+    const double gain = 6.9e-12 * vox + 0.97e-6 * box - (light ? 79e-6 : 165e-6) -
+                        (box <= 8.0 ? 0.093e-9 : 0.228e-9) * n;
+    if (gain > 0.0)
         return true;
-    const double share = std::max(small3_share(sample, nsample), 1.0 / (double)nstiles);
-    const double cells = (double)nd / ((double)nstiles * share);
-    return win < 0.75e-6 * vox / cells - 180e-6;
+    // the chance of a uniform set, whose last tile of an axis may be cut
+    const double w = (double)npix, last = w - (double)(kST3 * (nt - 1));
+    const double axis = ((double)(nt - 1) * kST3 * kST3 + last * last) / (w * w);
+    const double ex = std::max(small3_share(sample, nsample) / (axis * axis * axis) - 1.0, 0.0);
+    return gain + 0.283e-6 * ex * vox / (w * w * w) + 18e-12 * n * std::min(ex, 20.0) > 0.0;
 }
 
 }  // namespace s2g

@@ -876,7 +876,7 @@ void deposit3d_device(s2g_ctx *c, const Map3DArgs &a, double *d_image, hipStream
     if (partition_blocks(n) <= kPartLight && nstiles <= kMaxTiles)
         lt = light_lists(c, tm0, cl.lbase, {stm}, cl.sbase, ntiles, 64, 16,
                          (int64_t)sizeof(double) * 2 * kBT * kBT * kBT, s);
-    const bool windowed = small3_windowed(cl.ns, nstiles, hbox, nsample, nd, lt.ok);
+    const bool windowed = small3_windowed(cl.ns, npix, hbox, nsample, lt.ok);
 
     // Side streams, as in the 2D pass: the explicit normalisation and the
     // small-footprint scatter into the zeroed image, beside the pair lists

@@ -47,10 +47,11 @@ extern "C" int bad_cells(int iw, int jw, int kw)
 extern "C" int side() { return kSmallSide3D; }
 extern "C" int blocks() { return kSmall3Blocks; }
 extern "C" int tiles() { return kSmall3Tiles; }
+extern "C" int block(int i, int stride, int64_t n) { return small3_block(i, stride, n); }
 extern "C" double share(const int *s, int64_t n) { return small3_share((const Small3Sample *)s, n); }
-extern "C" int windowed(int64_t ns, int64_t nt, const int *s, int64_t n, int64_t nd, int light)
+extern "C" int windowed(int64_t ns, int64_t npix, const int *s, int64_t n, int light)
 {
-    return small3_windowed(ns, nt, (const Small3Sample *)s, n, nd, light != 0);
+    return small3_windowed(ns, npix, (const Small3Sample *)s, n, light != 0);
 }
 """
 
@@ -65,7 +66,8 @@ def lib(tmp_path_factory):
     L = C.CDLL(so)
     L.share.restype = C.c_double
     L.share.argtypes = [C.c_void_p, C.c_int64]
-    L.windowed.argtypes = [C.c_int64, C.c_int64, C.c_void_p, C.c_int64, C.c_int64, C.c_int]
+    L.block.argtypes = [C.c_int, C.c_int, C.c_int64]
+    L.windowed.argtypes = [C.c_int64, C.c_int64, C.c_void_p, C.c_int64, C.c_int]
     return L
 
 
@@ -86,7 +88,9 @@ def _sample(lib, tile, vox):
     nblk = -(-len(tile) // 256)
     stride = -(-nblk // lib.blocks())
     out = []
-    for b in range(0, nblk, stride):
+    for i in range(-(-nblk // stride)):
+        b = lib.block(i, stride, nblk)
+        assert i * stride <= b < min((i + 1) * stride, nblk)
         t, v = tile[256 * b: 256 * (b + 1)], vox[256 * b: 256 * (b + 1)]
         first = np.full(lib.tiles(), -1)
         first[: -(-len(t) // 16)] = t[::16]
@@ -102,7 +106,7 @@ def _sample(lib, tile, vox):
     (18, 3000, 300, 1.0, 1),
 ])
 def test_rule_does_not_depend_on_the_order(lib, npix, n, box, clump, want):
-    """The same set shuffled, tile by tile, and with its crowded part first."""
+    """The same set with its crowded part first, shuffled, and tile by tile."""
     r = np.random.default_rng(n + npix)
     x = r.random((n, 3))
     x[: n // 2] = 0.5 + clump * (x[: n // 2] - 0.5)
@@ -115,4 +119,17 @@ def test_rule_does_not_depend_on_the_order(lib, npix, n, box, clump, want):
         s = _sample(lib, tile[order], vox)
         # systematic samples of 192 to 1024 particles: the chance within a half
         assert 0.5 * true < max(lib.share(s.ctypes.data, len(s)), 1 / nt ** 3) < 1.5 * true
-        assert lib.windowed(n, nt ** 3, s.ctypes.data, len(s), npix ** 3, n <= 1 << 18) == want
+        assert lib.windowed(n, npix, s.ctypes.data, len(s), n <= 1 << 18) == want
+
+
+def test_share_of_a_lattice(lib):
+    """A lattice in its natural order, a plane of it as long as a sampled group
+    of blocks."""
+    npix, side = 24, 64
+    i = np.arange(side ** 3)
+    c = np.stack([i // side ** 2, i // side % side, i % side], 1) * npix // side // 9
+    tile = (c[:, 0] * 3 + c[:, 1]) * 3 + c[:, 2]
+    true = ((np.bincount(tile) / side ** 3) ** 2).sum()
+    s = _sample(lib, tile, np.full(side ** 3, 23))
+    assert abs(lib.share(s.ctypes.data, len(s)) / true - 1) < 0.5
+    assert lib.windowed(side ** 3, npix, s.ctypes.data, len(s), 1) == 0
