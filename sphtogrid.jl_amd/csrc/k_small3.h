@@ -108,20 +108,20 @@ inline double small3_share(const Small3Sample *sample, int64_t nsample)
 // The rule between the windowed and the flat scatter.  At least 32 particles
 // per tile, so that adding a window to the image costs less than their own
 // atomics (10^5 of the cluster set on 200^3, 7 per tile: 887 / 737 us), and
-// then the difference of the two, fitted to whole calls: a window saves 6.9 ps
-// of global atomics per voxel, 0.97 us for every voxel of a mean box (a wave's
+// then the difference of the two, fitted to whole calls: a window saves 7.2 ps
+// of global atomics per voxel, 0.54 us for every voxel of a mean box (a wave's
 // chain), and what the flat scatter waits where many particles share few
-// voxels; it costs the sort (165 us, 79 us for the lists that need none,
-// `light`) and 0.23 ns per particle (0.09 for boxes of at most 2^3).  The
-// crowding is the chance of a shared tile over that of a uniform set: beyond 1
-// it costs the flat scatter 0.28 us for every deposit on a mean voxel and 18 ps
-// per particle (up to 20 times).
+// voxels; it costs the sort (139 us, 83 us for the lists that need none,
+// `light`) and 0.23 ns per particle (boxes of at most 2^3, which it takes eight
+// to a wave: it saves 0.13).  The crowding is the chance of a shared tile over
+// that of a uniform set: beyond 1 it costs the flat scatter 0.28 us for every
+// deposit on a mean voxel and 18 ps per particle (up to 20 times).
 // Whole calls, windowed / flat, us: uniform sets, 10^6 particles of 29 voxels on
 // 48^3 762 / 488, in Morton order 721 / 497, 4 10^5 of 14 on 24^3 435 / 183,
 // 10^6 of 150 on 96^3 963 / 1846, 2.5 10^5 of 85 on 48^3 330 / 370; the cluster
 // set, 2 10^6 on 48^3 1169 / 2015, on 128^3 3198 / 4036, 3 10^4 on 24^3 145 /
 // 107.  Over 392 sets (uniform, lattices, clusters; shuffled and in Morton
-// order) the choice loses 1.7 % on average and 1.5 times at most (2 10^6 in 20
+// order) the choice loses 1.3 % on average and 1.5 times at most (2 10^6 in 20
 // clumps on 48^3, Morton order, 657 / 999).
 inline bool small3_dense(int64_t ns, int64_t nstiles)
 {
@@ -139,8 +139,8 @@ inline bool small3_windowed(int64_t ns, int64_t npix, const Small3Sample *sample
         boxes += sample[k].n;
     }
     const double n = (double)ns, box = boxes > 0.0 ? voxels / boxes : 1.0, vox = box * n;
-    const double gain = 6.9e-12 * vox + 0.97e-6 * box - (light ? 79e-6 : 165e-6) -
-                        (box <= 8.0 ? 0.093e-9 : 0.228e-9) * n;
+    const double gain = 7.2e-12 * vox + 0.54e-6 * box - (light ? 83e-6 : 139e-6) +
+                        (box <= 8.0 ? 0.135e-9 : -0.228e-9) * n;
     if (gain > 0.0)
         return true;
     // the chance of a uniform set, whose last tile of an axis may be cut

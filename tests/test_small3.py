@@ -104,6 +104,8 @@ def _sample(lib, tile, vox):
     (96, 1000000, 150, 1.0, 1),   # 1820, 960
     (48, 1000000, 35, 0.3, 1),    # many in few cells
     (18, 3000, 300, 1.0, 1),
+    (24, 2000000, 6, 1.0, 1),     # 633, 518
+    (40, 262144, 50, 1.0, 0),     # 297, 360
 ])
 def test_rule_does_not_depend_on_the_order(lib, npix, n, box, clump, want):
     """The same set with its crowded part first, shuffled, and tile by tile."""
