@@ -139,14 +139,15 @@ __global__ __launch_bounds__(kPartBlock) void k2d_setup(const Map2D *__restrict_
                                                         int64_t *__restrict__ counts)
 {
     const int64_t p = (int64_t)blockIdx.x * kPartBlock + threadIdx.x;
-    int c = kClsSkip;
+    int c = kClsSkip, tiles = 0;
     if (p < ntot) {
         const Rec2 r = setup2d<T>(maps, nmaps, p, nq, kernel);
         rec[p] = r;
         c = r.cls;
         cls[p] = c;
+        tiles = tile_count(r);
     }
-    block_class_counts(c, counts);
+    block_class_counts(c, tiles, counts);
 }
 
 

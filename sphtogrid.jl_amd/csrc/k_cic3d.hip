@@ -121,12 +121,13 @@ __global__ __launch_bounds__(kPartBlock) void k3d_setup(
     static_assert(kRun == 16, "four runs per wave");
     __shared__ int s_box[2], s_tile[kSmall3Tiles];
     const int64_t p = (int64_t)blockIdx.x * kPartBlock + threadIdx.x;
-    int c = kClsSkip, vox = 0, tile = -1;
+    int c = kClsSkip, tiles = 0, vox = 0, tile = -1;
     if (p < n) {
         const Rec3 r = setup3d(pos, hsml, m, rho, binq, w, npix, len2pix, kernel, flags, p);
         rec[p] = r;
         c = r.cls;
         cls[p] = c;
+        tiles = tile_count(r);
         if (c == kClsSmall) {
             vox = (r.i1 - r.i0 + 1) * (r.j1 - r.j0 + 1) * (r.k1 - r.k0 + 1);
             tile = (r.i0 / kST3) << 20 | (r.j0 / kST3) << 10 | r.k0 / kST3;
@@ -134,7 +135,7 @@ __global__ __launch_bounds__(kPartBlock) void k3d_setup(
     }
     if (threadIdx.x < 2)
         s_box[threadIdx.x] = 0;
-    block_class_counts(c, counts);  // holds a barrier
+    block_class_counts(c, tiles, counts);  // holds a barrier
     const int group = (int)blockIdx.x / stride;
     if (!box || (int)blockIdx.x != small3_block(group, stride, gridDim.x))
         return;  // the whole block

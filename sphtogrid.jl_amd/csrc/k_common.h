@@ -15,16 +15,18 @@ constexpr int kPairChunk = 4096;
 constexpr int kMaxTiles = 16384;
 
 int64_t partition_blocks(int64_t n);
-// counts: 3*partition_blocks(n)+1 int64, the per-block class counts as the
-// setup kernels write them (block_class_counts); afterwards counts[c*nb] is
+// counts: class_count_elems(n) int64, of which the first 3*partition_blocks(n)+1
+// are the per-block class counts as the setup kernels write them
+// (block_class_counts); afterwards counts[c*nb] is
 // the first index of class c in the concatenation and counts[3*nb] the grand
 // total
 void launch_partition(const int32_t *cls, int64_t n, int64_t *counts, int64_t *scan_tmp,
                       int32_t *l0, int32_t *l1, int32_t *l2, hipStream_t s);
 // The partition and the class bounds of a small pass (at most kPartLight
 // blocks) in one launch instead of four: every block adds up the counts of
-// the blocks before it.  out as launch_class_bounds writes it; counts is left
-// as it is.
+// the blocks before it.  out as launch_class_bounds writes it, and after it, in
+// out[2 nmaps + 6], the (tile, particle) pairs of the large particles; counts
+// is left as it is.
 constexpr int64_t kPartLight = 1024;
 void launch_partition_light(const int32_t *cls, int64_t n, const int64_t *counts,
                             const int64_t *pbase, int nmaps, int32_t *l0, int32_t *l1,
@@ -39,20 +41,72 @@ __device__ __forceinline__ void part_flags(int cls, int &f0, int &f1, int &f2)
     f2 = cls == kClsLargeEx;
 }
 
+__device__ __forceinline__ void tile_rect(const Rec2 &r, int &a0, int &a1, int &b0, int &b1,
+                                          int &c0, int &c1)
+{
+    a0 = r.i0 / kGT;
+    a1 = r.i1 / kGT;
+    b0 = r.j0 / kGT;
+    b1 = r.j1 / kGT;
+    c0 = c1 = 0;
+}
+
+__device__ __forceinline__ void tile_rect(const Rec3 &r, int &a0, int &a1, int &b0, int &b1,
+                                          int &c0, int &c1)
+{
+    a0 = r.i0 / kBT;
+    a1 = r.i1 / kBT;
+    b0 = r.j0 / kBT;
+    b1 = r.j1 / kBT;
+    c0 = r.k0 / kBT;
+    c1 = r.k1 / kBT;
+}
+
+// tiles (bricks) that a footprint meets, and a block's large particles together:
+// from kPairsMost on just that
+constexpr int64_t kPairsMost = ((int64_t)1 << 24) - 1;
+template <typename R>
+__device__ __forceinline__ int tile_count(const R &r)
+{
+    int a0, a1, b0, b1, c0, c1;
+    tile_rect(r, a0, a1, b0, b1, c0, c1);
+    const int64_t t = (int64_t)(a1 - a0 + 1) * (b1 - b0 + 1) * (c1 - c0 + 1);
+    return (int)(t < kPairsMost ? t : kPairsMost);
+}
+
+// int64 elements of `counts` for n particles: the class counts, their sentinel,
+// and for a small pass each block's pairs
+inline int64_t class_count_elems(int64_t n)
+{
+    const int64_t nb = (n + kPartBlock - 1) / kPartBlock;
+    return 3 * nb + 1 + (nb <= kPartLight ? nb : 0);
+}
+
 // Per-block class counts of the partition, from the setup kernel's blocks of
 // kPartBlock threads (cls: this thread's particle's class, kClsSkip past the
-// end; every thread of the block calls it)
-__device__ __forceinline__ void block_class_counts(int cls, int64_t *__restrict__ counts)
+// end; every thread of the block calls it).  tiles: the tile_count of a large
+// particle; a small pass sizes its pair lists and partial sums by their sum.
+__device__ __forceinline__ void block_class_counts(int cls, int tiles,
+                                                   int64_t *__restrict__ counts)
 {
     __shared__ int s[3][kPartBlock / kWave];
+    __shared__ int s_tiles[kPartBlock / kWave];
     int f0, f1, f2;
     part_flags(cls, f0, f1, f2);
     const int wv = threadIdx.x / kWave, ln = threadIdx.x % kWave;
     const uint64_t b0 = __ballot(f0), b1 = __ballot(f1), b2 = __ballot(f2);
+    const bool light = gridDim.x <= kPartLight;  // uniform
+    if (light) {
+        tiles = f1 ? tiles : 0;
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1)
+            tiles += __shfl_xor(tiles, o, kWave);  // below 2^30
+    }
     if (ln == 0) {
         s[0][wv] = __popcll(b0);
         s[1][wv] = __popcll(b1);
         s[2][wv] = __popcll(b2);
+        s_tiles[wv] = tiles;
     }
     __syncthreads();
     if (threadIdx.x < 3) {
@@ -60,6 +114,12 @@ __device__ __forceinline__ void block_class_counts(int cls, int64_t *__restrict_
         for (int k = 0; k < kPartBlock / kWave; ++k)
             t += s[threadIdx.x][k];
         counts[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = t;
+    }
+    if (light && threadIdx.x == 4) {
+        int64_t t = 0;
+        for (int k = 0; k < kPartBlock / kWave; ++k)
+            t += s_tiles[k];
+        counts[3 * (int64_t)gridDim.x + 1 + blockIdx.x] = t < kPairsMost ? t : kPairsMost;
     }
     if (blockIdx.x == 0 && threadIdx.x == 3)
         counts[3 * (int64_t)gridDim.x] = 0;  // becomes the grand total after the scan

@@ -47,7 +47,8 @@ __global__ __launch_bounds__(kPartBlock) void k_part_scatter(
 
 // The same lists for a small pass: each block adds up the counts of the blocks
 // before it (at most kPartLight, 24 KB from the cache), so no scan runs, and
-// the block that holds a map's first particle writes the map's bounds.
+// the block that holds a map's first particle writes the map's bounds.  The
+// first block also adds up the pairs.
 __global__ __launch_bounds__(kPartBlock) void k_part_light(
     const int32_t *__restrict__ cls, int64_t n, const int64_t *__restrict__ counts,
     const int64_t *__restrict__ pbase, int nmaps, int32_t *__restrict__ l0,
@@ -55,6 +56,7 @@ __global__ __launch_bounds__(kPartBlock) void k_part_light(
 {
     constexpr int kW = kPartBlock / kWave;
     __shared__ int s_pre[3][kW], s_tot[3][kW];
+    __shared__ uint32_t s_pairs[kW];
     __shared__ uint64_t s_bal[3][kW];
     const int nb = gridDim.x;
     const int wv = threadIdx.x / kWave, ln = threadIdx.x % kWave;
@@ -75,6 +77,18 @@ __global__ __launch_bounds__(kPartBlock) void k_part_light(
             s_tot[k][wv] = tot;
         }
     }
+    if (blockIdx.x == 0) {
+        // at most kPartLight / kPartBlock blocks a thread: a wave's sum fits
+        uint32_t v = 0;
+        for (int b = threadIdx.x; b < nb; b += kPartBlock)
+            v += (uint32_t)counts[3 * (int64_t)nb + 1 + b];
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1)
+            v += __shfl_xor(v, o, kWave);
+        if (ln == 0)
+            s_pairs[wv] = v;
+    }
+    static_assert((int64_t)kWave * (kPartLight / kPartBlock) * kPairsMost < ((int64_t)1 << 32));
     const int64_t p = (int64_t)blockIdx.x * kPartBlock + threadIdx.x;
     int f[3];
     part_flags(p < n ? cls[p] : kClsSkip, f[0], f[1], f[2]);
@@ -107,6 +121,11 @@ __global__ __launch_bounds__(kPartBlock) void k_part_light(
         for (int k = 0; k < (int)threadIdx.x; ++k)
             v += tot[k];
         out[threadIdx.x] = v;
+    } else if (blockIdx.x == 0 && threadIdx.x == 4) {
+        int64_t v = 0;
+        for (int w = 0; w < kW; ++w)
+            v += s_pairs[w];
+        out[2 * nmaps + 6] = v;
     }
     for (int m = threadIdx.x; m <= nmaps; m += kPartBlock) {
         const int64_t p0 = m < nmaps ? pbase[m] : n;
@@ -209,26 +228,6 @@ void launch_class_bounds(const int64_t *counts, int64_t nb, const int32_t *small
 // Local tiles are t = (a * nt + b) * ntc + c over the map's tile grid
 // (ntc = 1 in 2D).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void tile_rect(const Rec2 &r, int &a0, int &a1, int &b0, int &b1,
-                                          int &c0, int &c1)
-{
-    a0 = r.i0 / kGT;
-    a1 = r.i1 / kGT;
-    b0 = r.j0 / kGT;
-    b1 = r.j1 / kGT;
-    c0 = c1 = 0;
-}
-
-__device__ __forceinline__ void tile_rect(const Rec3 &r, int &a0, int &a1, int &b0, int &b1,
-                                          int &c0, int &c1)
-{
-    a0 = r.i0 / kBT;
-    a1 = r.i1 / kBT;
-    b0 = r.j0 / kBT;
-    b1 = r.j1 / kBT;
-    c0 = r.k0 / kBT;
-    c1 = r.k1 / kBT;
-}
 
 // Order in which the tile lists take a map's large particles.  The map's
 // large-list segment e_0 .. e_{L-1} (particle order) is read as f_j =

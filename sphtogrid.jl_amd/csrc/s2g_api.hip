@@ -38,7 +38,7 @@ struct s2g_ctx {
     // explicit normalisation and the small-footprint scatter run there beside
     // the pair lists and the gather, ordered by the fork / join events
     hipStream_t side = nullptr;
-    // of a light pass: the small-footprint scatter beside the normalisation too
+    // of a small pass: the small-footprint scatter beside the normalisation too
     hipStream_t side2 = nullptr;
     hipEvent_t fork = nullptr, normed = nullptr, smalled = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -275,17 +275,28 @@ TilePlan build_tile_lists(s2g_ctx *c, const int32_t *large, const void *rec, boo
 }
 
 // ---------------------------------------------------------------------------
-// Light passes: of few particles and tiles, where the launches and the host's
+// Light passes: of few particles and pairs, where the launches and the host's
 // round trips take longer than the kernels.  One launch partitions the classes
 // (launch_partition_light), one scans each list's counts and cuts its items
 // (launch_lists_light), the small footprints are bucketed by the counting sort
 // instead of the radix sort, and the pair and item counts stay on the device
-// (capacities from true bounds), so the host reads back once, the class
-// sizes.  Measured whole calls: 65,536 particles on 256^2 @L1@ us; 4,096 on
-// 64^2 through sphMapping @L2@ us.
+// (the buffers are sized by the pairs that the set-up counts), so the host
+// waits twice, for the class sizes and at the end.  Measured whole calls:
+// 65,536 particles on 256^2 343 -> 222 us; 4,096 on 64^2 through sphMapping
+// 468 -> 352.
+// Up to 2^17 pairs, whose lists are filled from chunks of at most 128 large
+// particles, a wave each: past that the one block that scans and the long
+// chunks cost more than the launches (light / general, us: 65,536 on 512^2,
+// 188 k pairs, 444 / 413; 30,000 of a lattice on 128^3, 204 k pairs in chunks of
+// 256, 493 / 377; 262,000 on 1500^2, 1.7 M pairs in chunks of 4096, 3834 / 2560;
+// 150,001 on 777^2, four planes, 174 k pairs, 594 / 568; below it 20,000 on
+// 512^2, 13 k pairs, 178 / 254; over 339 small passes the choice loses 0.8 % on
+// average).
 // ---------------------------------------------------------------------------
-constexpr int64_t kLightPairs = (int64_t)1 << 24;     // pair capacity
-constexpr int64_t kLightPartial = (int64_t)1 << 29;   // bytes of item partials
+constexpr int64_t kLightPairs = (int64_t)1 << 17;
+constexpr int64_t kLightChunk = 128;
+constexpr int64_t kLightPartial = (int64_t)1 << 28;   // bytes of item partials
+static_assert(kLightPairs < kPairsMost, "the pairs are counted up to there");
 
 // Chunk size of a counting sort over `len` list entries and `ntl` tiles in a
 // light pass: at least `least` entries, grown until the counters are few
@@ -298,9 +309,10 @@ int64_t light_chunk(int64_t len, int64_t ntl, int64_t least)
 }
 
 // A counting sort's tables for a light pass: per map the chunks of its list
-// segment lens[m]; returns the counter count, or -1 if it is no light one
+// segment lens[m]; returns the counter count, or -1 if it is no light one (a
+// chunk longer than `most` among it)
 int64_t light_tables(std::vector<TileMap> &tm, const std::vector<int64_t> &lbase, int64_t least,
-                     std::vector<PairChunk> &chunks, int *max_tiles)
+                     int64_t most, std::vector<PairChunk> &chunks, int *max_tiles)
 {
     int64_t cb = 0;
     *max_tiles = 1;
@@ -310,6 +322,8 @@ int64_t light_tables(std::vector<TileMap> &tm, const std::vector<int64_t> &lbase
             return -1;
         *max_tiles = tm[m].ntiles > *max_tiles ? tm[m].ntiles : *max_tiles;
         const int64_t csz = light_chunk(len, tm[m].ntiles, least);
+        if (csz > most)
+            return -1;
         const int64_t nch = (len + csz - 1) / csz;
         tm[m].cbase = cb;
         tm[m].nch = (int32_t)nch;
@@ -332,20 +346,23 @@ struct LightTables {
 
 // tm / stm: tile grids of the large and of the small lists' maps (the small
 // ones may be empty: the caller buckets them otherwise); lbase / sbase: the
-// maps' list starts.  planes x plane_elems doubles of partials per item.
+// maps' list starts; npairs: the pairs of the pass; partial_bytes: of an item's
+// partial sums.
 LightTables light_lists(s2g_ctx *c, std::vector<TileMap> tm, const std::vector<int64_t> &lbase,
                         std::vector<TileMap> stm, const std::vector<int64_t> &sbase, int ntiles,
-                        int64_t gmin, int64_t per_cu, int64_t partial_bytes, hipStream_t s)
+                        int64_t npairs, int64_t gmin, int64_t per_cu, int64_t partial_bytes,
+                        hipStream_t s)
 {
     LightTables lt;
     std::vector<PairChunk> ch, sch;
-    lt.ncnt = light_tables(tm, lbase, 64, ch, &lt.max_tiles);
-    lt.sncnt = light_tables(stm, sbase, 512, sch, &lt.smax_tiles);
-    for (size_t m = 0; m < tm.size(); ++m)
-        lt.pair_cap += (lbase[m + 1] - lbase[m]) * tm[m].ntiles;
+    lt.ncnt = light_tables(tm, lbase, 64, kLightChunk, ch, &lt.max_tiles);
+    lt.sncnt = light_tables(stm, sbase, 512, INT64_MAX, sch, &lt.smax_tiles);
+    lt.pair_cap = npairs;
+    // one item per tile that holds pairs, and total / G more (G >= gmin and G
+    // >= total / target, item_size)
     const int64_t target = (int64_t)c->ncu * per_cu;
-    const int64_t byp = (lt.pair_cap + gmin - 1) / gmin;
-    lt.item_cap = ntiles + (byp < target ? byp : target);
+    const int64_t byp = (npairs + gmin - 1) / gmin;
+    lt.item_cap = (ntiles < npairs ? ntiles : npairs) + (byp < target ? byp : target);
     if (lt.ncnt < 0 || lt.sncnt < 0 || lt.pair_cap > kLightPairs ||
         lt.item_cap * partial_bytes > kLightPartial)
         return lt;
@@ -388,8 +405,7 @@ TilePlan light_tile_lists(s2g_ctx *c, const int32_t *large, const R *rec, const 
         S2G_HIP(hipEventRecord(E[4], s));
     launch_pairs<R>(large, rec, lt.d_ch, lt.nchunks, lt.d_tm, lt.max_tiles, cnt, lt.ncnt, nullptr,
                     nullptr, false, s, d_lbase, INT64_MAX, false);
-    // item_cap covers every item: ntiles + ceil(total / G) with G >= gmin
-    // and G >= total / target (gmax applies within that: tmax)
+    // item_cap covers every item (gmax applies within the target: tmax)
     const int64_t target = (int64_t)c->ncu * per_cu;
     launch_lists_light(cnt, lt.ncnt, lt.d_tm, nmaps, ntiles, gmin, target, gmax, target,
                        tp.d_npairs, nit, tp.items, lt.item_cap, tp.tile_items, s);
@@ -431,6 +447,7 @@ SmallItems light_small_lists(s2g_ctx *c, const int32_t *list, int64_t ns, const 
 
 struct ClassLists {
     int64_t ns = 0, nl = 0, ne = 0;
+    int64_t npairs = -1;  // of a small pass: the (tile, particle) pairs (tile_count)
     int32_t *l0 = nullptr, *l1 = nullptr, *l2 = nullptr;
     std::vector<int64_t> lbase;  // per-map first large-list entry (+ the total)
     const int64_t *d_lbase = nullptr;  // the same on the device
@@ -441,7 +458,7 @@ struct ClassLists {
 // the per-block class counts that the setup kernels write
 int64_t *class_counts(s2g_ctx *c, int64_t n)
 {
-    return (int64_t *)c->counts.get(sizeof(int64_t) * (3 * partition_blocks(n) + 1));
+    return (int64_t *)c->counts.get(sizeof(int64_t) * class_count_elems(n));
 }
 
 // stable class partition of the pass's particles (counts: class_counts, filled
@@ -455,7 +472,7 @@ ClassLists partition_classes(s2g_ctx *c, const int32_t *cls, int64_t n, int64_t 
     cl.l0 = (int32_t *)c->lists[0].get(sizeof(int32_t) * n);
     cl.l1 = (int32_t *)c->lists[1].get(sizeof(int32_t) * n);
     cl.l2 = (int32_t *)c->lists[2].get(sizeof(int32_t) * n);
-    int64_t *bounds = (int64_t *)c->bounds.get(sizeof(int64_t) * (2 * nmaps + 6));
+    int64_t *bounds = (int64_t *)c->bounds.get(sizeof(int64_t) * (2 * nmaps + 7));
     if (nb <= kPartLight) {
         launch_partition_light(cls, n, counts, d_pbase, nmaps, cl.l0, cl.l1, cl.l2, bounds, s);
     } else {
@@ -465,8 +482,8 @@ ClassLists partition_classes(s2g_ctx *c, const int32_t *cls, int64_t n, int64_t 
     }
     if (timed)
         S2G_HIP(hipEventRecord(c->stage[1], s));
-    int64_t *h = (int64_t *)c->h_bounds.get(sizeof(int64_t) * (2 * nmaps + 6));
-    S2G_HIP(hipMemcpyAsync(h, bounds, sizeof(int64_t) * (2 * nmaps + 6), hipMemcpyDeviceToHost,
+    int64_t *h = (int64_t *)c->h_bounds.get(sizeof(int64_t) * (2 * nmaps + 7));
+    S2G_HIP(hipMemcpyAsync(h, bounds, sizeof(int64_t) * (2 * nmaps + 7), hipMemcpyDeviceToHost,
                            s));
     S2G_HIP(hipStreamSynchronize(s));
     cl.ns = h[1] - h[0];
@@ -476,6 +493,8 @@ ClassLists partition_classes(s2g_ctx *c, const int32_t *cls, int64_t n, int64_t 
     cl.d_lbase = bounds + 4;
     cl.sbase.assign(h + 5 + nmaps, h + 6 + 2 * nmaps);
     cl.d_sbase = bounds + 5 + nmaps;
+    if (nb <= kPartLight)
+        cl.npairs = h[2 * nmaps + 6];
     return cl;
 }
 
@@ -641,7 +660,7 @@ void deposit2d_pass(s2g_ctx *c, const MapIn *mi, int nmaps, hipStream_t s, s2g_s
     const int64_t gmin = c->tune.gather_item_min * (np0 > 2 && !fp32acc ? 2 : 1);
     LightTables lt;
     if (ntot > 0 && partition_blocks(ntot) <= kPartLight)
-        lt = light_lists(c, tm, cl.lbase, pt.stm, cl.sbase, ntiles, gmin,
+        lt = light_lists(c, tm, cl.lbase, pt.stm, cl.sbase, ntiles, cl.npairs, gmin,
                          c->tune.gather_items_per_cu,
                          (int64_t)sizeof(double) * np0 * kGT * kGT, s);
 
@@ -652,9 +671,9 @@ void deposit2d_pass(s2g_ctx *c, const MapIn *mi, int nmaps, hipStream_t s, s2g_s
     // waits for it and adds the large particles' sums (2^24 cluster set on
     // 4096^2: the 5.7 ms normalisation runs beside the 5.7 ms pair lists and
     // the 6.4 ms small scatter beside the gather; 288 -> 284 ms per step).
-    // A light pass leaves CUs idle in every stage: there the small scatter
-    // has a stream of its own.
-    hipStream_t s2 = c->side, s3 = lt.ok ? c->side2 : s2;
+    // A small pass leaves CUs idle in every stage: there the small scatter
+    // has a stream of its own (3D, 130,000 on 80^3: 787 -> 648 us).
+    hipStream_t s2 = c->side, s3 = partition_blocks(ntot) <= kPartLight ? c->side2 : s2;
     S2G_HIP(hipEventRecord(c->fork, s));
     S2G_HIP(hipStreamWaitEvent(s2, c->fork, 0));
     if (s3 != s2)
@@ -874,7 +893,7 @@ void deposit3d_device(s2g_ctx *c, const Map3DArgs &a, double *d_image, hipStream
     const std::vector<TileMap> tm0{TileMap{0, 0, ntiles, nb, nb, 0, 0}};
     LightTables lt;
     if (partition_blocks(n) <= kPartLight && nstiles <= kMaxTiles)
-        lt = light_lists(c, tm0, cl.lbase, {stm}, cl.sbase, ntiles, 64, 16,
+        lt = light_lists(c, tm0, cl.lbase, {stm}, cl.sbase, ntiles, cl.npairs, 64, 16,
                          (int64_t)sizeof(double) * 2 * kBT * kBT * kBT, s);
     const bool windowed = small3_windowed(cl.ns, npix, hbox, nsample, lt.ok);
 
@@ -882,7 +901,7 @@ void deposit3d_device(s2g_ctx *c, const Map3DArgs &a, double *d_image, hipStream
     // small-footprint scatter into the zeroed image, beside the pair lists
     // and the gather; the gather waits for the normalisation and the
     // finalize for the scatter, to whose sums it adds.
-    hipStream_t s2 = c->side, s3 = lt.ok ? c->side2 : s2;
+    hipStream_t s2 = c->side, s3 = partition_blocks(n) <= kPartLight ? c->side2 : s2;
     S2G_HIP(hipEventRecord(c->fork, s));
     S2G_HIP(hipStreamWaitEvent(s2, c->fork, 0));
     if (s3 != s2)
@@ -1531,11 +1550,11 @@ void plan_pass_build(s2g_ctx *c, PlanPass &pp, double headroom, hipStream_t s)
     pp.nb = partition_blocks(n);
     pp.rec.get(sizeof(Rec2) * n);
     pp.cls.get(sizeof(int32_t) * n);
-    pp.counts.get(sizeof(int64_t) * (3 * pp.nb + 1));
+    pp.counts.get(sizeof(int64_t) * class_count_elems(n));
     pp.l0.get(sizeof(int32_t) * n);
     pp.l1.get(sizeof(int32_t) * n);
     pp.l2.get(sizeof(int32_t) * n);
-    pp.bounds.get(sizeof(int64_t) * (2 * nmaps + 6));
+    pp.bounds.get(sizeof(int64_t) * (2 * nmaps + 7));
     pp.flag.get(sizeof(int) * 2);
     // creation run of the class stages: the per-map large counts
     launch_2d_setup(pp.dtype, pp.d_maps, nmaps, pp.ntot, pp.nq, pp.kernel, (Rec2 *)pp.rec.p,

@@ -334,6 +334,7 @@ struct DevBuf {
             b = (b + 255) & ~size_t(255);
             if (hipMalloc(&p, b) != hipSuccess) {
                 p = nullptr;
+                (void)hipGetLastError();  // told here, not by a later check
                 throw Error(S2G_ENOMEM, "device allocation of " + std::to_string(b) +
                                             " bytes failed");
             }
@@ -341,9 +342,19 @@ struct DevBuf {
         }
         return p;
     }
-    // the same, grown by a quarter more than asked for: sizes that vary a
-    // little from call to call would otherwise reallocate again and again
-    void *get_roomy(size_t need) { return need > bytes ? get(need + need / 4) : p; }
+    // the same, grown by a quarter more than asked for, 16 MB at most: sizes
+    // that vary a little from call to call would otherwise reallocate again
+    // and again (where that much is not to be had, just the size)
+    void *get_roomy(size_t need)
+    {
+        if (need <= bytes)
+            return p;
+        try {
+            return get(need + (need / 4 < ((size_t)16 << 20) ? need / 4 : (size_t)16 << 20));
+        } catch (const Error &) {
+            return get(need);
+        }
+    }
     void release()
     {
         if (p)

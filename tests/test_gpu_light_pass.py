@@ -83,3 +83,33 @@ def test_small_item_floor(s2g, orc, n):
     for k in range(2):
         assert np.abs(gpu[:, k] - ref[:, k]).sum() <= 1e-5 * np.abs(ref[:, k]).sum(), k
     assert abs(gpu[:, 1].sum() / ref[:, 1].sum() - 1) <= 1e-6
+
+
+@pytest.mark.parametrize("dims,npix,n,nq,hmax", [(2, 256, 65536, 1, 24.0), (2, 777, 100000, 3, 60.0),
+                                                 (3, 100, 100000, 1, 7.0)])
+def test_light_pass_memory_follows_its_pairs(s2g, dims, npix, n, nq, hmax):
+    """A light pass holds what its (tile, particle) pairs need, not what every
+    large footprint on every tile would: the partial sums of one work item per
+    tile and one per least item size, a quarter or 16 MB to spare, and per
+    particle and pixel less than 400 and 100 bytes."""
+    import torch
+    from sph2grid import _lib
+    x, h, m, rho, q, w = _set(n, npix, 7, hmax)
+    q = np.stack([q] * nq, 1) if nq > 1 else q
+    ctx = _lib.Context()
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    st = {}
+    s2g.deposit(x, h, m, rho, q, w, npix=npix, len2pix=float(npix), dimensions=dims,
+                kernel=s2g.Cubic(dims), calc_mean=False, context=ctx, stats=st)
+    held = free - torch.cuda.mem_get_info()[0]
+    ctx.close()
+    side, planes, least = (64, nq + 1, 64 if nq < 2 else 128) if dims == 2 else (16, 2, 64)
+    tiles = (-(-npix // side)) ** dims
+    items = min(tiles, st["n_pairs"]) + min(-(-st["n_pairs"] // least), 16 * 256)
+    partial = items * planes * 8 * side ** dims
+    assert 0 < st["n_pairs"] < st["n_large"] * tiles / 2
+    bound = 1.25 * partial + (16 << 20) + 400 * n + 100 * (nq + 1) * npix ** dims
+    print(f"[light memory {dims}d {npix}] held {held >> 20} MB, partials {partial >> 20} MB, "
+          f"{st['n_pairs']} pairs", flush=True)
+    assert held <= bound, (held, bound)
