@@ -149,14 +149,17 @@ typedef struct s2g_tuning {
                                     (>= 5 keeps every particle of hsml < 2 px, whose
                                     weights need FP64, in the scatter) */
     int32_t small_item_min;      /* least particles per small-footprint work item;
-                                    16..4096, default 256 (half of it in a pass of at
-                                    most 2^18 particles, a quarter where half
-                                    would not give every CU an item) */
+                                    16..4096, default 256 (on a context whose tuning was
+                                    not set, half of it in a pass of at most 2^18
+                                    particles and 2^17 (tile, particle) pairs, a quarter
+                                    where half would not give every CU an item; plans
+                                    take it as it stands) */
     int32_t small_items_per_cu;  /* small-footprint work items per CU aimed at;
                                     1..64, default 16 */
     int32_t gather_item_min;     /* least (tile, particle) pairs per gather work item;
-                                    8..4096, default 64 (twice that where a launch
-                                    accumulates three or four FP64 planes) */
+                                    8..4096, default 64 (on a context whose tuning was
+                                    not set, twice that where a launch accumulates three
+                                    or four FP64 planes; plans take it as it stands) */
     int32_t gather_items_per_cu; /* gather work items per CU aimed at; 1..256, default 16 */
     int32_t gather_planes;       /* image planes per gather launch; 1..4, default 4 */
     int32_t small_planes;        /* image planes per small-footprint launch; 1..4, default 4 */
@@ -173,7 +176,8 @@ void s2g_destroy(s2g_ctx *ctx);
 const char *s2g_last_error(const s2g_ctx *ctx);
 /* library version string, e.g. "sph2grid 0.1.0 gfx950" */
 const char *s2g_version(void);
-/* Work split of later 2D deposits on this context (NULL: the defaults);
+/* Work split of later 2D deposits on this context (NULL: the defaults), taken
+ * as it stands, also where it equals the defaults;
  * out-of-range fields give S2G_EINVAL and leave the setting unchanged.  No
  * counterpart in the reference (its deposit is one loop per worker). */
 int s2g_set_tuning(s2g_ctx *ctx, const s2g_tuning *tuning);

@@ -70,6 +70,7 @@ struct s2g_ctx {
     std::string scratch_err;
     // work split of the 2D deposit
     s2g_tuning tune = kDefaultTuning;
+    bool tuned = false;  // set by the caller: the least item sizes are taken as they stand
 };
 
 namespace {
@@ -655,9 +656,9 @@ void deposit2d_pass(s2g_ctx *c, const MapIn *mi, int nmaps, hipStream_t s, s2g_s
     const int gstep = c->tune.gather_planes;
     // three or four FP64 planes run two blocks per CU: items of twice the
     // least size halve their partials for little balance (777^2, four planes:
-    // gather 229 -> 243 us, finalize 111 -> 42 us)
+    // gather 229 -> 243 us, finalize 111 -> 42 us), unless the caller set a size
     const int np0 = nplanes < gstep ? nplanes : gstep;
-    const int64_t gmin = c->tune.gather_item_min * (np0 > 2 && !fp32acc ? 2 : 1);
+    const int64_t gmin = c->tune.gather_item_min * (np0 > 2 && !fp32acc && !c->tuned ? 2 : 1);
     LightTables lt;
     if (ntot > 0 && partition_blocks(ntot) <= kPartLight)
         lt = light_lists(c, tm, cl.lbase, pt.stm, cl.sbase, ntiles, cl.npairs, gmin,
@@ -699,9 +700,10 @@ void deposit2d_pass(s2g_ctx *c, const MapIn *mi, int nmaps, hipStream_t s, s2g_s
         // particles on 256^2: scatter 97 -> 70 us; quartered 78 us, the
         // windows' own cost), and quarters it where half would not give every
         // CU one (whole calls, half / quarter: 4,096 particles on 64^2 151 /
-        // 133 us, 8,000 of a blast on 128^2 170 / 136, 30,000 on 128^2 187 / 173)
+        // 133 us, 8,000 of a blast on 128^2 170 / 136, 30,000 on 128^2 187 /
+        // 173), unless the caller set a size
         const int64_t half = (c->tune.small_item_min + 1) / 2;
-        const int64_t smin = !lt.ok               ? c->tune.small_item_min
+        const int64_t smin = !lt.ok || c->tuned   ? c->tune.small_item_min
                              : ns < half * c->ncu ? (half + 1) / 2
                                                   : half;
         if (Gs < smin)
@@ -1791,6 +1793,7 @@ int s2g_set_tuning(s2g_ctx *c, const s2g_tuning *t)
     return guarded(c, [&] {
         if (!t) {
             c->tune = kDefaultTuning;
+            c->tuned = false;
             return S2G_OK;
         }
         auto in = [](int32_t v, int32_t lo, int32_t hi) { return v >= lo && v <= hi; };
@@ -1812,6 +1815,7 @@ int s2g_set_tuning(s2g_ctx *c, const s2g_tuning *t)
             throw Error(S2G_EINVAL, "gather_item_max out of range (0, or gather_item_min "
                                     "to 2^30)");
         c->tune = *t;
+        c->tuned = true;
         return S2G_OK;
     });
 }

@@ -97,3 +97,30 @@ def test_autotune_small_map(s2g, orc, ctx, tmp_path):
     ref = orc.cic_mapping_2D(x, h, m, rho, q[:, 0], w, npix, float(npix), "cubic", 2, False)
     for k in range(2):
         assert rel_l1(got[:, k], ref[:, k]) <= 1e-5
+
+
+@pytest.mark.parametrize("least", [64, 128])
+def test_set_item_size_is_taken_as_it_stands(s2g, ctx, least):
+    """A set gather_item_min cuts the items of an eager call as it cuts those of
+    a plan, which takes it as it stands: the same FP64 sums in the same order,
+    bit for bit (large footprints only, three FP64 planes per launch)."""
+    import torch
+    npix, n, nq = 128, 900, 2
+    r = np.random.default_rng(least)
+    x = r.uniform(-0.5, 0.5, (n, 3))
+    h = r.uniform(20.0, 40.0, n) / npix
+    m, rho, w = (r.uniform(0.5, 2.0, n) for _ in range(3))
+    q = r.uniform(0.1, 5.0, (n, nq))
+    t = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (x, h, m, rho, q, w)]
+    out = [torch.empty((nq + 1) * npix * npix, dtype=torch.float64, device="cuda")
+           for _ in range(2)]
+    desc = lambda o: [dict(pos=t[0], hsml=t[1], m=t[2], rho=t[3], bin_q=t[4], weights=t[5], out=o,
+                           n=n, nq=nq, npix=npix, len2pix=float(npix), kernel=s2g.WendlandC6(2))]
+    ctx.set_tuning(dict(gather_item_min=least, small_side=5))  # no footprint in the scatter
+    with s2g.BatchPlan(desc(out[0]), dtype="f64", context=ctx) as plan:
+        st = {}
+        plan.run(stats=st)
+    assert st["n_small"] == 0 and st["n_pairs"] > 4 * 2 * least
+    s2g.deposit_batch_device(desc(out[1]), dtype="f64", context=ctx)
+    torch.cuda.synchronize()
+    assert torch.equal(out[0], out[1])
