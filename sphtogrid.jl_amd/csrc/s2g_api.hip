@@ -158,6 +158,22 @@ void read_i64(s2g_ctx *c, hipStream_t s, std::initializer_list<const int64_t *> 
         dst[i] = c->h_small[i];
 }
 
+// Of a deposit from its fork on: if the call fails before its streams have been
+// joined and waited for, what it has enqueued ends before it returns, since the
+// next call (on whichever stream) takes the same buffers.
+struct ForkGuard {
+    s2g_ctx *c;
+    hipStream_t s;
+    bool joined = false;
+    ~ForkGuard()
+    {
+        if (joined)
+            return;
+        for (hipStream_t q : {s, c->side, c->side2})
+            (void)hipStreamSynchronize(q);
+    }
+};
+
 float elapsed(hipEvent_t a, hipEvent_t b)
 {
     float ms = 0.f;
@@ -675,6 +691,7 @@ void deposit2d_pass(s2g_ctx *c, const MapIn *mi, int nmaps, hipStream_t s, s2g_s
     // A small pass leaves CUs idle in every stage: there the small scatter
     // has a stream of its own (3D, 130,000 on 80^3: 787 -> 648 us).
     hipStream_t s2 = c->side, s3 = partition_blocks(ntot) <= kPartLight ? c->side2 : s2;
+    ForkGuard forked{c, s};
     S2G_HIP(hipEventRecord(c->fork, s));
     S2G_HIP(hipStreamWaitEvent(s2, c->fork, 0));
     if (s3 != s2)
@@ -807,6 +824,7 @@ void deposit2d_pass(s2g_ctx *c, const MapIn *mi, int nmaps, hipStream_t s, s2g_s
         S2G_HIP(hipMemcpyAsync(c->h_small, tp.d_npairs, sizeof(int64_t), hipMemcpyDeviceToHost,
                                s));
     S2G_HIP(hipStreamSynchronize(s));
+    forked.joined = true;
     if (st) {
         double ms_gather = 0.0, ms_fin = 0.0;
         for (int k = 10; k < ev; k += 4) {
@@ -904,6 +922,7 @@ void deposit3d_device(s2g_ctx *c, const Map3DArgs &a, double *d_image, hipStream
     // and the gather; the gather waits for the normalisation and the
     // finalize for the scatter, to whose sums it adds.
     hipStream_t s2 = c->side, s3 = partition_blocks(n) <= kPartLight ? c->side2 : s2;
+    ForkGuard forked{c, s};
     S2G_HIP(hipEventRecord(c->fork, s));
     S2G_HIP(hipStreamWaitEvent(s2, c->fork, 0));
     if (s3 != s2)
@@ -1017,6 +1036,7 @@ void deposit3d_device(s2g_ctx *c, const Map3DArgs &a, double *d_image, hipStream
         S2G_HIP(hipMemcpyAsync(c->h_small, tp.d_npairs, sizeof(int64_t), hipMemcpyDeviceToHost,
                                s));
     S2G_HIP(hipStreamSynchronize(s));
+    forked.joined = true;
     if (st) {
         if (cl.nl > 0) {
             st->ms_gather = elapsed(E[10], E[11]);
@@ -1888,6 +1908,8 @@ void s2g_destroy(s2g_ctx *c)
         (void)hipStreamSynchronize(c->stream);
     if (c->side)
         (void)hipStreamSynchronize(c->side);
+    if (c->side2)
+        (void)hipStreamSynchronize(c->side2);
     for (auto &b : c->in) b.release();
     c->rec.release();
     c->cls.release();
