@@ -60,33 +60,37 @@ __global__ __launch_bounds__(kPartBlock) void k_part_light(
     __shared__ uint64_t s_bal[3][kW];
     const int nb = gridDim.x;
     const int wv = threadIdx.x / kWave, ln = threadIdx.x % kWave;
-    for (int k = 0; k < 3; ++k) {
-        int pre = 0, tot = 0;
-        for (int b = threadIdx.x; b < nb; b += kPartBlock) {
+    // the counts of the blocks before this one, all counts, and in the first
+    // block the pairs (at most kPartLight / kPartBlock blocks a thread: a wave's
+    // sum fits); the loads and the reductions overlap
+    int spre[3] = {}, stot[3] = {};
+    uint32_t spairs = 0;
+    for (int b = threadIdx.x; b < nb; b += kPartBlock) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
             const int v = (int)counts[(int64_t)k * nb + b];
-            pre += b < (int)blockIdx.x ? v : 0;
-            tot += v;
+            spre[k] += b < (int)blockIdx.x ? v : 0;
+            stot[k] += v;
         }
-#pragma unroll
-        for (int o = 1; o < kWave; o <<= 1) {
-            pre += __shfl_xor(pre, o, kWave);
-            tot += __shfl_xor(tot, o, kWave);
-        }
-        if (ln == 0) {
-            s_pre[k][wv] = pre;
-            s_tot[k][wv] = tot;
-        }
+        if (blockIdx.x == 0)
+            spairs += (uint32_t)counts[3 * (int64_t)nb + 1 + b];
     }
-    if (blockIdx.x == 0) {
-        // at most kPartLight / kPartBlock blocks a thread: a wave's sum fits
-        uint32_t v = 0;
-        for (int b = threadIdx.x; b < nb; b += kPartBlock)
-            v += (uint32_t)counts[3 * (int64_t)nb + 1 + b];
 #pragma unroll
-        for (int o = 1; o < kWave; o <<= 1)
-            v += __shfl_xor(v, o, kWave);
-        if (ln == 0)
-            s_pairs[wv] = v;
+    for (int o = 1; o < kWave; o <<= 1) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            spre[k] += __shfl_xor(spre[k], o, kWave);
+            stot[k] += __shfl_xor(stot[k], o, kWave);
+        }
+        spairs += __shfl_xor(spairs, o, kWave);
+    }
+    if (ln == 0) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            s_pre[k][wv] = spre[k];
+            s_tot[k][wv] = stot[k];
+        }
+        s_pairs[wv] = spairs;
     }
     static_assert((int64_t)kWave * (kPartLight / kPartBlock) * kPairsMost < ((int64_t)1 << 32));
     const int64_t p = (int64_t)blockIdx.x * kPartBlock + threadIdx.x;
