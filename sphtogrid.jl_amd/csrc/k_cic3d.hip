@@ -910,11 +910,11 @@ __global__ __launch_bounds__(kS3Waves *kWave) void k3d_small_window(
             const int64_t idx = ((int64_t)i * npix + j) * npix + k;
             const int cell = di * kSW3x + dj * kSW3y + dk;
             const double q = acc[0][cell], w = acc[1][cell];
-            // each plane by itself: signed weights may cancel where quantities do not
-            if (q != 0.0)
+            // signed weights may cancel where quantities do not
+            if (q != 0.0 || w != 0.0) {
                 unsafeAtomicAdd(&image[idx], q);
-            if (w != 0.0)
                 unsafeAtomicAdd(&image[nd + idx], w);
+            }
         }
         __syncthreads();
     }
