@@ -125,9 +125,9 @@ typedef struct s2g_stats {
     int64_t n_pairs;          /* (tile, particle) pairs of the gather path */
     double sum_footprint;     /* reserved (0) */
     /* device time per stage (HIP events), ms.  In the 2D / 3D deposits the
-     * normalisation sums and the small-footprint scatter run on a side stream
+     * normalisation sums and the small-footprint scatter run on side streams
      * beside the pair sort and the gather, so those stages overlap: ms_norm
-     * and ms_small are the spans on the side stream (they include its wait
+     * and ms_small are the spans on their side streams (they include the wait
      * for a share of the GPU), ms_device the whole call. */
     double ms_setup;          /* per-particle setup + class partition */
     double ms_norm;           /* explicit footprint normalisation sums */

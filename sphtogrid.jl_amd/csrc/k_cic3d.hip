@@ -407,7 +407,8 @@ __global__ __launch_bounds__(256) void k3d_norm(const int32_t *__restrict__ list
 // multipliers: one instruction per voxel more than the 2D gather's per
 // pixel, and a per-particle set-up of one FP64 multiplier per plane.
 // ---------------------------------------------------------------------------
-// Issue takes three quarters of the time, the rest are waits: the chain of a
+// Counted at four cycles an instruction, VALU issue takes three quarters of the
+// time; the rest are waits: the chain of a
 // sub-brick, which four waves per SIMD (64 accumulator registers) do not
 // cover, and the barriers, so batches are as long as the four blocks of a CU
 // have LDS for and the records of two are read at once.  Cluster set at 256^3,
@@ -763,8 +764,10 @@ __global__ __launch_bounds__(256) void k3d_small_flat(const int32_t *__restrict_
 // window cell.  A wave takes a particle: lanes over the box's (y, z) columns,
 // R = 64 / columns x planes per step, the y and z terms in registers and the
 // x terms in a per-wave LDS table; the weights stay in registers between the
-// sum and the deposit.  Boxes of at most 2^3 voxels go eight to a wave, a
-// lane per voxel.  FP64 throughout.
+// sum and the deposit.  A lane without a voxel of the box is left out by its
+// index (small3_lane), not by its weight alone, which a scale that is not finite
+// turns into NaN (0.6 % of a windowed call).  Boxes of at most 2^3 voxels go
+// eight to a wave, a lane per voxel.  FP64 throughout.
 // Bound by the FP64 arithmetic (a square root per voxel) and the LDS
 // atomics.  Measured: 200,003 particles on 101^3 (113 k small), flat 589 us,
 // windowed 155 us; 2^24 cluster set on 256^3 (12.0 M small), 7.1 ms alone,

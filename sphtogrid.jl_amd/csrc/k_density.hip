@@ -525,7 +525,7 @@ __global__ __launch_bounds__(kWave, 4) void k_md_knn(
                 int r = t;
                 double dd = 0.0;
                 for (int d = 0; d < 3; ++d) {
-                    // r = q cl + rem with r < 216, cl <= 6: the float
+                    // r = q cl + rem with r < 128, cl <= 6: the float
                     // quotient of r + 1/2 is at least 1/12 from an integer
                     const int qd = d < 2 ? (int)(((float)r + 0.5f) * rcl[d]) : 0;
                     int o = ca[d] + (r - qd * cl[d]);

@@ -609,7 +609,7 @@ __device__ __forceinline__ void k_hp_norm_one(int64_t gw, const int2 *__restrict
     if (ln == 0)
         part[gw] = make_double4(swa, sad, 0.0, 0.0);
 }
-// Bound by VALU issue (0.99 of the rate before), so the loop is cut to what a
+// VALU issue is the largest claim on its time, so the loop is cut to what a
 // pixel's value needs: chord tables in half angles with an end mark, list
 // positions kept in FP32, no clamp or library branch for discs below 1 radian
 // and no sum of A where the fallback is ruled out take 45 VALU instructions
