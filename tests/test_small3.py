@@ -135,3 +135,43 @@ def test_share_of_a_lattice(lib):
     s = _sample(lib, tile, np.full(side ** 3, 23))
     assert abs(lib.share(s.ctypes.data, len(s)) / true - 1) < 0.5
     assert lib.windowed(side ** 3, npix, s.ctypes.data, len(s), 1) == 0
+
+
+def _boxes(x, h, npix):
+    """Voxels and first tile of the footprint boxes of particles at x (box
+    units around 0), as the set-up clips them."""
+    g = x * npix + 0.5 * npix
+    lo = np.clip(np.floor(g - h[:, None] * npix), 0, npix - 1).astype(np.int64)
+    hi = np.clip(np.floor(g + h[:, None] * npix), 0, npix - 1).astype(np.int64)
+    c, nt = lo // 9, -(-npix // 9)
+    return (hi - lo + 1).prod(1), (c[:, 0] * nt + c[:, 1]) * nt + c[:, 2]
+
+
+@pytest.mark.parametrize("npix,n,hpix,clump,want", [
+    (18, 3000, 0.4, 1.0, 0),
+    (18, 3000, 3.4, 1.0, 1),
+    (27, 300000, 0.4, 1.0, 0),
+    (27, 300000, 2.0, 1.0, 1),
+    (48, 300000, 0.5, 0.05, 1),
+])
+def test_which_scatter_the_gpu_tests_take(lib, npix, n, hpix, clump, want):
+    """The sets of test_gpu_cic3d.py's test_small_scatter_rule: both scatters,
+    the windowed one on the lists of small passes and on sorted ones."""
+    r = np.random.default_rng(n + npix)
+    x = clump * r.uniform(-0.5, 0.5, (n, 3))
+    h = hpix / npix * r.uniform(0.9, 1.0, n)
+    vox, tile = _boxes(x, h, npix)
+    s = _sample(lib, tile, vox)
+    assert lib.windowed(n, npix, s.ctypes.data, len(s), n <= 1 << 18) == want
+
+
+def test_the_special_value_sets_are_windowed(lib):
+    """The sets of test_gpu_small3.py."""
+    import test_gpu_small3 as t
+    for seed, lo, hi in ((11, 0.0, t.NPIX), (12, 0.0, t.NPIX), (13, 0.0, 8.0)):
+        p = t._set(3000, seed, lo, hi)
+        if seed == 12:
+            p[1][::5] = 0.4 / t.NPIX
+        vox, tile = _boxes(p[0], p[1], t.NPIX)
+        s = _sample(lib, tile, vox)
+        assert lib.windowed(3000, t.NPIX, s.ctypes.data, len(s), 1) == 1
